@@ -74,20 +74,21 @@ bool mfma16_path(const xdit_attn_args* a) {
 //          + for a balanced launch: its extra launches, and the partial results a compute unit writes and folds.
 // `plain`: the launch will not be balanced (a call without a workspace); `fold_only`: the ring step,
 // whose shared tiles are folded inside the attention kernel (plans of at most 16 parts per tile and
-// 128- or 256-row workgroups, and about 25 us for the fold on top).  fp8 at head_dim 64 is planned
-// with the fp8 constants of head_dim 128.
-// Rate and segment cost depend on what a compute unit holds.  One 4-wavefront workgroup leaves
-// every SIMD a single wavefront with nothing to overlap its softmax with (1.5 times the time per
+// 128- or 256-row workgroups, and about 25 us for the fold on top).
+// Rate and segment cost depend on what a compute unit holds (Cost below).  One 4-wavefront workgroup
+// leaves every SIMD a single wavefront with nothing to overlap its softmax with (1.5 times the time per
 // row of 12 wavefronts); two of them hide each other's prologue and epilogue, which a lone 8- or
 // 12-wavefront workgroup exposes in full (what decides cross-attention on a few dozen keys).
 // Balancing pays wherever the tiles leave compute units idle in the last round (the best plain
 // launch is 21 % slower on average than the best of the six, up to 3.8 times on a few heads of
-// 1000 to 3000 tokens) and costs a few per cent where they do not.  The constants (ns per query
-// row and KV tile; us) are fitted to the times of every option, taken at settled clocks, on 413
-// 16-bit problems (B*H 1..48, S 1024..118800, head_dim 64..128; self-attention, ring chunks and
-// cross-attention on 77..4608 keys) and 207 fp8 problems.  There the choice is 1.0 % (head_dim
-// 128), 1.4 % (64) and 0.6 % (fp8) slower than the fastest option on average, 11 % at worst; on
-// 140 problems kept out of an earlier fit of the same form, 1.4 % and 2.0 %.
+// 1000 to 3000 tokens) and costs a few per cent where they do not.  The constants are fitted to the
+// times of every option, taken at settled clocks: on 413 16-bit problems (B*H 1..48, S 1024..118800,
+// head_dim 64..128; self-attention, ring chunks and cross-attention on 77..4608 keys), 207 fp8 problems at
+// head_dim 128 and 56 at head_dim 64 (B*H 1..96, S 512..60000, keys 77..60000).  There the choice is 1.0 %
+// (16-bit, head_dim 128), 1.4 % (16-bit, 64), 0.6 % (fp8, 128) and 0.1 % (fp8, 64) slower than the fastest
+// option on average, 11 % at worst (3 % for the last).  (fp8 at head_dim 64 planned with the constants of head_dim 128,
+// which take 384-row workgroups for long sequences: 3 % on average, 19 % at worst; B*H = 96, S = 17776: 6.16
+// against 5.47 ms.)
 struct LaunchChoice {
   int rows;    // query rows per workgroup
   int policy;  // AttnParams::split_policy: 1 plain launch, 2 balanced when the planner offers a plan
@@ -102,23 +103,24 @@ LaunchChoice choose_launch(const xdit_attn_args* a, bool plain = false, bool fol
   const int64_t bh = (int64_t)a->B * a->H;
   const int64_t nt = (a->Sk + xdit::kKeysPerTile - 1) / xdit::kKeysPerTile + (a->Sk2 + xdit::kKeysPerTile - 1) / xdit::kKeysPerTile;
   static const int kRows[3] = {384, 256, 128};
-  // 16-bit: {384 rows, 256 rows, 128 rows with two workgroups on the compute unit, 128 rows alone}
-  static const double kRate128[4] = {5.65, 5.88, 6.93, 8.65}, kRate64[4] = {3.59, 3.56, 4.26, 6.17};
-  static const double kSeg128[4] = {8.25, 6.36, 2.05, 6.57}, kSeg64[4] = {2.57, 1.70, 0.42, 2.18};
-  const double* rate = D == 64 ? kRate64 : kRate128;
-  const double* seg_us = D == 64 ? kSeg64 : kSeg128;
-  // a balanced launch: its extra launches, and the partial results per compute unit (us per thousand rows)
-  const double split_us = D == 64 ? 1.73 : 3.72;
-  const double parts_us = D == 64 ? 18.12 : 28.82;
-  // fp8 (head_dim 128, up to three 4-wavefront workgroups per compute unit):
-  // {384 rows, 256 rows, 128 rows x 3 / x 2 / alone}
-  static const double kRateFp8[5] = {3.64, 4.01, 4.02, 4.99, 6.06}, kSegFp8[5] = {6.18, 5.00, 0.16, 1.62, 5.70};
-  const double split_fp8_us = 1.04, parts_fp8_us = 30.50;
+  // What the compute unit holds: 0 one 384-row workgroup; 1, 2 that many 256-row ones; 3..6 one to four 128-row ones.
+  struct Cost {
+    double rate[7];   // ns per query row and KV tile
+    double seg_us[7];
+    double split_us;  // a balanced launch: its extra launches ...
+    double parts_us;  // ... and the partial results per compute unit (us per thousand rows)
+    bool tail;        // fitted with the last, partial round of a plain launch priced by what a compute unit holds in it
+  };
+  static const Cost k16_128 = {{5.65, 5.88, 0, 8.65, 6.93, 0, 0}, {8.25, 6.36, 0, 6.57, 2.05, 0, 0}, 3.72, 28.82, false};
+  static const Cost k16_64 = {{3.59, 3.56, 0, 6.17, 4.26, 0, 0}, {2.57, 1.70, 0, 2.18, 0.42, 0, 0}, 1.73, 18.12, false};
+  static const Cost k8_128 = {{3.64, 4.01, 0, 6.06, 4.99, 4.02, 0}, {6.18, 5.00, 0, 5.70, 1.62, 0.16, 0}, 1.04, 30.50, false};
+  static const Cost k8_64 = {{3.23, 3.22, 2.69, 5.26, 3.29, 3.20, 2.96}, {6.59, 6.55, 2.93, 5.08, 2.79, 2.12, 0.79}, 3.51, 15.82, true};
+  const Cost& k = fp8 ? (D == 64 ? k8_64 : k8_128) : (D == 64 ? k16_64 : k16_128);
   double best_cost = -1;
   for (int i = 0; i < 3; i++) {
     const int rows = kRows[i];
     if (a->rows_per_workgroup != 0 && a->rows_per_workgroup != rows) continue;  // validated by check_tuning
-    const int per_cu = rows == 128 ? (fp8 ? 3 : 2) : 1;  // workgroups resident per compute unit
+    const int per_cu = xdit::workgroups_per_cu(fp8, D, rows);  // workgroups resident per compute unit
     const int64_t tiles = bh * ((a->Sq + rows - 1) / rows);
     if (tiles > 0x7fffffff) continue;
     const int slots = cus * per_cu;
@@ -142,23 +144,25 @@ LaunchChoice choose_launch(const xdit_attn_args* a, bool plain = false, bool fol
       int64_t sharing = (tiles + cus - 1) / cus;  // workgroups on the busiest compute unit at once
       if (sharing > per_cu || q.split_units) sharing = per_cu;
       // rounds of resident workgroups; a long plain launch streams its workgroups through the slots
-      const double rounds = q.split_units ? (double)(q.split_full / slots)
-                            : tiles <= 4 * (int64_t)slots ? (double)((tiles + slots - 1) / slots) : (double)tiles / slots + 0.5;
+      double rounds = q.split_units ? (double)(q.split_full / slots)
+                      : tiles <= 4 * (int64_t)slots ? (double)((tiles + slots - 1) / slots) : (double)tiles / slots + 0.5;
+      const int base = i == 0 ? 0 : i == 1 ? 1 : 3;
+      double last_us = 0.0;
+      if (k.tail && !q.split_units && tiles <= 4 * (int64_t)slots && tiles > slots && tiles % slots != 0) {
+        rounds -= 1.0;
+        const int left = (int)((tiles % slots + cus - 1) / cus);
+        last_us = (k.rate[base + left - 1] * nt * rows * 1e-3 + k.seg_us[base + left - 1]) * left;
+      }
       const double units = rounds * nt + (q.split_units ? q.split_share : 0);
       const double segs = rounds + (q.split_units ? 1 : 0);
       // partial results written and folded, in thousands of rows per compute unit
       const double parts = q.split_units ? (double)(tiles - q.split_full) * q.split_pmax * rows / cus * 1e-3 : 0.0;
-      double cost;
       // the ring step folds its shared tiles inside the attention kernel: a slice per workgroup at its end, or the whole
       // tile by whoever completes it, one round trip to memory after the other (measured: about 25 us)
       const double fold_us = fold_only && q.split_units ? 25.0 : 0.0;
-      if (fp8) {
-        const int cls = rows == 128 ? 5 - (int)sharing : i;
-        cost = kRateFp8[cls] * units * rows * (double)sharing * 1e-3 + kSegFp8[cls] * segs * (double)sharing + (q.split_units ? split_fp8_us + parts_fp8_us * parts : 0.0) + fold_us;
-      } else {
-        const int cls = rows == 128 ? (sharing > 1 ? 2 : 3) : i;
-        cost = rate[cls] * units * rows * (double)sharing * 1e-3 + seg_us[cls] * segs * (double)sharing + (q.split_units ? split_us + parts_us * parts : 0.0) + fold_us;
-      }
+      const int cls = base + (int)sharing - 1;
+      const double cost = k.rate[cls] * units * rows * (double)sharing * 1e-3 + k.seg_us[cls] * segs * (double)sharing +
+                          (q.split_units ? k.split_us + k.parts_us * parts : 0.0) + last_us + fold_us;
       if (best_cost < 0 || cost < best_cost) { best.rows = rows; best.policy = policy; best_cost = cost; }
     }
   }

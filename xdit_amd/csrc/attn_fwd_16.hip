@@ -13,7 +13,7 @@ static size_t workspace_one(const AttnParams& p, AttnParams* plan, bool fold_onl
   q.nq_tiles = (p.Sq + rows - 1) / rows;
   q.total_tiles = p.B * p.H * q.nq_tiles;
   q.tiles_per_xcd = (q.total_tiles + 7) / 8;
-  const size_t need = plan_split(q, rows, resident_workgroups(NW, p.cu_count), D, 2, kClaimsPerWorkgroup, true, fold_only);
+  const size_t need = plan_split(q, rows, resident_cus(p.cu_count) * workgroups_per_cu(false, D, rows), D, 2, kClaimsPerWorkgroup, true, fold_only);
   if (plan != nullptr) *plan = q;
   return need;
 }

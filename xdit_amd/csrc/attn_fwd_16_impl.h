@@ -125,33 +125,38 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
   const unsigned ld_kdst = lds_base + wave * G::K_PITCH;      // LDS address of K piece `wave`, buffer 0
   const unsigned ld_vdst = lds_base + G::K_BYTES + wave * G::V_PITCH;
 
-  // Where the K/V rows of the current (batch, head) lie, set per segment: per KV segment the
-  // pointers to its first rows, the row strides in bytes (below 2^24) and its number of keys.
-  const T* kv_k1;
-  const T* kv_v1;
-  const T* kv_k2;
-  const T* kv_v2;
-  unsigned kss1, vss1, kss2, vss2;
-  int keys1, keys2;
-  // Loads KV tile t of the current (batch, head) into buffer `buf`.
-  auto issue_tile = [&](int t, int buf) {
+  // Where the KV tile to be loaded next lies: pointers to its first rows, the row strides in bytes
+  // (below 2^24) and the keys of its KV segment from there on.  A segment's tiles are loaded one after the other, so that a tile costs two pointer additions.
+  const unsigned char* ld_k;
+  const unsigned char* ld_v;
+  unsigned ld_kss, ld_vss;
+  int ld_left;
+  auto aim_loader = [&](int b, int h, int t) {
+    const bool second = t >= nt1;
+    const unsigned row0 = (unsigned)(second ? t - nt1 : t) * kKeysPerTile;   // first key of the tile within its segment
+    ld_kss = (unsigned)(second ? pp->k2s_s : pp->ks_s) * 2;
+    ld_vss = (unsigned)(second ? pp->v2s_s : pp->vs_s) * 2;
+    ld_k = (const unsigned char*)(second ? (const T*)pp->k2 + b * pp->k2s_b + h * pp->k2s_h : (const T*)pp->k + b * pp->ks_b + h * pp->ks_h);
+    ld_v = (const unsigned char*)(second ? (const T*)pp->v2 + b * pp->v2s_b + h * pp->v2s_h : (const T*)pp->v + b * pp->vs_b + h * pp->vs_h);
+    ld_k += (uint64_t)row0 * ld_kss;
+    ld_v += (uint64_t)row0 * ld_vss;
+    ld_left = (second ? pp->Sk2 : pp->Sk) - (int)row0;
+  };
+  // Loads that tile into the buffer at LDS offset bo and moves on to the one behind it.
+  auto issue_tile = [&](unsigned bo) {
     if ((kWaves == LW || wave < LW) && ld_on) {
-      const bool second = t >= nt1;
-      const unsigned row0 = (unsigned)(second ? t - nt1 : t) * kKeysPerTile;   // first key of the tile within its segment
-      const unsigned kss = second ? kss2 : kss1, vss = second ? vss2 : vss1;
-      const T* kp = (const T*)((const unsigned char*)(second ? kv_k2 : kv_k1) + (uint64_t)row0 * kss);
-      const T* vp = (const T*)((const unsigned char*)(second ? kv_v2 : kv_v1) + (uint64_t)row0 * vss);
-      const int left = (second ? keys2 : keys1) - (int)row0;
-      const int last = (left < kKeysPerTile ? left : kKeysPerTile) - 1;
-      const unsigned bo = buf * G::BUF_BYTES;
+      const int last = (ld_left < kKeysPerTile ? ld_left : kKeysPerTile) - 1;
 #pragma unroll
       for (int i = 0; i < PAIRS; i++) {
         int r = ld_row0 + LW * i;
         r = r < last ? r : last;  // rows past the end of the segment re-read its last row
-        load_lds_16(kp, __umul24((unsigned)r, kss) + ld_colb, ld_kdst + bo + i * LW * G::K_PITCH);
-        load_lds_16(vp, __umul24((unsigned)r, vss) + ld_colb, ld_vdst + bo + i * LW * G::V_PITCH);
+        load_lds_16(ld_k, __umul24((unsigned)r, ld_kss) + ld_colb, ld_kdst + bo + i * LW * G::K_PITCH);
+        load_lds_16(ld_v, __umul24((unsigned)r, ld_vss) + ld_colb, ld_vdst + bo + i * LW * G::V_PITCH);
       }
     }
+    ld_k += (uint64_t)ld_kss * kKeysPerTile;
+    ld_v += (uint64_t)ld_vss * kKeysPerTile;
+    ld_left -= kKeysPerTile;
   };
 
   // ---- LDS read addresses: one per-lane base each for K and V, the rest are immediates ------
@@ -193,17 +198,6 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
     qt = sg.tile - bh * nq_tiles;
     b = bh / H;
     h = bh - b * H;
-    kv_k1 = (const T*)pp->k + b * pp->ks_b + h * pp->ks_h;
-    kv_v1 = (const T*)pp->v + b * pp->vs_b + h * pp->vs_h;
-    kss1 = (unsigned)pp->ks_s * 2; vss1 = (unsigned)pp->vs_s * 2;
-    keys1 = pp->Sk; keys2 = pp->Sk2;
-    if (keys2 > 0) {
-      kv_k2 = (const T*)pp->k2 + b * pp->k2s_b + h * pp->k2s_h;
-      kv_v2 = (const T*)pp->v2 + b * pp->v2s_b + h * pp->v2s_h;
-      kss2 = (unsigned)pp->k2s_s * 2; vss2 = (unsigned)pp->v2s_s * 2;
-    } else {
-      kv_k2 = kv_k1; kv_v2 = kv_v1; kss2 = kss1; vss2 = vss1;
-    }
     const int Sq = pp->Sq;
     const int qrow = qt * kRowsPerBlock + wave * kRowsPerWave + l32;
     const int qrow_c = qrow < Sq ? qrow : Sq - 1;
@@ -217,7 +211,8 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
         for (int e = 0; e < 8; e++) qf[ks][e] = (T)0.f;
       }
     }
-    issue_tile(sg.it0, 0);
+    aim_loader(b, h, sg.it0);
+    issue_tile(0);
   };
   XDIT_TRACE_POINT(seg.slot >= 0, 0);
   open_segment(seg);
@@ -237,7 +232,7 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
     const int pool_len = nt - seg.pool0;
     unsigned* const draw_counter = streamed ? pp->split_counter + seg.dyn : nullptr;
     bool pool_open = streamed;  // thread 0: no ticket has come back past the end of the pool yet
-    const int keys_1 = keys1, keys_2 = keys2;
+    int left = ld_left + kKeysPerTile;  // keys of the KV segment from the current tile on
 
     // ---- online softmax state: one query per lane (both halves of the wavefront agree) ------
     float m_used = -INFINITY;          // running (lazily updated) row maximum of the raw dot products
@@ -268,7 +263,12 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
       if (i + 1 < n_own) t_next = t + 1;
       else if (streamed) t_next = __builtin_amdgcn_readfirstlane(drawn[(i + 1) & 1]);  // posted during the previous iteration
       else t_next = -1;
-      if (t_next >= 0) issue_tile(t_next, buf ^ 1);
+      int left_next = 0;
+      if (t_next >= 0) {
+        if (t_next == nt1 || t_next != t + 1) aim_loader(cb, ch, t_next);  // the second KV segment's first tile, or a drawn one
+        left_next = ld_left;
+        issue_tile((buf ^ 1) * G::BUF_BYTES);
+      }
       // Streamed sharing: thread 0 draws the ticket of position i + 2 now and posts the KV tile
       // it stands for at the end of this iteration, when the ticket has long come back.
       const bool drawing = streamed && i + 2 >= n_own && t_next >= 0;
@@ -305,15 +305,14 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
         });
       }
       // ---- mask keys past the end of the segment (only its last tile can be partial) -------
-      const int valid = (t < nt1) ? keys_1 - t * kKeysPerTile : keys_2 - (t - nt1) * kKeysPerTile;
-      if (valid < kKeysPerTile) {
+      if (left < kKeysPerTile) {
         const int hh = lane_now() >> 5;
 #pragma unroll
         for (int kb = 0; kb < 2; kb++)
 #pragma unroll
           for (int e = 0; e < 16; e++) {
             int key = 32 * kb + 8 * (e >> 2) + 4 * hh + (e & 3);
-            if (key >= valid) sacc[kb][e] = -INFINITY;
+            if (key >= left) sacc[kb][e] = -INFINITY;
           }
       }
 
@@ -386,6 +385,7 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
       }
       if (t_next < 0) break;
       t = t_next;
+      left = left_next;
     }
     XDIT_TRACE_POINT(seg.slot >= 0, 2);
     asm volatile("" : "+s"(pp));  // from here on the kernel arguments are read afresh
@@ -581,10 +581,6 @@ __global__ __launch_bounds__(64 * NW, NW == 12 ? 3 : 2) void attn_fwd_16_kernel(
   attn_workgroup<T, D, DC, NW, PAD, FUSED>(smem);
 }
 
-// Workgroups of NW wavefronts resident at once: LDS and registers allow two 4-wavefront
-// workgroups per CU, one otherwise.
-static int resident_workgroups(int NW, int planned_cus) { return resident_cus(planned_cus) * (NW == 4 ? 2 : 1); }
-
 template <typename T, int D, int DC, int NW, bool PAD, bool FUSED>
 static hipError_t launch_kernel(const AttnParams& q, hipStream_t stream) {
   static std::atomic<bool> lds_ready[kMaxDevices];
@@ -607,7 +603,7 @@ static hipError_t launch_one(const AttnParams& p, hipStream_t stream) {
   q.total_tiles = p.B * p.H * q.nq_tiles;
   q.tiles_per_xcd = (q.total_tiles + 7) / 8;
   // the ring step takes a balanced plan only when the attention kernel folds the parts itself (the fold goes on into the accumulator)
-  bind_workspace(q, p, plan_split(q, rows, resident_workgroups(NW, p.cu_count), D, 2, kClaimsPerWorkgroup, true, FUSED), rows, D, 2);
+  bind_workspace(q, p, plan_split(q, rows, resident_cus(p.cu_count) * workgroups_per_cu(false, D, rows), D, 2, kClaimsPerWorkgroup, true, FUSED), rows, D, 2);
   if (q.d_actual == D) q.d_actual = 0;
   // computed head_dims built for tensors smaller than D: 80, 96, 112 (and 128) of 128; 32 (and 64) of 64
   hipError_t e;

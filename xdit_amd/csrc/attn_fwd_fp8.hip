@@ -98,38 +98,51 @@ __device__ __forceinline__ void attn_workgroup_fp8(unsigned char* smem) {
   constexpr int LW = kWaves < NG ? kWaves : NG;
   constexpr int PAIRS = NG / LW;
   constexpr int LANES_PER_ROW = ROW_BYTES / 16;
-  int ld_row0 = NG * (lane / LANES_PER_ROW) + wave;    // row of this lane in pair 0
-  unsigned ld_colb = (lane % LANES_PER_ROW) * 16;
-  asm volatile("" : "+v"(ld_row0), "+v"(ld_colb));
   const unsigned lds_base = (unsigned)(uintptr_t)(XDIT_LDS u8*)smem;
   const unsigned ld_kdst = lds_base + wave * K_PITCH;  // LDS address of K piece `wave`, buffer 0
   const unsigned ld_vdst = lds_base + K_BYTES + wave * V_PITCH;
 
-  // Where the K/V rows of the current (batch, head) lie, set per segment (row strides in bytes).
-  const u8* kv_k1;
-  const u8* kv_v1;
-  const u8* kv_k2;
-  const u8* kv_v2;
-  unsigned kss1, vss1, kss2, vss2;
-  int keys1, keys2;
-  auto issue_tile = [&](int t, int buf) {
+  int ld_row0 = NG * (lane / LANES_PER_ROW) + wave;    // row of this lane in pair 0
+  unsigned ld_colb = (lane % LANES_PER_ROW) * 16;
+  asm volatile("" : "+v"(ld_row0), "+v"(ld_colb));
+
+  // The K/V tiles of a segment are requested one after the other, so that a tile costs two pointer
+  // additions: where the next one lies (its first rows), the row strides in bytes and the keys of its
+  // KV segment from there on.  Nothing of it is read from the kernel arguments in the KV loop: a scalar
+  // load there would put a wait for every LDS read in flight behind it (1.2 % on the Wan-size shard).
+  // Against forming both addresses from (tile, segment) for every tile: B*H = 20, S = 581, head_dim 128
+  // 14.8 -> 13.6 us; B*H = 96, S = 17776, head_dim 64, 128-row workgroups 8 % ; no change at 384 rows.
+  const u8* ld_k;
+  const u8* ld_v;
+  unsigned ld_kss, ld_vss;
+  int ld_left;
+  // Points the loader at KV tile t of (b, h).
+  auto aim_loader = [&](int b, int h, int t) {
+    const bool second = t >= nt1;
+    const unsigned row0 = (unsigned)(second ? t - nt1 : t) * kKeysPerTile;
+    ld_kss = (unsigned)(second ? pp->k2s_s : pp->ks_s);
+    ld_vss = (unsigned)(second ? pp->v2s_s : pp->vs_s);
+    ld_k = second ? (const u8*)pp->k2 + b * pp->k2s_b + h * pp->k2s_h : (const u8*)pp->k + b * pp->ks_b + h * pp->ks_h;
+    ld_v = second ? (const u8*)pp->v2 + b * pp->v2s_b + h * pp->v2s_h : (const u8*)pp->v + b * pp->vs_b + h * pp->vs_h;
+    ld_k += (uint64_t)row0 * ld_kss;
+    ld_v += (uint64_t)row0 * ld_vss;
+    ld_left = (second ? pp->Sk2 : pp->Sk) - (int)row0;
+  };
+  // Requests the next KV tile into the buffer at LDS offset bo.
+  auto issue_tile = [&](unsigned bo) {
     if (kWaves == LW || wave < LW) {
-      const bool second = t >= nt1;
-      const unsigned row0 = (unsigned)(second ? t - nt1 : t) * kKeysPerTile;
-      const unsigned kss = second ? kss2 : kss1, vss = second ? vss2 : vss1;
-      const u8* kp = (second ? kv_k2 : kv_k1) + (uint64_t)row0 * kss;
-      const u8* vp = (second ? kv_v2 : kv_v1) + (uint64_t)row0 * vss;
-      const int left = (second ? keys2 : keys1) - (int)row0;
-      const int last = (left < kKeysPerTile ? left : kKeysPerTile) - 1;
-      const unsigned bo = buf * BUF_BYTES;
+      const int last = (ld_left < kKeysPerTile ? ld_left : kKeysPerTile) - 1;
 #pragma unroll
       for (int i = 0; i < PAIRS; i++) {
         int r = ld_row0 + LW * i;
         r = r < last ? r : last;  // rows past the end of the segment re-read its last row
-        load_lds_16(kp, __umul24((unsigned)r, kss) + ld_colb, ld_kdst + bo + i * LW * K_PITCH);
-        load_lds_16(vp, __umul24((unsigned)r, vss) + ld_colb, ld_vdst + bo + i * LW * V_PITCH);
+        load_lds_16(ld_k, __umul24((unsigned)r, ld_kss) + ld_colb, ld_kdst + bo + i * LW * K_PITCH);
+        load_lds_16(ld_v, __umul24((unsigned)r, ld_vss) + ld_colb, ld_vdst + bo + i * LW * V_PITCH);
       }
     }
+    ld_k += (uint64_t)ld_kss * kKeysPerTile;
+    ld_v += (uint64_t)ld_vss * kKeysPerTile;
+    ld_left -= kKeysPerTile;
   };
 
   // ---- LDS read bases ------------------------------------------------------------------------
@@ -158,17 +171,6 @@ __device__ __forceinline__ void attn_workgroup_fp8(unsigned char* smem) {
     qt = sg.tile - bh * nq_tiles;
     b = bh / H;
     h = bh - b * H;
-    kv_k1 = (const u8*)pp->k + b * pp->ks_b + h * pp->ks_h;
-    kv_v1 = (const u8*)pp->v + b * pp->vs_b + h * pp->vs_h;
-    kss1 = (unsigned)pp->ks_s; vss1 = (unsigned)pp->vs_s;
-    keys1 = pp->Sk; keys2 = pp->Sk2;
-    if (keys2 > 0) {
-      kv_k2 = (const u8*)pp->k2 + b * pp->k2s_b + h * pp->k2s_h;
-      kv_v2 = (const u8*)pp->v2 + b * pp->v2s_b + h * pp->v2s_h;
-      kss2 = (unsigned)pp->k2s_s; vss2 = (unsigned)pp->v2s_s;
-    } else {
-      kv_k2 = kv_k1; kv_v2 = kv_v1; kss2 = kss1; vss2 = vss1;
-    }
     float sq = 1.f, sk = 1.f;
     sv = 1.f;
     const int64_t ds = b * pp->ds_b + h * pp->ds_h;
@@ -186,7 +188,8 @@ __device__ __forceinline__ void attn_workgroup_fp8(unsigned char* smem) {
       i32x4 hi = *(const i32x4*)(qptr + ks * 64 + 16);
       qf[ks] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     }
-    issue_tile(sg.it0, 0);
+    aim_loader(b, h, sg.it0);
+    issue_tile(0);
   };
   open_segment(seg);
   for (;;) {  // segments of this workgroup
@@ -198,7 +201,6 @@ __device__ __forceinline__ void attn_workgroup_fp8(unsigned char* smem) {
       part_out = (TO*)pp->ws_out + seg.slot * kRowsPerBlock * D;
       part_lse = pp->ws_lse + seg.slot * kRowsPerBlock;
     }
-    const int keys_1 = keys1, keys_2 = keys2;
     float m_used = -INFINITY;
     float l_part = 0.f;
     f32x16 oacc[DB];
@@ -209,11 +211,17 @@ __device__ __forceinline__ void attn_workgroup_fp8(unsigned char* smem) {
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) asm volatile("" : "+v"(qf[ks]));
 
+    int left = ld_left + kKeysPerTile;  // keys of the KV segment from tile t on
     for (int t = seg.it0; t < seg.it1; t++) {
       const int buf = (t - seg.it0) & 1;
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
-      if (t + 1 < seg.it1) issue_tile(t + 1, buf ^ 1);
+      int left_next = 0;
+      if (t + 1 < seg.it1) {
+        if (t + 1 == nt1) aim_loader(cb, ch, t + 1);   // the first tile of the second KV segment
+        left_next = ld_left;
+        issue_tile((buf ^ 1) * BUF_BYTES);
+      }
 
       const unsigned kaddr = kbase_off + buf * BUF_BYTES;
       const unsigned vaddr = vbase_off + buf * BUF_BYTES;
@@ -251,15 +259,14 @@ __device__ __forceinline__ void attn_workgroup_fp8(unsigned char* smem) {
         });
       }
 
-      const int valid = (t < nt1) ? keys_1 - t * kKeysPerTile : keys_2 - (t - nt1) * kKeysPerTile;
-      if (valid < kKeysPerTile) {
+      if (left < kKeysPerTile) {
         const int hh = lane_now() >> 5;
 #pragma unroll
         for (int kb = 0; kb < 2; kb++)
 #pragma unroll
           for (int i = 0; i < 16; i++) {
             int key = 32 * kb + 8 * (i >> 2) + 4 * hh + (i & 3);
-            if (key >= valid) sacc[kb][i] = -INFINITY;
+            if (key >= left) sacc[kb][i] = -INFINITY;
           }
       }
 
@@ -333,6 +340,7 @@ __device__ __forceinline__ void attn_workgroup_fp8(unsigned char* smem) {
           }
         });
       }
+      left = left_next;
     }
     asm volatile("" : "+s"(pp));  // from here on the kernel arguments are read afresh
 
@@ -497,9 +505,6 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 3) void attn_fwd_fp8_kernel(
   attn_workgroup_fp8<TO, D, NW, FUSED>(smem);
 }
 
-// Workgroups of NW wavefronts resident at once (3 wavefronts per SIMD by registers; 2 for NW = 8).
-static int resident_workgroups(int NW, int planned_cus) { return resident_cus(planned_cus) * (NW == 4 ? 3 : 1); }
-
 template <typename TO, int D, int NW, bool FUSED>
 static hipError_t launch_one(const AttnParams& p, hipStream_t stream) {
   AttnParams q = p;
@@ -508,7 +513,7 @@ static hipError_t launch_one(const AttnParams& p, hipStream_t stream) {
   q.total_tiles = p.B * p.H * q.nq_tiles;
   q.tiles_per_xcd = (q.total_tiles + 7) / 8;
   // the ring step takes a balanced plan only when the attention kernel folds the parts itself (the fold goes on into the accumulator)
-  bind_workspace(q, p, plan_split(q, rows, resident_workgroups(NW, p.cu_count), D, 2, 1, false, FUSED), rows, D, 2);
+  bind_workspace(q, p, plan_split(q, rows, resident_cus(p.cu_count) * workgroups_per_cu(true, D, rows), D, 2, 1, false, FUSED), rows, D, 2);
   static std::atomic<bool> lds_ready[kMaxDevices];
   constexpr int lds = lds_bytes<D, NW>();
   const int slot = current_device_slot();
@@ -536,7 +541,7 @@ static size_t workspace_one(const AttnParams& p, AttnParams* plan, bool fold_onl
   q.nq_tiles = (p.Sq + rows - 1) / rows;
   q.total_tiles = p.B * p.H * q.nq_tiles;
   q.tiles_per_xcd = (q.total_tiles + 7) / 8;
-  const size_t need = plan_split(q, rows, resident_workgroups(NW, p.cu_count), D, 2, 1, false, fold_only);
+  const size_t need = plan_split(q, rows, resident_cus(p.cu_count) * workgroups_per_cu(true, D, rows), D, 2, 1, false, fold_only);
   if (plan != nullptr) *plan = q;
   return need;
 }

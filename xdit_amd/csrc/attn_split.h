@@ -323,6 +323,16 @@ static inline int resident_cus(int planned = 0) {
   return n;
 }
 
+// Workgroups of an attention kernel that a launch is planned to have resident on a compute unit.  One of
+// the larger shapes and, of 128 rows, two (16-bit) or three (fp8), by the registers.  The fp8 kernel at
+// head_dim 64 needs at most 128 registers: four wavefronts share a SIMD, i.e. four 128-row or two 256-row
+// workgroups a compute unit, which is also where it is fastest (B*H = 96, S = 17776: 5.47 ms with
+// either against 6.16 ms for one 384-row workgroup).
+static inline int workgroups_per_cu(bool fp8, int D, int rows) {
+  if (fp8 && D == 64) return rows == 128 ? 4 : (rows == 256 ? 2 : 1);
+  return rows == 128 ? (fp8 ? 3 : 2) : 1;
+}
+
 // Ranges shorter than this many KV iterations are not worth a claim of their own (prologue,
 // epilogue and partial result of a segment cost about four iterations).
 constexpr int kMinClaimLen = 64;
