@@ -323,6 +323,13 @@ typedef struct {
 int xdit_fp8_quant(const xdit_quant_args* args);
 
 /*
+ * Up to four quantiser calls (the q, k and v of one attention call) in the same launches: `jobs` is an
+ * array of `count` structs of one in_dtype and one stream, each as for xdit_fp8_quant.  Jobs with
+ * scratch must not share it.  The results are those of `count` single calls, bit for bit.
+ */
+int xdit_fp8_quant_batch(const xdit_quant_args* jobs, int32_t count);
+
+/*
  * Pre-attention prologue of an xDiT attention processor, fused into one pass over Q (or K):
  *     y = rotary(norm(x)), written through its own strides (e.g. BSHD in, BHSD-contiguous out)
  * replacing `attn.norm_q(query)`, `apply_rotary_emb(query, image_rotary_emb)` and the later

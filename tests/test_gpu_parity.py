@@ -1480,3 +1480,29 @@ def test_claimed_ranges_in_a_graph_and_on_two_streams(gpu, force_rows):
     for a, b in outs:
         assert torch.equal(a[0], want[0]) and torch.equal(a[1], want[1])
         assert torch.equal(b[0], want2[0]) and torch.equal(b[1], want2[1])
+
+
+@pytest.mark.parametrize("S,Sq,D,S2,dtype", [(1, 3, 128, 0, torch.bfloat16), (129, 64, 64, 5, torch.float16), (500, 700, 72, 33, torch.bfloat16),
+                                             (37, 4, 256, 200, torch.float32)])
+@pytest.mark.parametrize("per_tensor", [False, True])
+def test_fp8_quant_batch_equals_single_calls(gpu, S, Sq, D, S2, dtype, per_tensor):
+    """Tensors of different lengths quantised in one batch (the jobs' workgroups share a grid sized for
+    the largest) against one call per tensor, bit for bit, with and without rotation, a second tensor and
+    a static scale; scales down to where the division by reciprocal hands over to the true division,
+    against torch's division."""
+    g = torch.Generator().manual_seed(S + D)
+    q, k, v = (torch.randn(2, 3, n, D, generator=g).to(dtype).to(gpu) for n in (Sq, S, S))
+    k2 = torch.randn(2, 3, S2, D, generator=g).to(dtype).to(gpu) if S2 else None
+    block = 64 if D % 64 == 0 else 8
+    static = torch.tensor([0.037], device=gpu)
+    jobs = [(q, per_tensor, None, block, None), (k, per_tensor, None, block, k2), (v, per_tensor, static, 0, None)]
+    for got, (x, pt, scale, had, x2) in zip(ops.fp8_quant_batch(jobs), jobs):
+        want = ops.fp8_quant(x, per_tensor=pt, scale=scale, hadamard_block=had, x2=x2)
+        assert len(got) == len(want) == (2 if x2 is None else 3)
+        for a, b in zip(got, want):
+            assert torch.equal(a.view(torch.uint8) if a.dtype == torch.float8_e4m3fn else a, b.view(torch.uint8) if b.dtype == torch.float8_e4m3fn else b)
+    for scale in (2.0 ** -81, 1.7 * 2.0 ** -80, 3e-5, 0.9999999, 1.1 * 2.0 ** 79, 2.0 ** 81):
+        x = (torch.randn(1, 1, 64, D, generator=g).clamp(-4, 4) * 100).float().to(gpu) * scale
+        y, _ = ops.fp8_quant(x, per_tensor=True, scale=torch.tensor([scale], device=gpu))
+        quotient = x / torch.full_like(x, scale)   # a tensor: torch turns the division by a number into a product
+        assert torch.equal(y.view(torch.uint8), quotient.to(torch.float8_e4m3fn).view(torch.uint8))

@@ -184,7 +184,7 @@ class PrologueArgs(ctypes.Structure):
 NORM_NONE, NORM_HEAD, NORM_TOKEN = 0, 1, 2
 ROPE_NONE, ROPE_INTERLEAVED, ROPE_SPLIT_HALF, ROPE_WAN = 0, 1, 2, 3
 
-EXPORTS = ("xdit_attn_fwd", "xdit_attn_fwd_noalloc", "xdit_attn_fwd_accumulate", "xdit_attn_workspace_bytes", "xdit_attn_launch_plan", "xdit_lse_merge", "xdit_fp8_quant", "xdit_qk_prologue", "xdit_qk_prologue_batch", "xdit_attn_last_error", "xdit_attn_abi_version")
+EXPORTS = ("xdit_attn_fwd", "xdit_attn_fwd_noalloc", "xdit_attn_fwd_accumulate", "xdit_attn_workspace_bytes", "xdit_attn_launch_plan", "xdit_lse_merge", "xdit_fp8_quant", "xdit_fp8_quant_batch", "xdit_qk_prologue", "xdit_qk_prologue_batch", "xdit_attn_last_error", "xdit_attn_abi_version")
 
 _lib = None
 _lock = threading.Lock()
@@ -218,6 +218,8 @@ def lib():
         L.xdit_lse_merge.restype = ctypes.c_int
         L.xdit_fp8_quant.argtypes = [ctypes.POINTER(QuantArgs)]
         L.xdit_fp8_quant.restype = ctypes.c_int
+        L.xdit_fp8_quant_batch.argtypes = [ctypes.POINTER(QuantArgs), ctypes.c_int32]
+        L.xdit_fp8_quant_batch.restype = ctypes.c_int
         L.xdit_qk_prologue.argtypes = [ctypes.POINTER(PrologueArgs)]
         L.xdit_qk_prologue.restype = ctypes.c_int
         L.xdit_qk_prologue_batch.argtypes = [ctypes.POINTER(PrologueArgs), ctypes.c_int32]

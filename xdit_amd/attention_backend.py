@@ -156,20 +156,29 @@ def _mi355_fp8_attn_call(query, key, value, dropout_p, is_causal, attention_kwar
     if had > 1 and query.shape[-1] % had != 0:
         had = 0
     static = kw.get("fp8_static_scale", FP8_STATIC_SCALE)
-    # rotating q and k alike leaves q.k unchanged and spreads outliers before the fp8 cast
-    q8, qd = per_tensor_quant(query, scale=static, hadamard_block=had)
-    if jk is None:
-        k8, kd = per_tensor_quant(key, scale=static, hadamard_block=had)
-        v8, vd = per_tensor_quant(value, scale=static)
-        k2 = v2 = None
-    else:
-        # the joint keys / values share the scale of the keys / values they are attended with (one
-        # abs-max over both, as quantising their concatenation would give) and go to the kernel as
-        # its second KV segment: no concatenated copy of K and V is made
-        k8, k2, kd = per_tensor_quant(key, scale=static, hadamard_block=had, x2=jk)
-        v8, v2, vd = per_tensor_quant(value, scale=static, x2=jv)
-        if strategy == "front":
-            k8, v8, k2, v2 = k2, v2, k8, v8
+    # rotating q and k alike leaves q.k unchanged and spreads outliers before the fp8 cast.  The joint
+    # keys / values share the scale of the keys / values they are attended with (one abs-max over both,
+    # as quantising their concatenation would give) and go to the kernel as its second KV segment: no
+    # concatenated copy of K and V is made.
+    k2 = v2 = None
+    if torch.compiler.is_compiling():
+        q8, qd = per_tensor_quant(query, scale=static, hadamard_block=had)
+        if jk is None:
+            k8, kd = per_tensor_quant(key, scale=static, hadamard_block=had)
+            v8, vd = per_tensor_quant(value, scale=static)
+        else:
+            k8, k2, kd = per_tensor_quant(key, scale=static, hadamard_block=had, x2=jk)
+            v8, v2, vd = per_tensor_quant(value, scale=static, x2=jv)
+    else:  # the three tensors in the same launches
+        scale_in = None if static is None else torch.as_tensor(static, dtype=torch.float32, device=query.device).reshape(1)
+        (q8, qd), kq, vq = ops.fp8_quant_batch([(query, True, scale_in, had, None), (key, True, scale_in, had, jk),
+                                                (value, True, scale_in, 0, jv)])
+        if jk is None:
+            (k8, kd), (v8, vd) = kq, vq
+        else:
+            (k8, k2, kd), (v8, v2, vd) = kq, vq
+    if strategy == "front":
+        k8, v8, k2, v2 = k2, v2, k8, v8
     if torch.compiler.is_compiling():
         if k2 is None:
             return torch.ops.xdit_amd.attn_fwd_fp8(q8, k8, v8, qd, kd, vd, scale, out_dtype == torch.float16)

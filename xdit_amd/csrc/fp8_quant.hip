@@ -10,9 +10,13 @@
 // be captured in a HIP graph), (2) abs-max reduction with one atomic max per workgroup, (3) scale
 // and cast, (4) turn the abs-max buffer into the descale values.  An optional second tensor (the
 // joint keys or values) shares the scales of the first.  Both tensor passes are HBM-bound and read
-// 16 bytes per lane; the division is a true fp32 division so results match the reference's
+// 16 bytes per lane; the quotient is that of a true fp32 division, so results match the reference's
 // `x / scale` bit for bit.  Optionally both passes first rotate each row along head_dim by a
 // block Hadamard matrix (_fp8_hadamard_rotate, attention_backend.py:703-714), in registers.
+// Several tensors (the q, k and v of one attention call) go through the same launches, blockIdx.z
+// selecting the tensor.  Flux-1024's q, k and v (85 MB) with the rotation of q and k: 18.6 us for the
+// abs-max (4.6 TB/s) and 32.2 us for the cast (4.0 TB/s), two launches; with a launch pair per tensor, the
+// rotation by shuffles and a compiler-made division it was six launches and 116 us.
 #include "common.h"
 #include "launchers.h"
 
@@ -36,10 +40,37 @@ template <> __device__ __forceinline__ void load8<_Float16>(const _Float16* p, f
   for (int i = 0; i < 8; i++) x[i] = (float)v[i];
 }
 
+// The value of the lane whose index differs in exactly bit log2(M) (M = 1, 2, 4 or 8), within the 16
+// lanes of a DPP row: quad permutes, the rotation by 8, and for 4 the half-row mirror (lane ^ 7)
+// followed by the quad mirror (^ 3).  A DPP operand rides on the addition that uses it, where a
+// shuffle is an LDS-pipe instruction per value and level (32 of them per 8 elements at block 128).
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+template <int M>
+__device__ __forceinline__ float lane_xor(float x) {
+  static_assert(M == 1 || M == 2 || M == 4 || M == 8, "within a DPP row");
+  if constexpr (M == 1) return dpp_move<0xB1>(x);        // quad_perm [1,0,3,2]
+  else if constexpr (M == 2) return dpp_move<0x4E>(x);   // quad_perm [2,3,0,1]
+  else if constexpr (M == 4) return dpp_move<0x1B>(dpp_move<0x141>(x));  // row_half_mirror, quad_perm [3,2,1,0]
+  else return dpp_move<0x128>(x);                        // row_ror:8
+}
+// One butterfly level across chunks: the upper chunk of a pair takes (other - own), the lower (own + other).
+template <int M>
+__device__ __forceinline__ void hadamard_level(float (&v)[8], int c) {
+  const unsigned flip = (c & M) != 0 ? 0x80000000u : 0u;
+#pragma unroll
+  for (int j = 0; j < 8; j++) {
+    const float own = __uint_as_float(__float_as_uint(v[j]) ^ flip);
+    v[j] = lane_xor<M>(v[j]) + own;
+  }
+}
+
 // Rotates the rows by the Sylvester-Hadamard matrix of size `block` along head_dim, in place in
 // the 8-element chunks the threads hold: the three butterfly levels inside a chunk in
 // registers, the levels across chunks by exchanging with the lane that holds chunk c ^ m of the
-// same row (the chunks of a block sit in consecutive, block-aligned lanes of one wavefront).
+// same row (the chunks of a block, at most 16, sit in consecutive, block-aligned lanes of one wavefront).
 // Entries are +-r with r = `scale` rounded to T and the result is rounded to T, like the output
 // of a matmul with the matrix held in T.  `c` is the chunk's index within its row.
 template <typename T>
@@ -59,14 +90,10 @@ __device__ __forceinline__ void hadamard_rows(float (&v)[8], int block, float sc
 #pragma unroll
     for (int i = 0; i < 4; i++) { const float a = v[i], b = v[i + 4]; v[i] = a + b; v[i + 4] = a - b; }
   }
-  for (int m = 1; m * 8 < block; m <<= 1) {
-    const bool upper = (c & m) != 0;
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const float o = __shfl_xor(v[j], m);
-      v[j] = upper ? o - v[j] : v[j] + o;
-    }
-  }
+  if (block >= 16) hadamard_level<1>(v, c);
+  if (block >= 32) hadamard_level<2>(v, c);
+  if (block >= 64) hadamard_level<4>(v, c);
+  if (block >= 128) hadamard_level<8>(v, c);
   const float r = (float)(T)scale;
 #pragma unroll
   for (int j = 0; j < 8; j++) v[j] = (float)(T)(v[j] * r);
@@ -77,7 +104,8 @@ __global__ void fill_zero_kernel(float* p, int n) {
   if (i < n) p[i] = 0.f;
 }
 
-// Both tensor passes: grid = (blocks per slice, B*H).  A row of D elements is held by D/8
+// Both tensor passes: grid = (most blocks per slice, most B*H, tensors of the batch); a job's slices
+// have `blocks` workgroups, what is beyond them leaves at once.  A row of D elements is held by D/8
 // consecutive threads (8 elements each), a workgroup covers 256 / (D/8) rows per step and every
 // thread keeps kRowsInFlight rows in flight; rows advance by whole grid steps, so there is no
 // division in the loop and the trip count is the same for every thread of a workgroup (the
@@ -85,14 +113,15 @@ __global__ void fill_zero_kernel(float* p, int n) {
 constexpr int kRowsInFlight = 4;
 constexpr int kAbsmaxRowsInFlight = 8;  // the read-only pass: nothing but loads to keep in flight
 
-template <typename T, int kRowsInFlight = quant::kRowsInFlight, typename F>
-__device__ __forceinline__ void for_each_chunk(const QuantParams& p, const T* x, int64_t S, int64_t xs_s, F&& f) {
+// `before` runs once per step, between a step's loads and their use.
+template <typename T, int kRowsInFlight = quant::kRowsInFlight, typename G, typename F>
+__device__ __forceinline__ void for_each_chunk(const QuantParams& p, const T* x, int64_t S, int64_t xs_s, int blocks, G&& before, F&& f) {
   const int cpr = p.D >> 3;
   const int rpb = 256 / cpr;              // rows per workgroup step
   const int c = threadIdx.x % cpr;
   const int r = threadIdx.x / cpr;
   const bool lane_live = r < rpb;
-  const int64_t step = (int64_t)gridDim.x * rpb;
+  const int64_t step = (int64_t)blocks * rpb;
   for (int64_t base = (int64_t)blockIdx.x * rpb; base < S; base += step * kRowsInFlight) {
     float v[kRowsInFlight][8];
     int64_t s[kRowsInFlight];
@@ -102,6 +131,7 @@ __device__ __forceinline__ void for_each_chunk(const QuantParams& p, const T* x,
       const int64_t sc = s[j] < S ? s[j] : S - 1;  // rows past the end re-read the last row
       load8<T>(x + sc * xs_s + c * 8, v[j]);
     }
+    before();
 #pragma unroll
     for (int j = 0; j < kRowsInFlight; j++) {
       if (p.had_block > 1) hadamard_rows<T>(v[j], p.had_block, p.had_scale, c);
@@ -125,8 +155,10 @@ __device__ __forceinline__ float block_max(float m) {
 // its maximum in a slot of its own (no clearing, no atomics); otherwise one atomic max per
 // workgroup goes to the slice's entry of the (cleared) amax buffer.
 template <typename T>
-__global__ __launch_bounds__(256) void absmax_kernel(const QuantParams p) {
+__global__ __launch_bounds__(256) void absmax_kernel(const QuantBatch batch) {
+  const QuantParams& p = batch.job[blockIdx.z];
   const int bh = blockIdx.y;
+  if ((int)blockIdx.x >= p.reduce_blocks || bh >= p.B * p.H) return;
   const int b = bh / p.H, h = bh - b * p.H;
   float m = 0.f;
   auto take = [&](float (&v)[8], int64_t, int, bool live) {
@@ -135,42 +167,73 @@ __global__ __launch_bounds__(256) void absmax_kernel(const QuantParams p) {
       for (int j = 0; j < 8; j++) m = fmaxf(m, fabsf(v[j]));  // fmaxf drops NaN operands
     }
   };
-  for_each_chunk<T, kAbsmaxRowsInFlight>(p, (const T*)p.x + b * p.xs_b + h * p.xs_h, p.S, p.xs_s, take);
-  if (p.S2 > 0) for_each_chunk<T, kAbsmaxRowsInFlight>(p, (const T*)p.x2 + b * p.x2s_b + h * p.x2s_h, p.S2, p.x2s_s, take);
+  for_each_chunk<T, kAbsmaxRowsInFlight>(p, (const T*)p.x + b * p.xs_b + h * p.xs_h, p.S, p.xs_s, p.reduce_blocks, [] {}, take);
+  if (p.S2 > 0) for_each_chunk<T, kAbsmaxRowsInFlight>(p, (const T*)p.x2 + b * p.x2s_b + h * p.x2s_h, p.S2, p.x2s_s, p.reduce_blocks, [] {}, take);
   m = block_max(m);
   if (threadIdx.x == 0) {
-    if (p.partials != nullptr) p.partials[(int64_t)bh * gridDim.x + blockIdx.x] = m;
+    if (p.partials != nullptr) p.partials[(int64_t)bh * p.reduce_blocks + blockIdx.x] = m;
     // non-negative floats order like their bit patterns
     else atomicMax((unsigned int*)(p.amax + (p.per_tensor ? 0 : bh)), __float_as_uint(m));
   }
 }
 
-// Scale and cast of a (batch, head) slice of both tensors.  The scale is the static one, or comes
-// from the partial maxima of the abs-max pass (folded here by every workgroup; the first
-// workgroup of a slice also stores the slice's descale), or from the amax buffer.
-template <typename T>
-__global__ __launch_bounds__(256) void cast_kernel(const QuantParams p, const int partials_per_slice) {
-  const int bh = blockIdx.y;
-  const int b = bh / p.H, h = bh - b * p.H;
-  float scale;
-  if (p.scale_in != nullptr) {
-    scale = *p.scale_in;
-  } else if (p.partials != nullptr) {
-    const int n = p.per_tensor ? partials_per_slice * (int)gridDim.y : partials_per_slice;
-    const float* src = p.partials + (p.per_tensor ? 0 : (int64_t)bh * partials_per_slice);
-    float am = 0.f;
-    for (int i = threadIdx.x; i < n; i += 256) am = fmaxf(am, src[i]);
-    am = block_max(am);
-    scale = am > 0.f ? am / kFp8Max : 1.0f;
-  } else {
-    const float am = p.amax[p.per_tensor ? 0 : bh];
-    scale = am > 0.f ? am / kFp8Max : 1.0f;
+// x / scale with the rounding of a true fp32 division, in three instructions instead of the dozen of
+// the compiler's sequence: with r the correctly rounded 1 / scale, q = x r is within one unit of the
+// quotient, the remainder x - q scale is exact in one fused multiply-add, and q + r (x - q scale) rounds
+// to the quotient's nearest (Markstein, "Computation of elementary functions on the IBM RISC System/6000
+// processor", 1990).  That needs the remainder's and the reciprocal's exponents in range:
+// scales outside [2^-80, 2^80] take the division itself.
+struct Divider {
+  float scale, r;
+  bool plain;
+  __device__ __forceinline__ explicit Divider(float s) : scale(s), r(1.0f / s), plain(!(s >= 0x1p-80f && s <= 0x1p80f)) {}
+  __device__ __forceinline__ float operator()(float x) const {
+    const float q = x * r;
+    return __builtin_fmaf(__builtin_fmaf(-q, scale, x), r, q);
   }
-  if ((p.scale_in != nullptr || p.partials != nullptr) && blockIdx.x == 0 && threadIdx.x == 0) p.descale[bh] = scale;
+};
+
+// Scale and cast of a (batch, head) slice of both tensors.  The scale is the static one, or comes
+// from the partial maxima of the abs-max pass (folded here by every workgroup while its first rows
+// are on their way; the first workgroup of a slice also stores the slice's descale), or from the amax
+// buffer.
+template <typename T>
+__global__ __launch_bounds__(256) void cast_kernel(const QuantBatch batch) {
+  const QuantParams& p = batch.job[blockIdx.z];
+  const int bh = blockIdx.y;
+  if ((int)blockIdx.x >= p.cast_blocks || bh >= p.B * p.H) return;
+  const int b = bh / p.H, h = bh - b * p.H;
+  Divider div(1.0f);
+  bool have_scale = false;
+  auto need_scale = [&] {
+    if (have_scale) return;
+    have_scale = true;
+    float scale;
+    if (p.scale_in != nullptr) {
+      scale = *p.scale_in;
+    } else if (p.partials != nullptr) {
+      const int n = p.per_tensor ? p.reduce_blocks * p.B * p.H : p.reduce_blocks;
+      const float* src = p.partials + (p.per_tensor ? 0 : (int64_t)bh * p.reduce_blocks);
+      float am = 0.f;
+      for (int i = threadIdx.x; i < n; i += 256) am = fmaxf(am, src[i]);
+      am = block_max(am);
+      scale = am > 0.f ? am / kFp8Max : 1.0f;
+    } else {
+      const float am = p.amax[p.per_tensor ? 0 : bh];
+      scale = am > 0.f ? am / kFp8Max : 1.0f;
+    }
+    if ((p.scale_in != nullptr || p.partials != nullptr) && blockIdx.x == 0 && threadIdx.x == 0) p.descale[bh] = scale;
+    div = Divider(scale);
+  };
   auto cast_to = [&](unsigned char* y, int64_t ys_s) {
     return [&, y, ys_s](float (&v)[8], int64_t s, int c, bool live) {
+      if (div.plain) {
 #pragma unroll
-      for (int j = 0; j < 8; j++) v[j] = v[j] / scale;
+        for (int j = 0; j < 8; j++) v[j] = v[j] / div.scale;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = div(v[j]);
+      }
       int w0 = __builtin_amdgcn_cvt_pk_fp8_f32(v[0], v[1], 0, false);
       w0 = __builtin_amdgcn_cvt_pk_fp8_f32(v[2], v[3], w0, true);
       int w1 = __builtin_amdgcn_cvt_pk_fp8_f32(v[4], v[5], 0, false);
@@ -179,10 +242,10 @@ __global__ __launch_bounds__(256) void cast_kernel(const QuantParams p, const in
       if (live) *(i32x2*)(y + s * ys_s + c * 8) = w;
     };
   };
-  for_each_chunk<T>(p, (const T*)p.x + b * p.xs_b + h * p.xs_h, p.S, p.xs_s,
+  for_each_chunk<T>(p, (const T*)p.x + b * p.xs_b + h * p.xs_h, p.S, p.xs_s, p.cast_blocks, need_scale,
                     cast_to((unsigned char*)p.y + b * p.ys_b + h * p.ys_h, p.ys_s));
   if (p.S2 > 0)
-    for_each_chunk<T>(p, (const T*)p.x2 + b * p.x2s_b + h * p.x2s_h, p.S2, p.x2s_s,
+    for_each_chunk<T>(p, (const T*)p.x2 + b * p.x2s_b + h * p.x2s_h, p.S2, p.x2s_s, p.cast_blocks, need_scale,
                       cast_to((unsigned char*)p.y2 + b * p.y2s_b + h * p.y2s_h, p.y2s_s));
 }
 
@@ -198,49 +261,59 @@ __global__ void finalize_kernel(const QuantParams p, int n) {
 }
 
 template <typename T>
-static hipError_t run(const QuantParams& p, hipStream_t stream) {
-  const int BH = p.B * p.H;
-  const int rpb = 256 / (p.D >> 3);
-  const int64_t rows = (int64_t)p.S + p.S2;
-  int per_slice = (int)((rows + rpb * 2 * quant::kRowsInFlight - 1) / (rpb * 2 * quant::kRowsInFlight));  // ~8 rows per thread
-  if (per_slice < 1) per_slice = 1;
-  if (per_slice > 2048) per_slice = 2048;
-  dim3 grid(per_slice, BH), block(256);
-  int partials_per_slice = 0;
-  if (p.scale_in == nullptr) {
-    int reduce_slice;
-    if (p.partials != nullptr) {
-      // one slot per workgroup: as many workgroups as the scratch holds slots for
-      reduce_slice = (int)(p.partial_slots / BH);
-      if (reduce_slice > per_slice) reduce_slice = per_slice;
-      if (reduce_slice < 1) return hipErrorInvalidValue;
-      partials_per_slice = reduce_slice;
-    } else {
-      // every workgroup ends in one atomic max on its slice's entry: keep their number near 1024,
-      // same-address atomics are served one at a time
-      reduce_slice = 1024 / BH;
-      if (reduce_slice < 1) reduce_slice = 1;
-      if (reduce_slice > per_slice) reduce_slice = per_slice;
-      hipLaunchKernelGGL(fill_zero_kernel, dim3((BH + 255) / 256), dim3(256), 0, stream, p.amax, BH);
+static hipError_t run(QuantBatch& batch, hipStream_t stream) {
+  int cast_x = 1, reduce_x = 0, bh_max = 1;
+  for (int i = 0; i < batch.n; i++) {
+    QuantParams& p = batch.job[i];
+    const int BH = p.B * p.H;
+    const int rpb = 256 / (p.D >> 3);
+    const int64_t rows = (int64_t)p.S + p.S2;
+    int per_slice = (int)((rows + rpb * 2 * quant::kRowsInFlight - 1) / (rpb * 2 * quant::kRowsInFlight));  // ~8 rows per thread
+    if (per_slice < 1) per_slice = 1;
+    if (per_slice > 2048) per_slice = 2048;
+    p.cast_blocks = per_slice;
+    p.reduce_blocks = 0;
+    if (p.scale_in == nullptr) {
+      if (p.partials != nullptr) {
+        // one slot per workgroup: as many workgroups as the scratch holds slots for
+        p.reduce_blocks = (int)(p.partial_slots / BH);
+        if (p.reduce_blocks > per_slice) p.reduce_blocks = per_slice;
+        if (p.reduce_blocks < 1) return hipErrorInvalidValue;
+      } else {
+        // every workgroup ends in one atomic max on its slice's entry: keep their number near 1024,
+        // same-address atomics are served one at a time
+        p.reduce_blocks = 1024 / BH;
+        if (p.reduce_blocks < 1) p.reduce_blocks = 1;
+        if (p.reduce_blocks > per_slice) p.reduce_blocks = per_slice;
+        hipLaunchKernelGGL(fill_zero_kernel, dim3((BH + 255) / 256), dim3(256), 0, stream, p.amax, BH);
+      }
     }
-    hipLaunchKernelGGL((absmax_kernel<T>), dim3(reduce_slice, BH), block, 0, stream, p);
+    if (p.cast_blocks > cast_x) cast_x = p.cast_blocks;
+    if (p.reduce_blocks > reduce_x) reduce_x = p.reduce_blocks;
+    if (BH > bh_max) bh_max = BH;
   }
-  hipLaunchKernelGGL((cast_kernel<T>), grid, block, 0, stream, p, partials_per_slice);
-  if (p.scale_in == nullptr && p.partials == nullptr) {
-    // per_tensor broadcasts entry 0: keep it to one workgroup so the barrier orders read/write
-    if (p.per_tensor && BH > 1024) return hipErrorInvalidValue;
-    const int fb = p.per_tensor ? BH : 256;
-    hipLaunchKernelGGL(finalize_kernel, dim3((BH + fb - 1) / fb), dim3(fb < 64 ? 64 : fb), 0, stream, p, BH);
+  const dim3 block(256);
+  if (reduce_x > 0) hipLaunchKernelGGL((absmax_kernel<T>), dim3(reduce_x, bh_max, batch.n), block, 0, stream, batch);
+  hipLaunchKernelGGL((cast_kernel<T>), dim3(cast_x, bh_max, batch.n), block, 0, stream, batch);
+  for (int i = 0; i < batch.n; i++) {
+    const QuantParams& p = batch.job[i];
+    if (p.scale_in == nullptr && p.partials == nullptr) {
+      // per_tensor broadcasts entry 0: keep it to one workgroup so the barrier orders read/write
+      const int BH = p.B * p.H;
+      if (p.per_tensor && BH > 1024) return hipErrorInvalidValue;
+      const int fb = p.per_tensor ? BH : 256;
+      hipLaunchKernelGGL(finalize_kernel, dim3((BH + fb - 1) / fb), dim3(fb < 64 ? 64 : fb), 0, stream, p, BH);
+    }
   }
   return hipGetLastError();
 }
 
 }  // namespace quant
 
-hipError_t launch_fp8_quant(const QuantParams& p, int in_dtype, hipStream_t stream) {
-  if (in_dtype == 0) return quant::run<__bf16>(p, stream);
-  if (in_dtype == 1) return quant::run<_Float16>(p, stream);
-  if (in_dtype == 2) return quant::run<float>(p, stream);
+hipError_t launch_fp8_quant(QuantBatch& b, int in_dtype, hipStream_t stream) {
+  if (in_dtype == 0) return quant::run<__bf16>(b, stream);
+  if (in_dtype == 1) return quant::run<_Float16>(b, stream);
+  if (in_dtype == 2) return quant::run<float>(b, stream);
   return hipErrorInvalidValue;
 }
 

@@ -47,6 +47,15 @@ struct QuantParams {
   // optional scratch: partial_slots floats, one per workgroup of the abs-max pass
   float* partials;
   int64_t partial_slots;
+  // filled by the launcher: workgroups per (batch, head) slice in the abs-max and in the cast pass
+  int reduce_blocks, cast_blocks;
+};
+
+// Up to kQuantBatchMax quantiser calls of one input dtype in the same launches.
+constexpr int kQuantBatchMax = 4;
+struct QuantBatch {
+  QuantParams job[kQuantBatchMax];
+  int n;
 };
 
 // Parameters of one prologue launch (RMSNorm + rotary embedding + re-layout of Q or K).
@@ -83,7 +92,7 @@ hipError_t launch_attn_fwd_fp8(const AttnParams& p, int D, int out_is_fp16, int 
 size_t attn_fwd_fp8_workspace(const AttnParams& p, int D, int rows_per_block, AttnParams* plan = nullptr, bool fold_only = false);
 hipError_t launch_attn_fwd_f32(const AttnParams& p, int D, hipStream_t stream);  // fp32 tensors only
 int attn_fwd_f32_rows(const AttnParams& p);  // query rows per workgroup the fp32 launch takes: 128, or 64 (64-key tiles split between wavefront pairs)
-hipError_t launch_fp8_quant(const QuantParams& p, int in_dtype, hipStream_t stream);
+hipError_t launch_fp8_quant(QuantBatch& b, int in_dtype, hipStream_t stream);
 hipError_t launch_qk_prologue(const PrologueParams& p, int dtype, hipStream_t stream);
 hipError_t launch_qk_prologue_batch(const PrologueBatch& b, int dtype, hipStream_t stream);
 int prologue_max_token_elems();

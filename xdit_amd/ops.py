@@ -375,6 +375,78 @@ def lse_merge(acc_out, acc_lse, block_out, block_lse, first=False, final_out=Non
 _QUANT_SCRATCH = {}
 
 
+def _quant_job(a, x, per_tensor, hadamard_block, x2):
+    """Fills the fields of a QuantArgs that the shapes, strides and options decide."""
+    device = x.device
+    _check4("x", x, device)
+    B, H, S, D = x.shape
+    a.struct_size = ctypes.sizeof(_lib.QuantArgs)
+    a.in_dtype = _code(x.dtype)
+    a.per_tensor = 1 if per_tensor else 0
+    a.hadamard_block = int(hadamard_block)
+    a.B, a.H, a.D, a.S = B, H, D, S
+    a.x_stride, a.y_stride = _strides(x), _lib.Strides(H * S * D, S * D, D)
+    if x2 is not None:
+        _check4("x2", x2, device)
+        if x2.shape[0] != B or x2.shape[1] != H or x2.shape[3] != D or x2.dtype != x.dtype:
+            raise ValueError("x2 %s does not match x %s" % (tuple(x2.shape), tuple(x.shape)))
+        S2 = x2.shape[2]
+        if S2 > 0:
+            a.S2 = S2
+            a.x2_stride, a.y2_stride = _strides(x2), _lib.Strides(H * S2 * D, S2 * D, D)
+
+
+def fp8_quant_batch(jobs):
+    """Up to four `fp8_quant` calls (tuples x, per_tensor, scale, hadamard_block, x2) on tensors of one
+    dtype and device in the same launches -> list of (y, descale) or (y, y2, descale).  The outputs
+    are new tensors; the argument structs are kept per signature and thread like those of `attn_fwd`."""
+    device = jobs[0][0].device
+    key = ("quant",) + tuple((_sig(x), bool(pt), scale is not None, int(had), _sig(x2)) for x, pt, scale, had, x2 in jobs)
+    plans = _TLS.__dict__.setdefault("plans", {})
+    arr = plans.get(key)
+    n = len(jobs)
+    if arr is None:
+        arr = (_lib.QuantArgs * n)()
+        for a, (x, pt, scale, had, x2) in zip(arr, jobs):
+            _quant_job(a, x, pt, had, x2)
+            if x.device != device:
+                raise ValueError("the tensors of a batch must be on one device")
+        if len(plans) >= _PLANS_MAX:
+            plans.clear()
+        plans[key] = arr
+    stream = _stream(device)
+    need = [4 * max(4096, a.B * a.H) for a in arr]
+    buf = _QUANT_SCRATCH.get((device, stream))
+    if buf is None or buf.numel() < sum(need):
+        buf = torch.empty(sum(need), dtype=torch.uint8, device=device)
+        _QUANT_SCRATCH[(device, stream)] = buf
+    scratch = buf.data_ptr()
+    keep, out = [], []
+    for a, size, (x, pt, scale, had, x2) in zip(arr, need, jobs):
+        y = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=device)
+        descale = torch.empty(x.shape[:2], dtype=torch.float32, device=device)
+        a.x, a.y, a.descale = x.data_ptr(), y.data_ptr(), descale.data_ptr()
+        if scale is not None:
+            scale = scale.to(device=device, dtype=torch.float32).reshape(1).contiguous()
+            keep.append(scale)
+            a.scale_in = scale.data_ptr()
+        a.stream = stream
+        a.scratch, a.scratch_bytes = scratch, size
+        scratch += size
+        if x2 is None:
+            out.append((y, descale))
+        else:
+            y2 = torch.empty(x2.shape, dtype=torch.float8_e4m3fn, device=device)
+            if a.S2:
+                a.x2, a.y2 = x2.data_ptr(), y2.data_ptr()
+            out.append((y, y2, descale))
+    with _on_device(device):
+        rc = _lib.lib().xdit_fp8_quant_batch(arr, n)
+    if rc != 0:
+        _lib.check(rc)
+    return out
+
+
 def fp8_quant(x, per_tensor=False, scale=None, hadamard_block=0, x2=None):
     """Abs-max fp8 quantiser on a logical BHSD tensor -> (y float8_e4m3fn BHSD-contiguous,
     descale (B,H) fp32).  `per_tensor` takes one abs-max over the whole tensor (the reference's
@@ -382,43 +454,7 @@ def fp8_quant(x, per_tensor=False, scale=None, hadamard_block=0, x2=None):
     (a power of two dividing head_dim) rotates the rows by a block Hadamard matrix first.
     `x2` (logical (B,H,S2,D), e.g. the joint keys) is quantised with the same scales, the abs-max
     taken over both tensors; the result is then (y, y2, descale)."""
-    device = x.device
-    _check4("x", x, device)
-    B, H, S, D = x.shape
-    y = torch.empty((B, H, S, D), dtype=torch.float8_e4m3fn, device=device)
-    descale = torch.empty((B, H), dtype=torch.float32, device=device)
-    a = _lib.QuantArgs()
-    a.struct_size = ctypes.sizeof(_lib.QuantArgs)
-    a.in_dtype = _code(x.dtype)
-    a.per_tensor = 1 if per_tensor else 0
-    a.hadamard_block = int(hadamard_block)
-    a.B, a.H, a.D, a.S = B, H, D, S
-    a.x, a.y, a.descale = x.data_ptr(), y.data_ptr(), descale.data_ptr()
-    y2 = None
-    if x2 is not None:
-        _check4("x2", x2, device)
-        if x2.shape[0] != B or x2.shape[1] != H or x2.shape[3] != D or x2.dtype != x.dtype:
-            raise ValueError("x2 %s does not match x %s" % (tuple(x2.shape), tuple(x.shape)))
-        y2 = torch.empty(tuple(x2.shape), dtype=torch.float8_e4m3fn, device=device)
-        if x2.shape[2] > 0:
-            a.S2 = x2.shape[2]
-            a.x2, a.y2 = x2.data_ptr(), y2.data_ptr()
-            a.x2_stride, a.y2_stride = _strides(x2), _strides(y2)
-    if scale is not None:
-        scale = scale.to(device=device, dtype=torch.float32).reshape(1).contiguous()
-        a.scale_in = scale.data_ptr()
-    a.x_stride, a.y_stride = _strides(x), _strides(y)
-    stream = _stream(device)
-    a.stream = stream
-    need = 4 * max(4096, B * H)
-    buf = _QUANT_SCRATCH.get((device, stream))
-    if buf is None or buf.numel() < need:
-        buf = torch.empty(need, dtype=torch.uint8, device=device)
-        _QUANT_SCRATCH[(device, stream)] = buf
-    a.scratch, a.scratch_bytes = buf.data_ptr(), buf.numel()
-    with _on_device(device):
-        _lib.check(_lib.lib().xdit_fp8_quant(ctypes.byref(a)))
-    return (y, descale) if x2 is None else (y, y2, descale)
+    return fp8_quant_batch([(x, per_tensor, scale, hadamard_block, x2)])[0]
 
 
 _NORM_MODES = {None: _lib.NORM_NONE, "none": _lib.NORM_NONE, "head": _lib.NORM_HEAD, "token": _lib.NORM_TOKEN}
