@@ -1506,3 +1506,17 @@ def test_fp8_quant_batch_equals_single_calls(gpu, S, Sq, D, S2, dtype, per_tenso
         y, _ = ops.fp8_quant(x, per_tensor=True, scale=torch.tensor([scale], device=gpu))
         quotient = x / torch.full_like(x, scale)   # a tensor: torch turns the division by a number into a product
         assert torch.equal(y.view(torch.uint8), quotient.to(torch.float8_e4m3fn).view(torch.uint8))
+
+
+@pytest.mark.parametrize("scale", [1.0, 0.037, 3e-5, 1.0e-24, 1.0e24])
+def test_fp8_quant_static_scale_of_every_bf16_value(gpu, scale):
+    """Every bf16 value but the NaNs under a static scale: the bytes of the true division, a negative
+    zero's sign and the overflows included (the quotient through the reciprocal's remainder alone would
+    lose the former and turn an infinite quotient into a NaN of the other sign)."""
+    x = torch.arange(65536, dtype=torch.int32).to(torch.uint16).view(torch.bfloat16)
+    x = x[~x.float().isnan()]
+    x = torch.cat([x, x.new_zeros(-len(x) % 64)]).view(1, 1, -1, 64).to(gpu)
+    s = torch.tensor([scale], device=gpu)
+    y, _ = ops.fp8_quant(x, per_tensor=True, scale=s)
+    want = (x.float() / s).to(torch.float8_e4m3fn).view(torch.uint8)
+    assert torch.equal(y.view(torch.uint8), want) and (y.view(torch.uint8) == 0x80).any()

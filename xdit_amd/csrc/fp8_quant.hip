@@ -182,14 +182,17 @@ __global__ __launch_bounds__(256) void absmax_kernel(const QuantBatch batch) {
 // quotient, the remainder x - q scale is exact in one fused multiply-add, and q + r (x - q scale) rounds
 // to the quotient's nearest (Markstein, "Computation of elementary functions on the IBM RISC System/6000
 // processor", 1990).  That needs the remainder's and the reciprocal's exponents in range:
-// scales outside [2^-80, 2^80] take the division itself.
+// scales outside [2^-80, 2^80] take the division itself, and where q is a zero, an infinity or a NaN it
+// is the quotient already (the remainder would cost a negative zero its sign and make an infinity a NaN).
+constexpr int kFiniteNonZero = 0x198;  // class mask: normal and subnormal numbers of either sign
 struct Divider {
   float scale, r;
   bool plain;
   __device__ __forceinline__ explicit Divider(float s) : scale(s), r(1.0f / s), plain(!(s >= 0x1p-80f && s <= 0x1p80f)) {}
   __device__ __forceinline__ float operator()(float x) const {
     const float q = x * r;
-    return __builtin_fmaf(__builtin_fmaf(-q, scale, x), r, q);
+    const float y = __builtin_fmaf(__builtin_fmaf(-q, scale, x), r, q);
+    return __builtin_amdgcn_classf(q, kFiniteNonZero) ? y : q;
   }
 };
 
