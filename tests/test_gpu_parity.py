@@ -1520,3 +1520,28 @@ def test_fp8_quant_static_scale_of_every_bf16_value(gpu, scale):
     y, _ = ops.fp8_quant(x, per_tensor=True, scale=s)
     want = (x.float() / s).to(torch.float8_e4m3fn).view(torch.uint8)
     assert torch.equal(y.view(torch.uint8), want) and (y.view(torch.uint8) == 0x80).any()
+
+
+@pytest.mark.parametrize("dtype,D,Sk,Sk2", [(torch.bfloat16, 128, 70, 0), (torch.float16, 72, 120, 0), (torch.bfloat16, 64, 129, 40), (torch.float8_e4m3fn, 128, 200, 0)])
+@pytest.mark.parametrize("rows", [128, 256, 384])
+def test_plain_launch_of_fewer_workgroups_than_tiles(gpu, force_rows, dtype, D, Sk, Sk2, rows):
+    """A plain launch planned for eight compute units (every workgroup runs several query tiles, the last
+    ones ragged, XCDs with one tile more than others) against one workgroup per tile: the same bits, as
+    a forward and as a ring step that folds into an accumulator."""
+    g = torch.Generator().manual_seed(D + Sk)
+    f8 = dtype == torch.float8_e4m3fn
+    mk = lambda s: torch.randn(2, 5, s, D, generator=g).to(dtype).to(gpu)
+    q, k, v = mk(9 * rows + 33), mk(Sk), mk(Sk)
+    kw = dict(k2=mk(Sk2), v2=mk(Sk2)) if Sk2 else {}
+    got = []
+    for cus in (0, 8):
+        force_rows(rows)
+        ops.TUNING["cu_count"] = cus
+        try:
+            o, l = ops.attn_fwd(q, k, v, balance=False, **kw)
+            acc, al = torch.zeros(q.shape, device=gpu), torch.full(q.shape[:3], -1.0, device=gpu)
+            ops.attn_fwd_accumulate(q, k, v, acc, al, balance=False, **kw)
+        finally:
+            ops.TUNING["cu_count"] = 0
+        got.append((o, l, acc, al))
+    assert all(torch.equal(a, b) for a, b in zip(*got))

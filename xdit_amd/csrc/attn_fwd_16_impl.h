@@ -95,9 +95,10 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
   __shared__ int drawn[2];      // streamed sharing: KV tile of the stream position after next, by parity
   WorkgroupWalk walk;
   Segment seg;
+  int plain_block = (int)blockIdx.x;
   {
     const WalkGeom g = walk_geom(pp);
-    if (!walk.start(g, nt, (int)blockIdx.x) || !walk.next(g, nt, seg)) return;
+    if (!walk.start(g, nt, plain_block) || !walk.next(g, nt, seg)) return;
   }
 
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -414,6 +415,10 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
         walk.claimed(g, (unsigned)__builtin_amdgcn_readfirstlane((int)ticket));
       }
       more = walk.next(g, nt, next_seg);
+      if (!more && pp->plain_stride != 0) {  // a plain launch of fewer workgroups than tiles: on to the next tile
+        plain_block += pp->plain_stride;
+        more = plain_block < 8 * g.tiles_per_xcd && walk.start(g, nt, plain_block) && walk.next(g, nt, next_seg);
+      }
     }
     __syncthreads();  // every wavefront is done with the K/V fragments of the last tile
     if (more) {
@@ -593,6 +598,7 @@ __global__ __launch_bounds__(64 * NW, NW == 12 ? 3 : 2) void attn_fwd_16_kernel(
 template <typename T, int D, int DC, int NW, bool PAD, bool FUSED>
 static hipError_t launch_kernel(const AttnParams& q, hipStream_t stream) {
   static std::atomic<bool> lds_ready[kMaxDevices];
+  static std::atomic<int> residency[kMaxDevices];
   constexpr int lds = lds_bytes_16<D, NW>();
   const int slot = current_device_slot();
   if (!lds_ready[slot].load(std::memory_order_relaxed)) {  // > 64 KiB of dynamic LDS must be enabled once per kernel and device
@@ -600,7 +606,9 @@ static hipError_t launch_kernel(const AttnParams& q, hipStream_t stream) {
     if (e != hipSuccess) return e;
     lds_ready[slot].store(true, std::memory_order_relaxed);
   }
-  hipLaunchKernelGGL((attn_fwd_16_kernel<T, D, DC, NW, PAD, FUSED>), dim3(split_grid(q)), dim3(64 * NW), lds, stream, q);
+  AttnParams r = q;  // with plain_stride set
+  const unsigned grid = resident_grid(r, (const void*)attn_fwd_16_kernel<T, D, DC, NW, PAD, FUSED>, 64 * NW, lds, residency[slot]);
+  hipLaunchKernelGGL((attn_fwd_16_kernel<T, D, DC, NW, PAD, FUSED>), dim3(grid), dim3(64 * NW), lds, stream, r);
   return hipSuccess;
 }
 

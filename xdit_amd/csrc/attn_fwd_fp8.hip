@@ -83,9 +83,10 @@ __device__ __forceinline__ void attn_workgroup_fp8(unsigned char* smem) {
   __shared__ unsigned fold_post;  // fold duties: the slices this workgroup folds, posted by thread 0
   WorkgroupWalk walk;
   Segment seg;
+  int plain_block = (int)blockIdx.x;
   {
     const WalkGeom g = walk_geom(pp);
-    if (!walk.start(g, nt, (int)blockIdx.x) || !walk.next(g, nt, seg)) return;
+    if (!walk.start(g, nt, plain_block) || !walk.next(g, nt, seg)) return;
   }
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int lane = lane_now();   // for the set-up below; later code asks again
@@ -357,6 +358,10 @@ __device__ __forceinline__ void attn_workgroup_fp8(unsigned char* smem) {
         walk.claimed(g, (unsigned)__builtin_amdgcn_readfirstlane((int)ticket));
       }
       more = walk.next(g, nt, next_seg);
+      if (!more && pp->plain_stride != 0) {  // a plain launch of fewer workgroups than tiles: on to the next tile
+        plain_block += pp->plain_stride;
+        more = plain_block < 8 * g.tiles_per_xcd && walk.start(g, nt, plain_block) && walk.next(g, nt, next_seg);
+      }
     }
     __syncthreads();  // every wavefront is done with the K/V fragments of the last tile
     if (more) open_segment(next_seg);  // Q fragments and first K/V tile (buffer 0) of the next segment
@@ -522,7 +527,8 @@ static hipError_t launch_one(const AttnParams& p, hipStream_t stream) {
     if (e != hipSuccess) return e;
     lds_ready[slot].store(true, std::memory_order_relaxed);
   }
-  dim3 grid(split_grid(q));
+  static std::atomic<int> residency[kMaxDevices];
+  const dim3 grid(resident_grid(q, (const void*)attn_fwd_fp8_kernel<TO, D, NW, FUSED>, 64 * NW, lds, residency[slot]));
   hipLaunchKernelGGL((attn_fwd_fp8_kernel<TO, D, NW, FUSED>), grid, dim3(64 * NW), lds, stream, q);
   if constexpr (!FUSED) {
     if (q.split_units && !q.split_fold) {  // tiles of many parts: folded by a launch of its own

@@ -69,6 +69,8 @@ struct AttnParams {
   int streamed_ok;    // the caller opted in to streamed sharing (results then reproducible to rounding only)
   int split_order;    // claimers process their range BEFORE their whole query tile (see WorkgroupWalk)
   int split_fold;     // the parts of a shared tile are folded inside the attention kernel (fold duties, attn_walk.h)
+  int plain_stride;   // plain launch of fewer workgroups than query tiles: workgroup w runs tiles w, w + plain_stride, ...
+                      // of the dispatch order (0: one tile per workgroup)
   int split_policy;   // 1: plain launch; 2: balance whenever the plan shortens the critical path by kMinSaving iterations
   // ring step (optional): the result is folded into an fp32 accumulator in the epilogue
   float* acc_out;     // (B,H,Sq,D) fp32 running output, nullptr: plain forward
