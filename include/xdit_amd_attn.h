@@ -121,6 +121,23 @@ typedef struct {
 int xdit_attn_fwd(const xdit_attn_args* args);
 
 /*
+ * xdit_attn_fwd on query rows that lie in two tensors (the image and the text queries of a joint
+ * attention call): of the args->Sq rows the last tail->Sq2 are read from tail->q2, those before them
+ * from args->q.  Everything else, the result included, is that of xdit_attn_fwd on the rows copied
+ * one behind the other; sizing and planning calls take `args` as it is.  bf16 / fp16.
+ * Replaces the torch.cat of the joint query at usp.py:286-288.
+ */
+typedef struct {
+  uint32_t struct_size;        /* = sizeof(xdit_query_tail) */
+  int32_t reserved0;           /* must be 0 */
+  int64_t Sq2;                 /* 0 < Sq2 < args->Sq */
+  const void* q2;              /* (B,H,Sq2,D), dtype of q */
+  xdit_strides q2_stride;
+} xdit_query_tail;
+
+int xdit_attn_fwd_two_queries(const xdit_attn_args* args, const xdit_query_tail* tail);
+
+/*
  * Scratch bytes with which xdit_attn_fwd can balance this problem over the chip: when the number
  * of query tiles is not a multiple of what the GPU holds at once, the key/value range of the
  * tiles of the last, partly filled round is shared between workgroups, whose partial

@@ -1545,3 +1545,43 @@ def test_plain_launch_of_fewer_workgroups_than_tiles(gpu, force_rows, dtype, D, 
             ops.TUNING["cu_count"] = 0
         got.append((o, l, acc, al))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("strategy", ["front", "rear"])
+@pytest.mark.parametrize("case", ["bf16", "fp16", "fp8", "bshd", "views"])
+def test_usp_joint_queries_are_read_where_they_are(gpu, monkeypatch, strategy, case):
+    """Joint attention through USP reads the two query tensors in place: the bits of the call on their
+    concatenation (ragged row counts, so wavefronts straddle the seam), no torch.cat; with tensors whose
+    rows the kernels cannot read (misaligned, transposed, expanded, empty) the concatenation is still
+    made and the result is the same."""
+    B, H, D, Sq, Sj = 2, 3, 64, 301, 77
+    dt = torch.float16 if case == "fp16" else torch.bfloat16
+    g = torch.Generator().manual_seed(11)
+    r = lambda *s: torch.randn(*s, generator=g).to(dt).to(gpu)
+    mk = (lambda s: r(B, s, H, D).transpose(1, 2)) if case == "bshd" else (lambda s: r(B, H, s, D))
+    k, v, jk, jv = mk(Sq), mk(Sq), mk(Sj), mk(Sj)
+    backend = AB.AttentionBackendType.MI355_FP8 if case == "fp8" else AB.AttentionBackendType.MI355
+    fn = AB.ATTENTION_FUNCTION_REGISTRY[backend]
+    if case == "views":
+        pairs = [(r(B, H, Sq, D + 4)[..., 4:], mk(Sj)), (mk(Sq), r(B, H, D, Sj).transpose(2, 3)),
+                 (mk(Sq), r(1, H, 1, D).expand(B, H, Sj, D)), (mk(Sq), mk(0)), (r(B * H * Sq * D + 1)[1:].view(B, H, Sq, D), mk(Sj))]
+    else:
+        pairs = [(mk(Sq), mk(Sj)), (mk(1), mk(Sj)), (mk(385), mk(1))]
+    real_cat, cats = torch.cat, []
+    for q, jq in pairs:
+        order = [q, jq] if strategy == "rear" else [jq, q]
+        want, _ = fn(real_cat(order, 2), k, v, 0.0, False, joint_kv=(jk, jv, strategy))
+        monkeypatch.setattr(torch, "cat", lambda *a, **kw: (cats.append(1), real_cat(*a, **kw))[1])
+        got = usp.USP(q, k, v, joint_query=jq, joint_key=jk, joint_value=jv, joint_strategy=strategy, backend=backend)
+        monkeypatch.undo()
+        assert torch.equal(got, want)
+    assert len(cats) == (len(pairs) if case == "views" else 0)
+
+
+def test_two_queries_entry_refuses_what_it_cannot_read(gpu):
+    q, k = (torch.randn(1, 2, s, 64, device=gpu, dtype=torch.bfloat16) for s in (64, 32))
+    for bad in (k.float(), k[:, :1], k[..., :32], k[:, :, :0], torch.randn(1, 2, 32, 68, device=gpu, dtype=torch.bfloat16)[..., :64]):
+        with pytest.raises((ValueError, NotImplementedError)):
+            ops.attn_fwd(q, k, k, q2=bad)
+    with pytest.raises((ValueError, NotImplementedError)):
+        ops.attn_fwd(q.float(), k.float(), k.float(), q2=q.float())

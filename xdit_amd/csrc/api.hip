@@ -294,7 +294,7 @@ const char* xdit_attn_last_error(void) { return g_err; }
 
 int xdit_attn_abi_version(void) { return XDIT_ATTN_ABI_VERSION; }
 
-static int attn_fwd_impl(const xdit_attn_args* a, const xdit_ring_acc* acc) {
+static int attn_fwd_impl(const xdit_attn_args* a, const xdit_ring_acc* acc, const xdit_query_tail* tail = nullptr) {
   g_err[0] = 0;
   if (a == nullptr) return fail(XDIT_ERR_INVALID_ARG, "args is NULL");
   if (a->struct_size != sizeof(xdit_attn_args))
@@ -324,6 +324,15 @@ static int attn_fwd_impl(const xdit_attn_args* a, const xdit_ring_acc* acc) {
   }
   int rc;
   if ((rc = check_tensor("q", a->q, a->q_stride, es, a->D))) return rc;
+  if (tail != nullptr) {
+    if (tail->struct_size != sizeof(xdit_query_tail))
+      return fail(XDIT_ERR_INVALID_ARG, "tail struct_size %u != %zu (ABI mismatch)", tail->struct_size, sizeof(xdit_query_tail));
+    if (tail->reserved0 != 0) return fail(XDIT_ERR_INVALID_ARG, "tail reserved0 must be 0");
+    if (tail->Sq2 <= 0 || tail->Sq2 >= a->Sq)
+      return fail(XDIT_ERR_INVALID_ARG, "Sq2=%lld must lie between 0 and Sq=%lld", (long long)tail->Sq2, (long long)a->Sq);
+    if (!mfma16_path(a)) return fail(XDIT_ERR_UNSUPPORTED, "queries in two tensors are implemented for bf16 and fp16");
+    if ((rc = check_tensor("q2", tail->q2, tail->q2_stride, es, a->D))) return rc;
+  }
   if ((rc = check_tensor("k", a->k, a->k_stride, es, a->D))) return rc;
   if ((rc = check_tensor("v", a->v, a->v_stride, es, a->D))) return rc;
   if (a->Sk2 > 0) {
@@ -361,6 +370,12 @@ static int attn_fwd_impl(const xdit_attn_args* a, const xdit_ring_acc* acc) {
   p.ds_b = a->descale_stride_b; p.ds_h = a->descale_stride_h;
   p.B = a->B; p.H = a->H;
   p.Sq = (int)a->Sq; p.Sk = (int)a->Sk; p.Sk2 = (int)a->Sk2;
+  p.Sq1 = p.Sq;
+  if (tail != nullptr) {
+    p.q2 = tail->q2;
+    p.q2s_b = tail->q2_stride.b; p.q2s_h = tail->q2_stride.h; p.q2s_s = tail->q2_stride.s;
+    p.Sq1 = (int)(a->Sq - tail->Sq2);
+  }
   p.scale = a->softmax_scale;
   p.cu_count = a->cu_count;
   p.streamed_ok = a->streamed_sharing != 0;
@@ -411,6 +426,14 @@ static int attn_fwd_impl(const xdit_attn_args* a, const xdit_ring_acc* acc) {
 }
 
 int xdit_attn_fwd(const xdit_attn_args* a) { return attn_fwd_impl(a, nullptr); }
+
+int xdit_attn_fwd_two_queries(const xdit_attn_args* a, const xdit_query_tail* tail) {
+  if (tail == nullptr) {
+    g_err[0] = 0;
+    return fail(XDIT_ERR_INVALID_ARG, "tail is NULL");
+  }
+  return attn_fwd_impl(a, nullptr, tail);
+}
 
 int xdit_attn_fwd_noalloc(const xdit_attn_args* a) {
   g_err[0] = 0;

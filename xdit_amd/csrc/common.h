@@ -72,6 +72,10 @@ struct AttnParams {
   int plain_stride;   // plain launch of fewer workgroups than query tiles: workgroup w runs tiles w, w + plain_stride, ...
                       // of the dispatch order (0: one tile per workgroup)
   int split_policy;   // 1: plain launch; 2: balance whenever the plan shortens the critical path by kMinSaving iterations
+  // the last rows of the queries may lie in a tensor of their own: rows Sq1 .. Sq-1 are rows 0 .. of q2 (Sq1 == Sq: none do)
+  const void* q2;
+  int64_t q2s_b, q2s_h, q2s_s;
+  int Sq1;
   // ring step (optional): the result is folded into an fp32 accumulator in the epilogue
   float* acc_out;     // (B,H,Sq,D) fp32 running output, nullptr: plain forward
   float* acc_lse;     // (B,H,Sq) fp32 running log-sum-exp

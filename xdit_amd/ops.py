@@ -97,14 +97,14 @@ _PLANS_MAX = 512
 
 
 class _AttnPlan:
-    __slots__ = ("args", "need", "shape", "out_dtype", "ring")
+    __slots__ = ("args", "need", "shape", "out_dtype", "ring", "tail")
 
 
 def _sig(t):
     return None if t is None else (t.shape, t.stride(), t.device, t.dtype)
 
 
-def _build_attn_plan(q, k, v, softmax_scale, causal, k2, v2, descales, out_dtype, out, lse, acc, streamed):
+def _build_attn_plan(q, k, v, softmax_scale, causal, k2, v2, descales, out_dtype, out, lse, acc, streamed, q2=None):
     device = q.device
     for name, t in (("q", q), ("k", k), ("v", v)):
         _check4(name, t, device)
@@ -113,6 +113,16 @@ def _build_attn_plan(q, k, v, softmax_scale, causal, k2, v2, descales, out_dtype
         raise ValueError("q %s, k %s, v %s do not agree (Hq must equal Hk)" % (tuple(q.shape), tuple(k.shape), tuple(v.shape)))
     if k.dtype != q.dtype or v.dtype != q.dtype:
         raise ValueError("q, k, v must share a dtype")
+    tail = None
+    if q2 is not None:
+        _check4("q2", q2, device)
+        if q2.shape[0] != B or q2.shape[1] != H or q2.shape[3] != D or q2.dtype != q.dtype:
+            raise ValueError("q2 %s does not match q %s" % (tuple(q2.shape), tuple(q.shape)))
+        tail = _lib.QueryTail()
+        tail.struct_size = ctypes.sizeof(_lib.QueryTail)
+        tail.Sq2 = q2.shape[2]
+        tail.q2_stride = _strides(q2)
+        Sq += q2.shape[2]
     a = _lib.AttnArgs()
     a.struct_size = ctypes.sizeof(_lib.AttnArgs)
     a.dtype = _code(q.dtype)
@@ -160,6 +170,7 @@ def _build_attn_plan(q, k, v, softmax_scale, causal, k2, v2, descales, out_dtype
     plan.shape = (B, H, Sq, D)
     plan.out_dtype = out_dtype
     plan.ring = None
+    plan.tail = tail
     plan.need = 0
     if acc is not None:
         acc_out, acc_lse, first, discard = acc
@@ -193,11 +204,12 @@ def _build_attn_plan(q, k, v, softmax_scale, causal, k2, v2, descales, out_dtype
 
 def attn_fwd(q, k, v, softmax_scale=None, causal=False, k2=None, v2=None,
              q_descale=None, k_descale=None, v_descale=None, out_dtype=None, out=None,
-             return_lse=True, balance=True, lse=None, noalloc=False, streamed=None, _acc=None):
+             return_lse=True, balance=True, lse=None, noalloc=False, streamed=None, q2=None, _acc=None):
     """Non-causal attention forward on logical BHSD tensors -> (out BHSD, lse (B,H,Sq) fp32).
 
     `k2`/`v2` are an optional second key/value segment (the joint text tokens) attended together
-    with `k`/`v`.  For fp8 (torch.float8_e4m3fn) inputs the descales are (B, H) fp32 tensors.
+    with `k`/`v`; `q2` optional further query rows (bf16 / fp16), attended as if they had been
+    concatenated behind those of `q`.  For fp8 (torch.float8_e4m3fn) inputs the descales are (B, H) fp32 tensors.
     `out` / `lse` receive the results when given (new tensors otherwise).
     `balance=False` withholds the scratch buffer with which the library evens out the last round
     of workgroups (results then come from one workgroup per query tile).
@@ -221,19 +233,21 @@ def attn_fwd(q, k, v, softmax_scale=None, causal=False, k2=None, v2=None,
         softmax_scale = float(q.shape[-1]) ** -0.5
     if noalloc and (out is None or (return_lse and lse is None) or _acc is not None):
         raise ValueError("noalloc needs out (and lse) from the caller and is not available for the ring step")
+    if q2 is not None and (noalloc or _acc is not None):
+        raise ValueError("q2 is not available with noalloc or for the ring step")
     if lse is not None:
         return_lse = True
     if streamed is None:
         streamed = bool(TUNING["streamed"])
     acc_sig = None if _acc is None else (_sig(_acc[0]), _sig(_acc[1]), _acc[2], _acc[3])
-    key = (q.dtype, out_dtype, device, _sig(q), _sig(k), _sig(v), _sig(k2), _sig(v2), _sig(out), _sig(lse),
+    key = (q.dtype, out_dtype, device, _sig(q), _sig(k), _sig(v), _sig(k2), _sig(v2), _sig(out), _sig(lse), _sig(q2),
            k.dtype, v.dtype, float(softmax_scale), bool(causal), q_descale is not None, k_descale is not None,
            v_descale is not None, acc_sig, TUNING["rows_per_workgroup"], TUNING["cu_count"], TUNING["balance"], bool(streamed))
     plans = _TLS.__dict__.setdefault("plans", {})
     plan = plans.get(key)
     if plan is None:
         plan = _build_attn_plan(q, k, v, softmax_scale, causal, k2, v2, (q_descale, k_descale, v_descale),
-                                out_dtype, out, lse, _acc, streamed)
+                                out_dtype, out, lse, _acc, streamed, q2)
         if len(plans) >= _PLANS_MAX:
             plans.clear()
         plans[key] = plan
@@ -276,6 +290,9 @@ def attn_fwd(q, k, v, softmax_scale=None, causal=False, k2=None, v2=None,
                 r = plan.ring
                 r.acc_out, r.acc_lse = _acc[0].data_ptr(), _acc[1].data_ptr()
                 rc = L.xdit_attn_fwd_accumulate(ctypes.byref(a), ctypes.byref(r))
+            elif q2 is not None:
+                plan.tail.q2 = q2.data_ptr()
+                rc = L.xdit_attn_fwd_two_queries(ctypes.byref(a), ctypes.byref(plan.tail))
             else:
                 rc = L.xdit_attn_fwd(ctypes.byref(a))
     if entry is not None:
@@ -375,7 +392,7 @@ def lse_merge(acc_out, acc_lse, block_out, block_lse, first=False, final_out=Non
 _QUANT_SCRATCH = {}
 
 
-def _quant_job(a, x, per_tensor, hadamard_block, x2):
+def _quant_job(a, x, per_tensor, hadamard_block, x2, joined):
     """Fills the fields of a QuantArgs that the shapes, strides and options decide."""
     device = x.device
     _check4("x", x, device)
@@ -394,21 +411,24 @@ def _quant_job(a, x, per_tensor, hadamard_block, x2):
         if S2 > 0:
             a.S2 = S2
             a.x2_stride, a.y2_stride = _strides(x2), _lib.Strides(H * S2 * D, S2 * D, D)
+            if joined:
+                a.y_stride = a.y2_stride = _lib.Strides(H * (S + S2) * D, (S + S2) * D, D)
 
 
-def fp8_quant_batch(jobs):
+def fp8_quant_batch(jobs, joined=()):
     """Up to four `fp8_quant` calls (tuples x, per_tensor, scale, hadamard_block, x2) on tensors of one
-    dtype and device in the same launches -> list of (y, descale) or (y, y2, descale).  The outputs
+    dtype and device in the same launches -> list of (y, descale) or (y, y2, descale).  The jobs whose
+    index is in `joined` write x and x2 as the rows of one tensor, x first -> (y, descale).  The outputs
     are new tensors; the argument structs are kept per signature and thread like those of `attn_fwd`."""
     device = jobs[0][0].device
-    key = ("quant",) + tuple((_sig(x), bool(pt), scale is not None, int(had), _sig(x2)) for x, pt, scale, had, x2 in jobs)
+    key = ("quant", joined) + tuple((_sig(x), bool(pt), scale is not None, int(had), _sig(x2)) for x, pt, scale, had, x2 in jobs)
     plans = _TLS.__dict__.setdefault("plans", {})
     arr = plans.get(key)
     n = len(jobs)
     if arr is None:
         arr = (_lib.QuantArgs * n)()
-        for a, (x, pt, scale, had, x2) in zip(arr, jobs):
-            _quant_job(a, x, pt, had, x2)
+        for i, (a, (x, pt, scale, had, x2)) in enumerate(zip(arr, jobs)):
+            _quant_job(a, x, pt, had, x2, i in joined)
             if x.device != device:
                 raise ValueError("the tensors of a batch must be on one device")
         if len(plans) >= _PLANS_MAX:
@@ -422,8 +442,9 @@ def fp8_quant_batch(jobs):
         _QUANT_SCRATCH[(device, stream)] = buf
     scratch = buf.data_ptr()
     keep, out = [], []
-    for a, size, (x, pt, scale, had, x2) in zip(arr, need, jobs):
-        y = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=device)
+    for i, (a, size, (x, pt, scale, had, x2)) in enumerate(zip(arr, need, jobs)):
+        B, H, S, D = x.shape
+        y = torch.empty((B, H, S + x2.shape[2], D) if i in joined else x.shape, dtype=torch.float8_e4m3fn, device=device)
         descale = torch.empty(x.shape[:2], dtype=torch.float32, device=device)
         a.x, a.y, a.descale = x.data_ptr(), y.data_ptr(), descale.data_ptr()
         if scale is not None:
@@ -433,7 +454,10 @@ def fp8_quant_batch(jobs):
         a.stream = stream
         a.scratch, a.scratch_bytes = scratch, size
         scratch += size
-        if x2 is None:
+        if i in joined:
+            a.x2, a.y2 = x2.data_ptr(), a.y + S * D
+            out.append((y, descale))
+        elif x2 is None:
             out.append((y, descale))
         else:
             y2 = torch.empty(x2.shape, dtype=torch.float8_e4m3fn, device=device)

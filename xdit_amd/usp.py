@@ -179,6 +179,12 @@ def USP(query, key, value, dropout_p=0.0, is_causal=False, joint_query=None, joi
         raise NotImplementedError("attn_layer (PipeFusion KV cache) is not supported on the single-device path")
     attention_function = _get_attention_function(backend=backend)
     joint_attn_kwargs = None
+    if joint_strategy and ring_chunks == 1:
+        joined = AB.joint_queries_call(_DECORATED[backend if backend is not None else _DEFAULT_BACKEND][0], query, joint_query,
+                                       joint_strategy, key, value, dropout_p, is_causal, attention_kwargs,
+                                       (joint_key, joint_value, joint_strategy))
+        if joined is not None:
+            return joined[0]
     if joint_strategy:
         query = _concat_joint_tensor(query, joint_query, joint_strategy, dim=2)
         joint_attn_kwargs = {
