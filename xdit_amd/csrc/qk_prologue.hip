@@ -260,9 +260,95 @@ __global__ __launch_bounds__(256) void prologue_token_kernel(const PrologueParam
   }
 }
 
+// The same with one wavefront per token, for 16-bit tensors: a lane keeps its N chunks (lane, lane + 64, ...)
+// as loaded, so all of a token is in flight at once, and the gains and the rotation's row are requested with
+// it instead of behind the reduction, which needs neither LDS nor a barrier.  Four consecutive tokens per
+// workgroup make the stores of a head 1 KiB runs of the BHSD output.
+template <typename T, int N>
+__global__ __launch_bounds__(256) void prologue_token_wave_kernel(const PrologueParams p) {
+  typedef typename Vec8<T>::type vec8;
+  const int64_t tok = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (tok >= (int64_t)p.B * p.S) return;  // whole wavefronts leave together
+  const int lane = threadIdx.x & 63;
+  const int s = (int)(tok % p.S);
+  const int b = (int)(tok / p.S);
+  const int cpr = p.D >> 3;             // a power of two, at most 64
+  const int c = lane & (cpr - 1);       // the chunk's place in its row: the same for all chunks of a lane
+  const int h0 = lane / cpr, hstep = 64 / cpr;
+  const T* x = (const T*)p.x + b * p.xs_b + (int64_t)s * p.xs_s + c * 8;
+  vec8 raw[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    const int h = h0 + k * hstep;
+    raw[k] = *(const vec8*)(x + (int64_t)(h < p.H ? h : p.H - 1) * p.xs_h);
+  }
+  const int sr = s - p.rope_row0;
+  const bool rope = p.rope_mode != 0 && sr >= 0 && sr < p.rope_rows;
+  float cs[8], sn[8];
+  if (rope) {
+    const int64_t off = (int64_t)sr * p.rope_stride + c * 8;
+    load8<float>(p.cos + off, cs);
+    load8<float>(p.sin + off, sn);
+  }
+  const bool gain = p.weight != nullptr;
+  vec8 g[N];
+  if (gain) {
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const int h = h0 + k * hstep;
+      g[k] = *(const vec8*)((const T*)p.weight + (int64_t)(h < p.H ? h : p.H - 1) * p.D + c * 8);
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    if (h0 + k * hstep < p.H) {
+#pragma unroll
+      for (int i = 0; i < 8; i++) ss += (float)raw[k][i] * (float)raw[k][i];
+    }
+  }
+#pragma unroll
+  for (int m = 32; m > 0; m >>= 1) ss += __shfl_xor(ss, m);
+  const float rs = 1.0f / sqrtf(ss * p.inv_n + p.eps);
+  T* y = (T*)p.y + b * p.ys_b + (int64_t)s * p.ys_s + c * 8;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    const int h = h0 + k * hstep;
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      v[i] = (float)(T)((float)raw[k][i] * rs);
+      if (gain) v[i] = (float)(T)(v[i] * (float)g[k][i]);
+    }
+    float partner[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (p.rope_mode == 2) {  // uniform: every lane takes part in the exchange
+#pragma unroll
+      for (int i = 0; i < 8; i++) partner[i] = __shfl_xor(v[i], cpr >> 1);
+    }
+    if (rope) rotate8(v, cs, sn, p.rope_mode, partner, (c & (cpr >> 1)) != 0);
+    if (h < p.H) store8<T>(y + (int64_t)h * p.ys_h, v);
+  }
+}
+
+// The wavefront form at the smallest N that holds a token's chunks.
+template <typename T>
+static void launch_token_wave(const PrologueParams& p, hipStream_t stream) {
+  const dim3 grid((unsigned)(((int64_t)p.B * p.S + 3) / 4)), block(256);
+  const int n = (p.H * (p.D >> 3) + 63) / 64;
+  if (n <= 2) hipLaunchKernelGGL((prologue_token_wave_kernel<T, 2>), grid, block, 0, stream, p);
+  else if (n <= 4) hipLaunchKernelGGL((prologue_token_wave_kernel<T, 4>), grid, block, 0, stream, p);
+  else if (n <= 6) hipLaunchKernelGGL((prologue_token_wave_kernel<T, 6>), grid, block, 0, stream, p);
+  else if (n <= 8) hipLaunchKernelGGL((prologue_token_wave_kernel<T, 8>), grid, block, 0, stream, p);
+  else if (n <= 10) hipLaunchKernelGGL((prologue_token_wave_kernel<T, 10>), grid, block, 0, stream, p);
+  else if (n <= 12) hipLaunchKernelGGL((prologue_token_wave_kernel<T, 12>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((prologue_token_wave_kernel<T, 16>), grid, block, 0, stream, p);
+}
+
 template <typename T>
 static hipError_t run(const PrologueParams& p, hipStream_t stream) {
-  if (p.norm == 2) {
+  if (p.norm == 2 && sizeof(T) == 2) {
+    if constexpr (sizeof(T) == 2) launch_token_wave<T>(p, stream);
+  } else if (p.norm == 2) {
     hipLaunchKernelGGL((prologue_token_kernel<T>), dim3((unsigned)((int64_t)p.B * p.S)), dim3(256), 0, stream, p);
   } else {
     const int64_t tokens = (int64_t)p.B * p.S;  // one wavefront each, four per workgroup
