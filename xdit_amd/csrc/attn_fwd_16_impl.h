@@ -210,14 +210,14 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
     qt = sg.tile - bh * nq_tiles;
     b = bh / H;
     h = bh - b * H;
-    const int Sq = pp->Sq;
+    const int Sq = pp->Sq, Sq1 = pp->Sq1;
     const int qrow = qt * kRowsPerBlock + wave * kRowsPerWave + l32;
     const int qrow_c = qrow < Sq ? qrow : Sq - 1;
     const T* qptr = (const T*)pp->q + b * pp->qs_b + h * pp->qs_h + (int64_t)qrow_c * pp->qs_s + hh * 8;
     // Joint attention's queries come as two tensors and are read where they are: copying them into one first
     // cost 24 us beside 232 us of attention (24 heads of 4096 + 512 rows), 5 beside 13 (3 heads of 1024 + 512).
-    if (!FUSED && qrow_c >= pp->Sq1)
-      qptr = (const T*)pp->q2 + b * pp->q2s_b + h * pp->q2s_h + (int64_t)(qrow_c - pp->Sq1) * pp->q2s_s + hh * 8;
+    if (!FUSED && qrow_c >= Sq1)
+      qptr = (const T*)pp->q2 + b * pp->q2s_b + h * pp->q2s_h + (int64_t)(qrow_c - Sq1) * pp->q2s_s + hh * 8;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ks++) {
       if (!PAD || ks * 16 + hh * 8 < dact) {
@@ -419,8 +419,8 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
         walk.claimed(g, (unsigned)__builtin_amdgcn_readfirstlane((int)ticket));
       }
       more = walk.next(g, nt, next_seg);
-      if (!more && pp->plain_stride != 0) {  // a plain launch of fewer workgroups than tiles: on to the next tile
-        plain_block += pp->plain_stride;
+      if (!more && g.plain_stride != 0) {  // a plain launch of fewer workgroups than tiles: on to the next tile
+        plain_block += g.plain_stride;
         more = plain_block < 8 * g.tiles_per_xcd && walk.start(g, nt, plain_block) && walk.next(g, nt, next_seg);
       }
     }

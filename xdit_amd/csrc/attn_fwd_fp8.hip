@@ -358,8 +358,8 @@ __device__ __forceinline__ void attn_workgroup_fp8(unsigned char* smem) {
         walk.claimed(g, (unsigned)__builtin_amdgcn_readfirstlane((int)ticket));
       }
       more = walk.next(g, nt, next_seg);
-      if (!more && pp->plain_stride != 0) {  // a plain launch of fewer workgroups than tiles: on to the next tile
-        plain_block += pp->plain_stride;
+      if (!more && g.plain_stride != 0) {  // a plain launch of fewer workgroups than tiles: on to the next tile
+        plain_block += g.plain_stride;
         more = plain_block < 8 * g.tiles_per_xcd && walk.start(g, nt, plain_block) && walk.next(g, nt, next_seg);
       }
     }

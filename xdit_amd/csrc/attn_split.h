@@ -29,12 +29,12 @@ __device__ __forceinline__ unsigned draw_ticket(unsigned* counter) {
 
 // The launch geometry the walker reads, gathered from the kernel arguments when needed.
 struct WalkGeom {
-  int total_tiles, tiles_per_xcd, split_full, split_units, split_len, split_pmax, split_fuse0, split_claimers, split_dyn, split_s0, split_order;
+  int total_tiles, tiles_per_xcd, split_full, split_units, split_len, split_pmax, split_fuse0, split_claimers, split_dyn, split_s0, split_order, plain_stride;
 };
 typedef const __attribute__((address_space(4))) AttnParams* ParamsPtr;
 __device__ __forceinline__ WalkGeom walk_geom(ParamsPtr pp) {
   WalkGeom g = {pp->total_tiles, pp->tiles_per_xcd, pp->split_full, pp->split_units, pp->split_len, pp->split_pmax,
-                pp->split_fuse0, pp->split_claimers, pp->split_dyn, pp->split_s0, pp->split_order};
+                pp->split_fuse0, pp->split_claimers, pp->split_dyn, pp->split_s0, pp->split_order, pp->plain_stride};
   return g;
 }
 
@@ -475,14 +475,15 @@ static inline unsigned split_grid(const AttnParams& q) {
   return (unsigned)(q.split_fuse0 <= q.split_full ? q.split_full : q.split_full + q.split_claimers);
 }
 
-// The grid to launch: that of split_grid, or, for a plain launch of more tiles than workgroups fit on
-// the compute units at once, as many workgroups as do fit, each running tile after tile (plain_stride):
-// the next tile's queries and first keys are then on their way while the rows of the current one are
-// stored, and no compute unit waits for a workgroup to be dispatched.  40 heads of 32760 queries on 512
-// keys 412 -> 391 us, 2 x 16 heads of 4096 on 120 keys (head_dim 72) 18.7 -> 18.1, four ring steps of
-// 24 heads of 4608 x 1152 345 -> 339, fp8 5 heads of 75600 7.51 -> 7.43 ms; nothing slower.  The tiles of
-// a workgroup lie a multiple of eight apart in the dispatch order, so they stay on its XCD.
-// `residency` caches the occupancy of the kernel (per device, the kernel's own).
+// The grid to launch: that of split_grid, or, for a plain launch of more tiles than compute units whose
+// workgroups fill a compute unit alone, one workgroup per compute unit that runs tile after tile
+// (plain_stride): the next tile's queries and first keys are then on their way while the rows of the current
+// one are stored, and no compute unit waits for a workgroup to be dispatched.  40 heads of 32760 queries on
+// 512 keys 412 -> 391 us, four ring steps of 24 heads of 4608 x 1152 345 -> 339.  Workgroups that share a
+// compute unit hide each other's start already, and dealing their tiles out beforehand costs more than it
+// gives (128 rows: 24 heads of 14933 on 512 keys 111.3 -> 116.2 us, head_dim 64, 24 heads of 18882 on 77 keys
+// 33.5 -> 34.6).  The tiles of a workgroup lie a multiple of eight apart in the dispatch order, so they stay
+// on its XCD.  `residency` caches the occupancy of the kernel (per device, the kernel's own).
 static inline unsigned resident_grid(AttnParams& q, const void* kernel, int threads, int lds, std::atomic<int>& residency) {
   const unsigned grid = split_grid(q);
   q.plain_stride = 0;
@@ -492,7 +493,7 @@ static inline unsigned resident_grid(AttnParams& q, const void* kernel, int thre
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, lds) != hipSuccess || n <= 0) n = -1;
     residency.store(n, std::memory_order_relaxed);
   }
-  const unsigned slots = n <= 0 ? 0u : (unsigned)(resident_cus(q.cu_count) * n) & ~7u;
+  const unsigned slots = n != 1 ? 0u : (unsigned)resident_cus(q.cu_count) & ~7u;
   if (slots == 0 || grid <= slots) return grid;
   q.plain_stride = (int)slots;
   return slots;

@@ -48,6 +48,7 @@ struct AttnParams {
   int64_t ds_b, ds_h;
   int B, H;
   int Sq, Sk, Sk2;
+  int Sq1;            // query rows in q; the others are in q2 (below)
   int nq_tiles;       // ceil(Sq / rows per workgroup)
   int total_tiles;    // B * H * nq_tiles
   int tiles_per_xcd;  // ceil(total_tiles / 8)
@@ -68,14 +69,14 @@ struct AttnParams {
   int split_s0;       // KV iterations every member of a tile's group owns before it draws from the counter
   int streamed_ok;    // the caller opted in to streamed sharing (results then reproducible to rounding only)
   int split_order;    // claimers process their range BEFORE their whole query tile (see WorkgroupWalk)
-  int split_fold;     // the parts of a shared tile are folded inside the attention kernel (fold duties, attn_walk.h)
   int plain_stride;   // plain launch of fewer workgroups than query tiles: workgroup w runs tiles w, w + plain_stride, ...
                       // of the dispatch order (0: one tile per workgroup)
+  int split_fold;     // the parts of a shared tile are folded inside the attention kernel (fold duties, attn_walk.h)
   int split_policy;   // 1: plain launch; 2: balance whenever the plan shortens the critical path by kMinSaving iterations
-  // the last rows of the queries may lie in a tensor of their own: rows Sq1 .. Sq-1 are rows 0 .. of q2 (Sq1 == Sq: none do)
+  // the last rows of the queries may lie in a tensor of their own: rows Sq1 .. Sq-1 are rows 0 .. of q2
+  // (Sq1 == Sq: none do)
   const void* q2;
   int64_t q2s_b, q2s_h, q2s_s;
-  int Sq1;
   // ring step (optional): the result is folded into an fp32 accumulator in the epilogue
   float* acc_out;     // (B,H,Sq,D) fp32 running output, nullptr: plain forward
   float* acc_lse;     // (B,H,Sq) fp32 running log-sum-exp
