@@ -1585,3 +1585,56 @@ def test_two_queries_entry_refuses_what_it_cannot_read(gpu):
             ops.attn_fwd(q, k, k, q2=bad)
     with pytest.raises((ValueError, NotImplementedError)):
         ops.attn_fwd(q.float(), k.float(), k.float(), q2=q.float())
+
+
+def _fp32_case(gpu, D, Sq, Sk, Sk2, seed=0):
+    g = torch.Generator().manual_seed(seed + D + Sk)
+    mk = lambda s: torch.randn(1, 2, s, D, generator=g)
+    q, k, v, k2, v2 = mk(Sq) * 1.5, mk(Sk) * 1.5, mk(Sk), mk(Sk2) * 1.5, mk(Sk2)
+    kw = dict(k2=k2.to(gpu), v2=v2.to(gpu)) if Sk2 else {}
+    kk, vv = torch.cat([k, k2], 2).double(), torch.cat([v, v2], 2).double()
+    s = q.double() @ kk.transpose(2, 3) * D ** -0.5
+    return q, k, v, kw, torch.softmax(s, -1) @ vv, torch.logsumexp(s, -1)
+
+
+@pytest.mark.parametrize("cus", [0, 1])
+@pytest.mark.parametrize("D,Sq,Sk,Sk2", [(8, 33, 65, 0), (40, 129, 64, 1), (64, 64, 31, 33), (72, 65, 257, 0), (96, 200, 96, 40), (104, 31, 1, 0), (128, 130, 300, 70)])
+def test_fp32_split_products_are_no_less_exact_than_fp32_ones(gpu, monkeypatch, cus, D, Sq, Sk, Sk2):
+    """fp32 attention on the bf16 matrix cores (three-way split operands) and, with queries scaled out of
+    the split's range by a power of two that the softmax scale takes back, on the fp32 ones, against
+    float64: the split's error is no larger (the factor covers the scatter of a small sample), at the
+    edges of the tiles, both workgroup shapes (one or 256 compute units) and a second KV segment."""
+    q, k, v, kw, ro, rl = _fp32_case(gpu, D, Sq, Sk, Sk2)
+    monkeypatch.setitem(ops.TUNING, "cu_count", cus)
+    f = 2.0 ** -96
+    split = ops.attn_fwd(q.to(gpu), k.to(gpu), v.to(gpu), softmax_scale=D ** -0.5, **kw)
+    exact = ops.attn_fwd((q * f).to(gpu), k.to(gpu), v.to(gpu), softmax_scale=D ** -0.5 / f, **kw)
+    for a, b, r in zip(split, exact, (ro, rl)):
+        ea, eb = ((x.cpu().double() - r).norm().item() / r.norm().item() for x in (a, b))
+        # both forms round at 2^-24; at one key the result is exact in either
+        assert ea <= max(1.25 * eb, 2.0 ** -24) and (a.cpu().double() - r).abs().max().item() <= 2e-5
+
+
+@pytest.mark.parametrize("cus", [0, 1])
+@pytest.mark.parametrize("what", ["inf value", "-inf value", "huge key", "nan key", "largest values", "tiny values"])
+def test_fp32_out_of_the_splits_range(gpu, monkeypatch, cus, what):
+    """Values the three-way split has no room for: an infinite value reaches its column only, a key whose
+    logits are -inf or hugely negative drops out, values at the ends of fp32's range keep their precision."""
+    q, k, v, _, _, _ = _fp32_case(gpu, 72, 130, 100, 0)
+    q = q.abs()
+    if what.endswith("inf value"): v[0, 1, 77, 5] = float(what.split()[0])
+    elif what == "huge key": k[0, 1, 40] = -1e37
+    elif what == "nan key": k[0, 1, 40, 3] = float("nan")
+    elif what == "largest values":  # logits near 0, so the unnormalised sum over 100 keys stays below 2^127
+        q, v = q * 2.0 ** -10, v * (2.0 ** 120 / v.abs().max())
+    else: v *= 2.0 ** -110
+    monkeypatch.setitem(ops.TUNING, "cu_count", cus)
+    o, l = ops.attn_fwd(q.to(gpu), k.to(gpu), v.to(gpu))
+    s = q.double() @ k.double().transpose(2, 3) * 72 ** -0.5
+    ro, rl = torch.softmax(s, -1) @ v.double(), torch.logsumexp(s, -1)
+    if what == "nan key":
+        assert o[0, 1].isnan().all() and o[0, 0].isfinite().all()
+        return
+    o, bad = o.cpu().double(), ~ro.isfinite()
+    assert torch.equal(o[bad], ro[bad]) and o[~bad].isfinite().all()
+    assert ((o - ro)[~bad].norm() / ro[~bad].norm()).item() <= 2e-6 and (l.cpu().double() - rl).abs().max().item() <= 2e-5
