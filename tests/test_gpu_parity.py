@@ -1638,3 +1638,18 @@ def test_fp32_out_of_the_splits_range(gpu, monkeypatch, cus, what):
     o, bad = o.cpu().double(), ~ro.isfinite()
     assert torch.equal(o[bad], ro[bad]) and o[~bad].isfinite().all()
     assert ((o - ro)[~bad].norm() / ro[~bad].norm()).item() <= 2e-6 and (l.cpu().double() - rl).abs().max().item() <= 2e-5
+
+
+@pytest.mark.parametrize("cus", [0, 1])
+@pytest.mark.parametrize("D", [64, 72, 128])
+def test_fp32_error_over_many_keys_stays_at_one_rounding_per_tile(gpu, monkeypatch, cus, D):
+    """16000 keys in 500 tiles of 32: every addition of a tile's products to O^T rounds at 2^-24 of a sum that
+    grows like the square root of its terms, so independent roundings add up to at most 2^-24 sqrt(500)
+    (a rounding per product instead of per tile, 1.5e-6 to 1.7e-6 measured, is over that)."""
+    q, k, v, _, _, _ = _fp32_case(gpu, D, 128, 16000, 0)
+    monkeypatch.setitem(ops.TUNING, "cu_count", cus)
+    o, l = ops.attn_fwd(q.to(gpu) / 1.5, k.to(gpu) / 1.5, v.to(gpu), softmax_scale=D ** -0.5)
+    s = (q / 1.5).double() @ (k / 1.5).double().transpose(2, 3) * D ** -0.5
+    ro, rl = torch.softmax(s, -1) @ v.double(), torch.logsumexp(s, -1)
+    assert (o.cpu().double() - ro).norm() / ro.norm() <= 2.0 ** -24 * 500 ** 0.5
+    assert (l.cpu().double() - rl).abs().max() <= 1e-5

@@ -5,10 +5,12 @@
 // Two loops: split_loop runs the products on the bf16 matrix cores with operands split into three bf16
 // values, and the loop in the kernel itself on the fp32 ones (v_mfma_f32_32x32x2_f32) for the values that the
 // split has no room for.  The fp32 instruction runs at a sixteenth of the bf16 rate; six split products cost
-// 3/8 of it.  2 x 16 heads of 4096 rows at head_dim 72: 1466 -> 900 us, 24 heads of 4608 at 128: 2618 -> 1618,
-// 16 heads of 1024 at 72: 67 -> 52 (same box); relative error against float64 1.28e-6 -> 1.06e-6,
-// 1.38e-6 -> 1.12e-6, 5.2e-7 -> 3.9e-7.  Bound now by the VALU work of splitting and softmax beside the
-// MFMAs (busy 33 % with one wavefront per SIMD, 49 % with two).
+// 3/8 of it.  2 x 16 heads of 4096 rows at head_dim 72: 1465 -> 964 us, 24 heads of 4608 at 128: 2625 -> 1646,
+// 16 heads of 1024 at 72: 67 -> 53, one head of 39500 at 64: 5753 -> 3029 (same box); relative error against
+// float64 1.26e-6 -> 2.8e-7, 1.37e-6 -> 3.1e-7, 5.2e-7 -> 1.8e-7, 3.9e-6 -> 7.9e-7, because a tile's products are
+// summed by themselves before they are added to O^T (added one by one: 1.06e-6, 1.10e-6, 3.9e-7, 3.3e-6, at 930,
+// 1651, 53, 3010 us).  Bound by the VALU work of splitting and softmax beside the MFMAs (busy 33 % with one
+// wavefront per SIMD, 49 % with two, before the tile sums).
 // In the fp32 loop, with a contraction depth of 2 per instruction every operand is ONE float per lane, so V^T
 // is a plain LDS read (lanes along head_dim) and needs no transposing load.
 //
@@ -89,8 +91,8 @@ __device__ __forceinline__ float max_abs(float m, float a, float b) { return fma
 
 // The KV loop on the bf16 matrix cores.  Every fp32 operand x is split into x0 + x1 + x2 (split2) and a
 // product is x0 y0 + (x0 y1 + x1 y0) + (x0 y2 + x1 y1 + x2 y0): what is left out is below 2^-25 of the
-// product, under the rounding of an fp32 product, and the accumulation is in fp32 with a rounding per 16
-// products instead of per 2.  Six bf16 instructions of 32 cycles do the work of eight fp32 ones of 64.
+// product, under the rounding of an fp32 product, and the accumulation is in fp32: one rounding per 32 keys at
+// the size of O^T instead of one per 2.  Six bf16 instructions of 32 cycles do the work of eight fp32 ones of 64.
 // K and V tiles are split once per workgroup on their way into LDS (row-major planes; V^T is read
 // transposed, as in the 16-bit kernel), Q once, P per tile in registers.
 // The split has no room at the ends of fp32's range, and 0 x inf turns up where the plain product has
@@ -271,42 +273,62 @@ __device__ __forceinline__ bool split_loop(const AttnParams& p, unsigned char* s
     // P^T as B operands: plane n, key step j (16 keys): registers 8j .. 8j+7 of S^T.  Results below 2^-126 are zero:
     // the row's sum is at least 2^-8.
     u32x4 pf[3][2];
+    float l_tile = 0.f;  // summed by itself: one rounding at the size of the row's sum per tile
     auto probabilities = [&](int j, int e) {
       const float p0 = fast_exp2(__builtin_fmaf(sacc[8 * j + 2 * e], c, -mc)), p1 = fast_exp2(__builtin_fmaf(sacc[8 * j + 2 * e + 1], c, -mc));
-      l_part += p0 + p1;
+      l_tile += p0 + p1;
       unsigned a, m, l;
       split2(p0, p1, a, m, l);
       pf[0][j][e] = a; pf[1][j][e] = m; pf[2][j][e] = l;
     };
 #pragma unroll
     for (int e = 0; e < 4; e++) probabilities(0, e);
-    // O^T += V^T P^T, small products first; the second key step's probabilities between the first one's MFMAs
+    // O^T += V^T P^T.  A tile's products are summed by themselves, small ones first, and added once: O^T grows
+    // with the number of keys and every addition to it rounds at its size.  The second key step's probabilities
+    // stand between the first MFMAs, the additions of one block of columns between the next one's.
     {
       bf16x8 vf[2][3];
       auto read_v = [&](int g, int n) {
-        const XDIT_LDS unsigned char* at = base + vfrag + n * G::SV_PLANE + 16 * (g / DB) * G::SV_PITCH + 64 * (g % DB);
+        const XDIT_LDS unsigned char* at = base + vfrag + n * G::SV_PLANE + 16 * (g % 2) * G::SV_PITCH + 64 * (g / 2);
         const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((XDIT_LDS s16x4*)at);
         const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((XDIT_LDS s16x4*)(at + 8 * G::SV_PITCH));
         vf[g % 2][n] = __builtin_bit_cast(bf16x8, (s16x8)__builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
       };
 #pragma unroll
       for (int n = 0; n < 3; n++) read_v(0, n);
+      // One sum where 256 registers do not hold two (16 heads of 4000 at head_dim 88, 96: 540, 554 us with two, 521, 514
+      // with one), two otherwise (37000 keys at head_dim 72: 3754 us, 3978 with one).
+      constexpr int NS = KS == 1 && (D8 == 11 || D8 == 12) ? 1 : 2;
+      f32x16 sum[NS];
       static_for<12 * DB>([&](auto I) {
-        constexpr int i = I, g = i / 6, op = i % 6, j = g / DB, db = g % DB;
+        constexpr int i = I, g = i / 6, op = i % 6, db = g / 2, j = g % 2;
         if constexpr (op == 0 && g + 1 < 2 * DB) {
 #pragma unroll
           for (int n = 0; n < 3; n++) read_v(g + 1, n);
         }
+        if constexpr (op == 0 && j == 0) {
+#pragma unroll
+          for (int e = 0; e < 16; e++) sum[db % NS][e] = 0.f;
+        }
         constexpr int vn = op == 0 ? 2 : (op == 2 || op == 3 ? 1 : 0);   // lo hi, hi lo, mid mid, mid hi, hi mid, hi hi
         constexpr int pn = op == 1 ? 2 : (op == 2 || op == 4 ? 1 : 0);
-        oacc[db] = Mfma16<__bf16>::mma(vf[g % 2][vn], __builtin_bit_cast(bf16x8, pf[pn][j]), oacc[db]);
-        if constexpr (j == 0) {
-          constexpr int first = i * 4 / (6 * DB), past = (i + 1) * 4 / (6 * DB);
+        sum[db % NS] = Mfma16<__bf16>::mma(vf[g % 2][vn], __builtin_bit_cast(bf16x8, pf[pn][j]), sum[db % NS]);
+        if constexpr (g == 0) {
+          constexpr int first = i * 4 / 6, past = (i + 1) * 4 / 6;
           static_for<past - first>([&](auto J) { probabilities(1, first + J); });
           __builtin_amdgcn_sched_barrier(0);
+        } else if constexpr (NS == 2 && db > 0 && j == 0 && op >= 2) {
+#pragma unroll
+          for (int e = 4 * (op - 2); e < 4 * (op - 1); e++) oacc[db - 1][e] += sum[(db - 1) % NS][e];
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (j == 1 && op == 5 && (NS == 1 || db == DB - 1)) {
+#pragma unroll
+          for (int e = 0; e < 16; e++) oacc[db][e] += sum[db % NS][e];
         }
       });
     }
+    l_part += l_tile;
   }
 
   // did the split have room?  Every tensor's largest magnitude in [2^-90, 2^120) (or zero throughout), and that
