@@ -1482,6 +1482,33 @@ def test_claimed_ranges_in_a_graph_and_on_two_streams(gpu, force_rows):
         assert torch.equal(b[0], want2[0]) and torch.equal(b[1], want2[1])
 
 
+def test_captured_quantiser_call_after_a_larger_call_on_its_stream(gpu):
+    """A quantiser call captured in a HIP graph, then a batch on the same stream that needs more scratch and
+    new tensors that would take freed memory: the replays leave those alone and give the eager bits."""
+    g = torch.Generator().manual_seed(5)
+    x, other = (torch.randn(2, 3, s, 128, generator=g).bfloat16().to(gpu) for s in (900, 700))
+    side = torch.cuda.Stream(gpu)
+    side.wait_stream(torch.cuda.current_stream(gpu))
+    with torch.cuda.stream(side):
+        ops.fp8_quant(x, per_tensor=True)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        y, d = ops.fp8_quant(x, per_tensor=True)
+    for step in range(3):
+        with torch.cuda.stream(side):
+            ops.fp8_quant_batch([(other, True, None, 0, None)] * (2 + step % 2))
+            fill = [torch.full((4096,), 7.0, device=gpu) for _ in range(8)]
+        x.copy_(torch.randn(x.shape, generator=g).bfloat16() * (step + 1))
+        torch.cuda.synchronize()
+        want = ops.fp8_quant(x, per_tensor=True)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.uint8), want[0].view(torch.uint8)) and torch.equal(d, want[1])
+        assert all((f == 7.0).all() for f in fill)
+
+
 @pytest.mark.parametrize("S,Sq,D,S2,dtype", [(1, 3, 128, 0, torch.bfloat16), (129, 64, 64, 5, torch.float16), (500, 700, 72, 33, torch.bfloat16),
                                              (37, 4, 256, 200, torch.float32)])
 @pytest.mark.parametrize("per_tensor", [False, True])

@@ -1,6 +1,10 @@
 """Host-side logic of the reference-shaped call surfaces, checked on the CPU (no kernels run):
 argument domains, the joint-tensor step rule, ring ordering, registry behaviour, and that
 nothing falls back to a CPU implementation."""
+import contextlib
+import gc
+import weakref
+
 import pytest
 import torch
 
@@ -218,3 +222,34 @@ def test_bench_refuses_more_than_one_gpu_and_lists_the_model_shapes():
         assert ops.fused_ring_step_supported(torch.empty(1, 1, 1, D, dtype=torch.bfloat16))
 
 
+
+
+def test_outgrown_quantiser_scratch_stays_allocated(monkeypatch):
+    """A captured graph keeps the address of the scratch its quantiser call was given: a later call on the
+    stream that needs a larger one must not free it (device calls stubbed, tensors on the CPU)."""
+    seen = []
+
+    class Lib:
+        def xdit_fp8_quant_batch(self, arr, n):
+            seen.append([(arr[i].scratch, arr[i].scratch_bytes) for i in range(n)])
+            return 0
+
+    monkeypatch.setattr(ops, "_check4", lambda *a: None)
+    monkeypatch.setattr(ops, "_stream", lambda device: 7)
+    monkeypatch.setattr(ops, "_on_device", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(ops._lib, "lib", Lib)
+    monkeypatch.setattr(ops, "_QUANT_SCRATCH", {})
+    x = torch.zeros(1, 2, 8, 64)
+    job = (x, True, None, 0, None)
+    ops.fp8_quant(x, per_tensor=True)
+    (old,) = ops._QUANT_SCRATCH.values()
+    assert seen[0][0][0] == old.data_ptr()
+    alive = weakref.ref(old)
+    del old
+    ops.fp8_quant_batch([job] * 4)                                     # four jobs: more scratch
+    ops.fp8_quant(torch.zeros(1, 9000, 8, 64))                         # a slot per (batch, head): more again
+    gc.collect()
+    assert alive() is not None
+    for call in seen:                                                  # the jobs of a call do not share scratch
+        spans = sorted(call)
+        assert all(a + n <= b for (a, n), (b, _) in zip(spans, spans[1:]))

@@ -438,6 +438,8 @@ def fp8_quant_batch(jobs, joined=()):
     need = [4 * max(4096, a.B * a.H) for a in arr]
     buf = _QUANT_SCRATCH.get((device, stream))
     if buf is None or buf.numel() < sum(need):
+        if buf is not None:
+            _RETIRED.append(buf)   # a graph captured on this stream may hold its address
         buf = torch.empty(sum(need), dtype=torch.uint8, device=device)
         _QUANT_SCRATCH[(device, stream)] = buf
     scratch = buf.data_ptr()
