@@ -1535,6 +1535,31 @@ def test_fp8_quant_batch_equals_single_calls(gpu, S, Sq, D, S2, dtype, per_tenso
         assert torch.equal(y.view(torch.uint8), quotient.to(torch.float8_e4m3fn).view(torch.uint8))
 
 
+@pytest.mark.parametrize("dtypes", [(torch.float32, torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32, torch.float32),
+                                    (torch.float16, torch.bfloat16, torch.float32)])
+@pytest.mark.parametrize("joint", [None, "front", "rear"])
+def test_fp8_adapter_takes_a_dtype_per_tensor(gpu, dtypes, joint):
+    """q, k and v of different dtypes (an fp32 norm over q and k, a 16-bit v): the fp8 adapter gives what
+    quantising each tensor by itself gives, with joint tensors through USP as well."""
+    B, H, S, Sj, D = 1, 2, 200, 33, 64
+    g = torch.Generator().manual_seed(3)
+    mk = lambda s, dt: torch.randn(B, H, s, D, generator=g).to(dt).to(gpu)
+    q, k, v = (mk(S, dt) for dt in dtypes)
+    jq, jk, jv = (mk(Sj, dt) for dt in dtypes)
+    q8, qd = AB.per_tensor_quant(q if joint is None else torch.cat([jq, q] if joint == "front" else [q, jq], 2), hadamard_block=D)
+    if joint is None:
+        (k8, kd), (v8, vd), k2, v2 = AB.per_tensor_quant(k, hadamard_block=D), AB.per_tensor_quant(v), None, None
+    else:   # the joint keys are a KV segment of their own
+        (k8, k2, kd), (v8, v2, vd) = AB.per_tensor_quant(k, hadamard_block=D, x2=jk), AB.per_tensor_quant(v, x2=jv)
+        if joint == "front":
+            k8, v8, k2, v2 = k2, v2, k8, v8
+    out_dtype = dtypes[0] if dtypes[0] != torch.float32 else torch.bfloat16
+    want, _ = ops.attn_fwd(q8, k8, v8, k2=k2, v2=v2, q_descale=qd, k_descale=kd, v_descale=vd, out_dtype=out_dtype)
+    kw = {} if joint is None else dict(joint_query=jq, joint_key=jk, joint_value=jv, joint_strategy=joint)
+    got = usp.USP(q, k, v, backend=AB.AttentionBackendType.MI355_FP8, attention_kwargs={"hadamard_block": D}, **kw)
+    assert got.dtype == out_dtype and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("scale", [1.0, 0.037, 3e-5, 1.0e-24, 1.0e24])
 def test_fp8_quant_static_scale_of_every_bf16_value(gpu, scale):
     """Every bf16 value but the NaNs under a static scale: the bytes of the true division, a negative

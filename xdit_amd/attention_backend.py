@@ -207,7 +207,7 @@ def _fp8_attn(query, query_tail, key, value, dropout_p, is_causal, attention_kwa
         else:
             k8, k2, kd = per_tensor_quant(key, scale=static, hadamard_block=had, x2=jk)
             v8, v2, vd = per_tensor_quant(value, scale=static, x2=jv)
-    else:  # the three tensors in the same launches
+    else:  # the three tensors in the same launches (where they share a dtype)
         scale_in = None if static is None else torch.as_tensor(static, dtype=torch.float32, device=query.device).reshape(1)
         (q8, qd), kq, vq = ops.fp8_quant_batch([(query, True, scale_in, had, query_tail), (key, True, scale_in, had, jk),
                                                 (value, True, scale_in, 0, jv)], joined=() if query_tail is None else (0,))

@@ -417,9 +417,18 @@ def _quant_job(a, x, per_tensor, hadamard_block, x2, joined):
 
 def fp8_quant_batch(jobs, joined=()):
     """Up to four `fp8_quant` calls (tuples x, per_tensor, scale, hadamard_block, x2) on tensors of one
-    dtype and device in the same launches -> list of (y, descale) or (y, y2, descale).  The jobs whose
-    index is in `joined` write x and x2 as the rows of one tensor, x first -> (y, descale).  The outputs
-    are new tensors; the argument structs are kept per signature and thread like those of `attn_fwd`."""
+    device -> list of (y, descale) or (y, y2, descale); those of one dtype go in the same launches.  The
+    jobs whose index is in `joined` write x and x2 as the rows of one tensor, x first -> (y, descale).  The
+    outputs are new tensors; the argument structs are kept per signature and thread like those of `attn_fwd`."""
+    dtypes = {job[0].dtype for job in jobs}
+    if len(dtypes) > 1:   # q and k out of an fp32 norm with a 16-bit v: a launch pair per dtype
+        out = [None] * len(jobs)
+        for dtype in dtypes:
+            idx = [i for i, job in enumerate(jobs) if job[0].dtype == dtype]
+            part = fp8_quant_batch([jobs[i] for i in idx], joined=tuple(n for n, i in enumerate(idx) if i in joined))
+            for i, result in zip(idx, part):
+                out[i] = result
+        return out
     device = jobs[0][0].device
     key = ("quant", joined) + tuple((_sig(x), bool(pt), scale is not None, int(had), _sig(x2)) for x, pt, scale, had, x2 in jobs)
     plans = _TLS.__dict__.setdefault("plans", {})
@@ -428,9 +437,9 @@ def fp8_quant_batch(jobs, joined=()):
     if arr is None:
         arr = (_lib.QuantArgs * n)()
         for i, (a, (x, pt, scale, had, x2)) in enumerate(zip(arr, jobs)):
-            _quant_job(a, x, pt, had, x2, i in joined)
             if x.device != device:
                 raise ValueError("the tensors of a batch must be on one device")
+            _quant_job(a, x, pt, had, x2, i in joined)
         if len(plans) >= _PLANS_MAX:
             plans.clear()
         plans[key] = arr
