@@ -1694,6 +1694,31 @@ def test_fp32_out_of_the_splits_range(gpu, monkeypatch, cus, what):
 
 @pytest.mark.parametrize("cus", [0, 1])
 @pytest.mark.parametrize("D", [64, 72, 128])
+@pytest.mark.parametrize("what", ["values", "queries", "keys"])
+def test_fp32_small_elements_beside_large_ones_keep_their_bits(gpu, monkeypatch, cus, D, what):
+    """Elements whose low pieces a bf16 value cannot hold (about 2^-120), in a tensor whose largest magnitude is of an
+    ordinary size: a column of small values beside columns of ones; small queries (keys) that decide the logits
+    because the large column meets zeros in the other tensor.  Bound: the fp32 loop, which the latter go through,
+    rounds O^T at 2^-24 with every key, independently for 300 keys, and as much again for the logits' own sums;
+    with pieces lost to underflow the error is 1e-5 and more."""
+    q, k, v, _, _, _ = _fp32_case(gpu, D, 130, 300, 0)
+    if what == "values":
+        v[..., D - 3] *= 2.0 ** -121
+    else:
+        small, big = (q, k) if what == "queries" else (k, q)
+        small *= 2.0 ** -118
+        big *= 2.0 ** 116
+        small[..., 5], big[..., 5] = 2.0 ** -80, 0.0
+    monkeypatch.setitem(ops.TUNING, "cu_count", cus)
+    o, l = ops.attn_fwd(q.to(gpu), k.to(gpu), v.to(gpu))
+    s = q.double() @ k.double().transpose(2, 3) * D ** -0.5
+    ro, rl = torch.softmax(s, -1) @ v.double(), torch.logsumexp(s, -1)
+    err = (o.cpu().double() - ro).norm(dim=2) / ro.norm(dim=2)   # per column
+    assert err.max().item() <= 2 * 300 ** 0.5 * 2.0 ** -24 and (l.cpu().double() - rl).abs().max().item() <= 2e-5
+
+
+@pytest.mark.parametrize("cus", [0, 1])
+@pytest.mark.parametrize("D", [64, 72, 128])
 def test_fp32_error_over_many_keys_stays_at_one_rounding_per_tile(gpu, monkeypatch, cus, D):
     """16000 keys in 500 tiles of 32: every addition of a tile's products to O^T rounds at 2^-24 of a sum that
     grows like the square root of its terms, so independent roundings add up to at most 2^-24 sqrt(500)

@@ -87,17 +87,28 @@ __device__ __forceinline__ const unsigned char* uniform(const unsigned char* x) 
   const uint64_t v = (uint64_t)x;
   return (const unsigned char*)(((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((int)v));
 }
+constexpr float kValueScale = 0x1p24f;  // of the V planes of the split loop
+constexpr float kValueMost = 0x1p80f;   // of those, so that the sums of 2^31 of them times probabilities of up to 2^8 stay finite
+constexpr float kDotMost = 0x1p120f;
 __device__ __forceinline__ float max_abs(float m, float a, float b) { return fmaxf(fmaxf(m, fabsf(a)), fabsf(b)); }
 
-// The KV loop on the bf16 matrix cores.  Every fp32 operand x is split into x0 + x1 + x2 (split2) and a
-// product is x0 y0 + (x0 y1 + x1 y0) + (x0 y2 + x1 y1 + x2 y0): what is left out is below 2^-25 of the
-// product, under the rounding of an fp32 product, and the accumulation is in fp32: one rounding per 32 keys at
-// the size of O^T instead of one per 2.  Six bf16 instructions of 32 cycles do the work of eight fp32 ones of 64.
+// The KV loop on the bf16 matrix cores.  Every fp32 operand x is split into x0 + x1 + x2 (split2; |x1| is at
+// most 2^-8 of x, |x2| 2^-17) and a product is x0 y0 + (x0 y1 + x1 y0) + (x0 y2 + x1 y1 + x2 y0): what is left
+// out, x1 y2 + x2 y1 and less, is at most 2^-24 of the product (2^-24.04 seen over random operands), which is the
+// rounding of an fp32 product, and the accumulation is in fp32: one rounding per 32 keys at the size of O^T
+// instead of one per 2.  Six bf16 instructions of 32 cycles do the work of eight fp32 ones of 64.
 // K and V tiles are split once per workgroup on their way into LDS (row-major planes; V^T is read
 // transposed, as in the 16-bit kernel), Q once, P per tile in registers.
 // The split has no room at the ends of fp32's range, and 0 x inf turns up where the plain product has
 // none: false (results meaningless) if the largest magnitudes seen do not leave it that room; the caller
 // then runs the fp32 loop.  NaN goes through as in the plain products.
+// The pieces of an element below 2^-110 reach below bf16's smallest subnormal, where up to 2^-134 of it is lost.
+//   V is multiplied by 2^24 on its way into the planes (and O^T by 2^-24 at the end), which leaves nothing of
+//   what fp32 holds below that, whatever the other columns hold.
+//   Q and K: the loop is used only where that puts no logit off by 2^-30, with a margin of 2^9 (which
+//   covers an instruction that takes subnormals as zeros).
+//   P: a probability below 2^-110 is off by up to 2^-134, and one below 2^-126 is zero, beside a row's sum
+//   of at least 2^-8.
 template <int D8, int KS>
 __device__ __forceinline__ bool split_loop(const AttnParams& p, unsigned char* smem, int b, int h, int qrow_c, int rg, int ksl,
                                            float c, f32x16 (&oacc)[Geom<D8, KS>::DB], float& m_used, float& l_part) {
@@ -110,6 +121,7 @@ __device__ __forceinline__ bool split_loop(const AttnParams& p, unsigned char* s
   typedef __attribute__((ext_vector_type(8))) short s16x8;
 
   float mq = 0.f, mk = 0.f, mv = 0.f;  // largest magnitudes seen by this thread
+  const float qk_limit = fminf(0x1p95f / (fabsf(c) * (float)D) - 4.f, kDotMost);   // of |q| + |k|
   bf16x8 qf[3][KST];
   const float* qptr = (const float*)p.q + b * p.qs_b + h * p.qs_h + (int64_t)qrow_c * p.qs_s + 8 * hh;
 #pragma unroll
@@ -171,14 +183,15 @@ __device__ __forceinline__ bool split_loop(const AttnParams& p, unsigned char* s
   auto store_piece = [&](auto I, int buf) {
     constexpr int i = I, n = i / 4;
     constexpr bool is_v = (i / 2) % 2 != 0;
+    constexpr int e = 2 * (i % 2);
     const f32x4 x = is_v ? vr[n] : kr[n];
+    const float xa = is_v ? x[e] * kValueScale : x[e], xb = is_v ? x[e + 1] * kValueScale : x[e + 1];
+    if (is_v) mv = max_abs(mv, xa, xb); else mk = max_abs(mk, xa, xb);
     if constexpr (i % 2 == 0) {
-      split2(x[0], x[1], ph, pm, pl);
-      if (is_v) mv = max_abs(mv, x[0], x[1]); else mk = max_abs(mk, x[0], x[1]);
+      split2(xa, xb, ph, pm, pl);
     } else {
       unsigned h1, m1, l1;
-      split2(x[2], x[3], h1, m1, l1);
-      if (is_v) mv = max_abs(mv, x[2], x[3]); else mk = max_abs(mk, x[2], x[3]);
+      split2(xa, xb, h1, m1, l1);
       const int cc = n + 1 < CPT ? c0 + TPR * n : chunk(n);
       const unsigned at = buf * G::SBUF_BYTES + (is_v ? 3 * G::SK_PLANE + row * G::SV_PITCH : row * G::SK_PITCH) + 8 * cc;
       constexpr int plane = is_v ? G::SV_PLANE : G::SK_PLANE;
@@ -331,8 +344,8 @@ __device__ __forceinline__ bool split_loop(const AttnParams& p, unsigned char* s
     l_part += l_tile;
   }
 
-  // did the split have room?  Every tensor's largest magnitude in [2^-90, 2^120) (or zero throughout), and that
-  // of the dot products below 2^120
+  // did the split have room?  The largest magnitudes of Q and K in [2^-90, 2^120) (or zero throughout) and within
+  // the limit on what their small elements lose, that of V as split below 2^80 and the dot products below 2^120
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     mq = fmaxf(mq, __shfl_xor(mq, off));
@@ -344,8 +357,12 @@ __device__ __forceinline__ bool split_loop(const AttnParams& p, unsigned char* s
   __syncthreads();  // also: the tile buffers are no longer read
 #pragma unroll
   for (int w = 0; w < 4; w++) { mq = fmaxf(mq, seen[w][0]); mk = fmaxf(mk, seen[w][1]); mv = fmaxf(mv, seen[w][2]); }
-  auto room = [](float m) { return m == 0.f || (m >= 0x1p-90f && m < 0x1p120f); };
-  const bool ok = room(mq) && room(mk) && room(mv) && mq * mk * (float)D < 0x1p120f;
+#pragma unroll
+  for (int db = 0; db < DB; db++)
+#pragma unroll
+    for (int i = 0; i < 16; i++) oacc[db][i] *= 1.f / kValueScale;
+  auto room = [](float m) { return m == 0.f || m >= 0x1p-90f; };
+  const bool ok = room(mq) && room(mk) && mq + mk < qk_limit && mv < kValueMost && mq * mk * (float)D < kDotMost;
   return __builtin_amdgcn_readfirstlane((int)ok) != 0;  // the same for the whole workgroup
 }
 
