@@ -542,6 +542,58 @@ def test_every_tile_and_kv_iteration_is_covered_exactly_once(tmp_path):
     assert out.returncode == 0 and out.stdout.split("\n")[0] == "ok %d" % len(lines) and "merge map ok" in out.stdout, out.stdout[-400:]
 
 
+STRIDED_HARNESS = r"""
+// Walks a plain launch of fewer workgroups than query tiles with the code the kernels run; arguments: tiles, compute units.
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+#include "attn_walk.h"
+struct Geom { int total_tiles, tiles_per_xcd, split_full, split_units, split_len, split_pmax, split_fuse0, split_claimers, split_dyn, split_s0, split_order, plain_stride; };
+int main() {
+  long strided = 0;
+  for (int cus = 1; cus <= 304; cus++)
+    for (int tiles = 1; tiles <= 900; tiles += cus < 40 ? 1 : 7) {
+      Geom g = {};
+      g.total_tiles = tiles;
+      g.tiles_per_xcd = (tiles + 7) / 8;
+      const int positions = 8 * g.tiles_per_xcd, nt = 3;
+      g.plain_stride = xdit::plain_launch_stride(positions, cus);
+      const int workgroups = g.plain_stride != 0 ? g.plain_stride : positions;
+      if (g.plain_stride % 8 != 0 || (g.plain_stride != 0 && (workgroups > cus || workgroups >= positions))) { printf("stride %d of %d tiles, %d units\n", g.plain_stride, tiles, cus); return 1; }
+      strided += g.plain_stride != 0;
+      std::vector<int> cover(tiles, 0);
+      for (int w = 0; w < workgroups; w++) {
+        xdit::WorkgroupWalk walk;
+        xdit::Segment s;
+        int position = w;
+        bool more = walk.start(g, nt, position) && walk.next(g, nt, s);
+        while (more) {  // the order of the kernels: first what the walk still has, then the next position
+          if (s.tile < 0 || s.tile >= tiles || s.tile / g.tiles_per_xcd != (w & 7) || s.it0 != 0 || s.it1 != nt || s.slot >= 0) { printf("segment of %d tiles, %d units\n", tiles, cus); return 1; }
+          cover[s.tile]++;
+          more = walk.next(g, nt, s);
+          if (!more) more = walk.next_position(g, nt, position, s);
+        }
+      }
+      for (int t = 0; t < tiles; t++) if (cover[t] != 1) { printf("tile %d of %d covered %d times, %d units\n", t, tiles, cover[t], cus); return 1; }
+    }
+  printf("ok %ld\n", strided);
+  return 0;
+}
+"""
+
+
+def test_plain_launch_of_fewer_workgroups_covers_every_tile_once(tmp_path):
+    """A plain launch whose workgroups run tile after tile, walked on the CPU with the code the kernels run: for
+    1 to 304 compute units and up to 900 query tiles every tile is run once, by a workgroup of its XCD, and
+    no more workgroups are started than compute units."""
+    src = tmp_path / "strided.cpp"
+    src.write_text(STRIDED_HARNESS)
+    exe = tmp_path / "strided"
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "xdit_amd", "csrc"), str(src), "-o", str(exe)])
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0 and int(out.stdout.split()[1]) > 10000, out.stdout
+
+
 def test_launch_plan_of_the_fp32_kernel():
     """fp32 problems run one workgroup per query tile: 128-row tiles with 32-key KV tiles, or
     64-row tiles with 64-key KV tiles when the 128-row tiles would fill less than three quarters

@@ -95,10 +95,10 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
   __shared__ int drawn[2];      // streamed sharing: KV tile of the stream position after next, by parity
   WorkgroupWalk walk;
   Segment seg;
-  int plain_block = (int)blockIdx.x;
+  int position = (int)blockIdx.x;  // of the dispatch order
   {
     const WalkGeom g = walk_geom(pp);
-    if (!walk.start(g, nt, plain_block) || !walk.next(g, nt, seg)) return;
+    if (!walk.start(g, nt, position) || !walk.next(g, nt, seg)) return;
   }
 
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -419,10 +419,7 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
         walk.claimed(g, (unsigned)__builtin_amdgcn_readfirstlane((int)ticket));
       }
       more = walk.next(g, nt, next_seg);
-      if (!more && g.plain_stride != 0) {  // a plain launch of fewer workgroups than tiles: on to the next tile
-        plain_block += g.plain_stride;
-        more = plain_block < 8 * g.tiles_per_xcd && walk.start(g, nt, plain_block) && walk.next(g, nt, next_seg);
-      }
+      if (!more) more = walk.next_position(g, nt, position, next_seg);  // a plain launch of fewer workgroups than tiles
     }
     __syncthreads();  // every wavefront is done with the K/V fragments of the last tile
     if (more) {

@@ -493,10 +493,8 @@ static inline unsigned resident_grid(AttnParams& q, const void* kernel, int thre
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, lds) != hipSuccess || n <= 0) n = -1;
     residency.store(n, std::memory_order_relaxed);
   }
-  const unsigned slots = n != 1 ? 0u : (unsigned)resident_cus(q.cu_count) & ~7u;
-  if (slots == 0 || grid <= slots) return grid;
-  q.plain_stride = (int)slots;
-  return slots;
+  if (n == 1) q.plain_stride = plain_launch_stride((int)grid, resident_cus(q.cu_count));
+  return q.plain_stride != 0 ? (unsigned)q.plain_stride : grid;
 }
 
 }  // namespace xdit

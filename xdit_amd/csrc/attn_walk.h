@@ -22,6 +22,14 @@ XDIT_HD int xcd_tile_index(int block, int tiles_per_xcd) {
   return (block & 7) * tiles_per_xcd + (block >> 3);
 }
 
+// The stride of a plain launch over `positions` of the dispatch order where `cus` workgroups run at once: the
+// workgroups to start, each going on to the position that far behind its last, or 0 where every position has a
+// workgroup of its own.
+XDIT_HD int plain_launch_stride(int positions, int cus) {
+  const int slots = cus & ~7;
+  return slots == 0 || positions <= slots ? 0 : slots;
+}
+
 // One piece of work of a workgroup: KV iterations [it0, it1) of query tile `tile`.  slot < 0: the
 // workgroup owns the whole tile and writes the final result; otherwise the piece is one part of a
 // query tile whose KV iterations are shared, and its partial result goes to that workspace slot.
@@ -38,7 +46,8 @@ struct Segment {
 // AttnParams (total_tiles, tiles_per_xcd, split_full, split_units, split_len, split_pmax,
 // split_fuse0, split_claimers, split_dyn, split_s0, split_order); `nt` is the number of KV iterations of a
 // whole tile.
-// Plain launch (split_units == 0): workgroup = one query tile over all KV iterations.  Balanced
+// Plain launch (split_units == 0): workgroup = one query tile over all KV iterations, or, started in
+// fewer workgroups than there are tiles, one such tile after the other (next_position).  Balanced
 // launch: the first split_full workgroups each take a whole query tile; the KV iterations of the
 // remaining query tiles, laid end to end, are cut into split_units ranges of split_len
 // iterations.  A range may cover the end of one query tile and the start of the next.  The ranges
@@ -130,6 +139,18 @@ struct WorkgroupWalk {
     s.tile = p.split_full + r;
     lin += s.it1 - s.it0;
     return true;
+  }
+
+  // Plain launch of fewer workgroups than positions of the dispatch order (plain_stride != 0; P has that
+  // member too): the workgroup that started at position w runs w, w + plain_stride, ... one after the
+  // other.  After its segment at `position`: the next one, false when there is none.  The stride is a multiple
+  // of eight, so a workgroup's tiles are of one XCD's range and ascend: past the first position without a
+  // tile there are only such.
+  template <typename P>
+  XDIT_HD bool next_position(const P& p, int nt, int& position, Segment& s) {
+    if (p.plain_stride == 0) return false;
+    position += p.plain_stride;
+    return position < 8 * p.tiles_per_xcd && start(p, nt, position) && next(p, nt, s);
   }
 
   // After a segment: true when the workgroup has to draw its next range from the counter
