@@ -4,6 +4,7 @@ nothing falls back to a CPU implementation."""
 import contextlib
 import gc
 import weakref
+from fractions import Fraction
 
 import pytest
 import torch
@@ -253,3 +254,36 @@ def test_outgrown_quantiser_scratch_stays_allocated(monkeypatch):
     for call in seen:                                                  # the jobs of a call do not share scratch
         spans = sorted(call)
         assert all(a + n <= b for (a, n), (b, _) in zip(spans, spans[1:]))
+
+
+def test_the_quantisers_quotient_lies_on_the_divisions_side_of_every_fp8_rounding_point():
+    """The quantiser divides by q = x r, y = q + r (x - q scale) with r the rounded reciprocal.  Before its last
+    rounding y is within 1.75 * 2^-23 units of the quotient (csrc/fp8_quant.hip), so it can only lie on another side of an
+    e4m3 rounding point m (sixteenths of a power of two) than the rounded quotient where x / scale comes that
+    close to the middle between m and a neighbouring fp32 number.  With 24-bit mantissas that is a congruence with a few
+    solutions per m: all of them, and as many again, are computed here in exact arithmetic."""
+    def rn(v):   # the nearest fp32 number, ties to even (no under- or overflow here)
+        e = 0
+        while abs(v) * Fraction(2) ** -e >= 2 ** 24: e += 1
+        while v != 0 and abs(v) * Fraction(2) ** -e < 2 ** 23: e -= 1
+        return round(v * Fraction(2) ** -e) * Fraction(2) ** e
+
+    seen = 0
+    for k in range(16, 32):
+        for bits, half in ((24, 1), (24, -1), (25, -1)) if k == 16 else ((24, 1), (24, -1)):
+            m = Fraction(k, 16)
+            middle = k * 2 ** (bits - 4) + half
+            for e in (0, 1):   # x / scale = mantissa of x / mantissa of scale, times two where that is below one
+                mod = 2 ** (bits + e)
+                for n in range(-16, 17):
+                    s = -n * pow(middle, -1, mod) % mod
+                    x = (middle * s + n) // mod
+                    if not (2 ** 23 <= s < 2 ** 24 and 2 ** 23 <= x < 2 ** 24): continue
+                    s, x = Fraction(s, 2 ** 23), Fraction(x << e, 2 ** 23)
+                    r = rn(1 / s)
+                    q = rn(x * r)
+                    y, quotient = rn(q + r * rn(x - q * s)), rn(x / s)
+                    assert abs(x / s - q) <= Fraction(3, 2) * (1 + Fraction(1, 2 ** 20)) * Fraction(1, 2 ** 23)
+                    assert ((y > m) - (y < m)) == ((quotient > m) - (quotient < m)), (x, s)
+                    seen += 1
+    assert seen > 200, seen
