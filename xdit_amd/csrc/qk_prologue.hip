@@ -203,7 +203,7 @@ __global__ __launch_bounds__(256) void prologue_rows_batch_kernel(const Prologue
 }
 
 // Across-heads form (the norm statistic runs over all H*D elements of a token and the gain has
-// H*D entries: Wan's norm_q / norm_k, transformer_wan.py:99-100): one workgroup per token, up to
+// H*D entries: Wan's norm_q / norm_k, transformer_wan.py:99-100), fp32 tensors: one workgroup per token, up to
 // kChunks 8-element chunks per thread held in registers between the reduction and the store.
 constexpr int kChunks = 4;
 
@@ -346,10 +346,9 @@ static void launch_token_wave(const PrologueParams& p, hipStream_t stream) {
 
 template <typename T>
 static hipError_t run(const PrologueParams& p, hipStream_t stream) {
-  if (p.norm == 2 && sizeof(T) == 2) {
+  if (p.norm == 2) {
     if constexpr (sizeof(T) == 2) launch_token_wave<T>(p, stream);
-  } else if (p.norm == 2) {
-    hipLaunchKernelGGL((prologue_token_kernel<T>), dim3((unsigned)((int64_t)p.B * p.S)), dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((prologue_token_kernel<T>), dim3((unsigned)((int64_t)p.B * p.S)), dim3(256), 0, stream, p);
   } else {
     const int64_t tokens = (int64_t)p.B * p.S;  // one wavefront each, four per workgroup
     hipLaunchKernelGGL((prologue_rows_kernel<T>), dim3((unsigned)((tokens + 3) / 4)), dim3(256), 0, stream, p);
