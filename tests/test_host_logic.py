@@ -3,6 +3,8 @@ argument domains, the joint-tensor step rule, ring ordering, registry behaviour,
 nothing falls back to a CPU implementation."""
 import contextlib
 import gc
+import threading
+import time
 import weakref
 from fractions import Fraction
 
@@ -254,6 +256,37 @@ def test_outgrown_quantiser_scratch_stays_allocated(monkeypatch):
     for call in seen:                                                  # the jobs of a call do not share scratch
         spans = sorted(call)
         assert all(a + n <= b for (a, n), (b, _) in zip(spans, spans[1:]))
+
+
+
+@pytest.mark.parametrize("what", ["quantiser", "attention"])
+def test_calls_of_several_threads_on_a_stream_do_not_mix_their_launches(monkeypatch, what):
+    """The scratch of a stream is written by a call's first launch and read by its last, and the C call that makes
+    them runs without the GIL: a second thread's call on the stream has to wait (device calls stubbed)."""
+    inside, most = [0], [0]
+
+    def launches(*args):
+        inside[0] += 1
+        most[0] = max(most[0], inside[0])
+        time.sleep(0.02)
+        inside[0] -= 1
+        return 0
+
+    class Lib:
+        xdit_fp8_quant_batch = xdit_attn_fwd = staticmethod(launches)
+        xdit_attn_workspace_bytes = staticmethod(lambda a: 4096)
+
+    monkeypatch.setattr(ops, "_check4", lambda *a: None)
+    monkeypatch.setattr(ops, "_stream", lambda device: 7)
+    monkeypatch.setattr(ops, "_on_device", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(ops._lib, "lib", Lib)
+    for pool in ("_QUANT_SCRATCH", "_WORKSPACE"):
+        monkeypatch.setattr(ops, pool, {})
+    x = torch.zeros(1, 2, 8, 64, dtype=torch.bfloat16)
+    threads = [threading.Thread(target=(lambda: ops.fp8_quant(x)) if what == "quantiser" else (lambda: ops.attn_fwd(x, x, x))) for _ in range(4)]
+    for t in threads: t.start()
+    for t in threads: t.join()
+    assert most[0] == 1
 
 
 def test_the_quantisers_quotient_lies_on_the_divisions_side_of_every_fp8_rounding_point():

@@ -64,6 +64,15 @@ class _on_device:
 
 _WORKSPACE = {}
 _RETIRED = []
+_STREAM_LOCKS = {}
+
+
+def _stream_lock(device, stream):
+    """Held while a call takes its scratch and launches: the scratch of a (device, stream) serves one call after
+    the other, and the C call releases the GIL between the launches that write it and those that read it."""
+    key = (device, stream)
+    lock = _STREAM_LOCKS.get(key)
+    return lock if lock is not None else _STREAM_LOCKS.setdefault(key, threading.Lock())
 
 
 def _workspace(device, stream, nbytes):
@@ -273,7 +282,7 @@ def attn_fwd(q, k, v, softmax_scale=None, causal=False, k2=None, v2=None,
     a.stream = stream
     L = _lib.lib()
     entry = None
-    with _on_device(device):
+    with _stream_lock(device, stream), _on_device(device):
         if noalloc:
             a.workspace, a.workspace_bytes = None, 0
             if not balance:
@@ -295,8 +304,8 @@ def attn_fwd(q, k, v, softmax_scale=None, causal=False, k2=None, v2=None,
                 rc = L.xdit_attn_fwd_two_queries(ctypes.byref(a), ctypes.byref(plan.tail))
             else:
                 rc = L.xdit_attn_fwd(ctypes.byref(a))
-    if entry is not None:
-        entry[1] = 1 if rc == 0 else 0   # after a failure the next call has the counters cleared again
+        if entry is not None:
+            entry[1] = 1 if rc == 0 else 0   # after a failure the next call has the counters cleared again
     if rc != 0:
         _lib.check(rc)
     return out, lse
@@ -445,15 +454,8 @@ def fp8_quant_batch(jobs, joined=()):
         plans[key] = arr
     stream = _stream(device)
     need = [4 * max(4096, a.B * a.H) for a in arr]
-    buf = _QUANT_SCRATCH.get((device, stream))
-    if buf is None or buf.numel() < sum(need):
-        if buf is not None:
-            _RETIRED.append(buf)   # a graph captured on this stream may hold its address
-        buf = torch.empty(sum(need), dtype=torch.uint8, device=device)
-        _QUANT_SCRATCH[(device, stream)] = buf
-    scratch = buf.data_ptr()
     keep, out = [], []
-    for i, (a, size, (x, pt, scale, had, x2)) in enumerate(zip(arr, need, jobs)):
+    for i, (a, (x, pt, scale, had, x2)) in enumerate(zip(arr, jobs)):
         B, H, S, D = x.shape
         y = torch.empty((B, H, S + x2.shape[2], D) if i in joined else x.shape, dtype=torch.float8_e4m3fn, device=device)
         descale = torch.empty(x.shape[:2], dtype=torch.float32, device=device)
@@ -463,8 +465,6 @@ def fp8_quant_batch(jobs, joined=()):
             keep.append(scale)
             a.scale_in = scale.data_ptr()
         a.stream = stream
-        a.scratch, a.scratch_bytes = scratch, size
-        scratch += size
         if i in joined:
             a.x2, a.y2 = x2.data_ptr(), a.y + S * D
             out.append((y, descale))
@@ -475,7 +475,17 @@ def fp8_quant_batch(jobs, joined=()):
             if a.S2:
                 a.x2, a.y2 = x2.data_ptr(), y2.data_ptr()
             out.append((y, y2, descale))
-    with _on_device(device):
+    with _stream_lock(device, stream), _on_device(device):
+        buf = _QUANT_SCRATCH.get((device, stream))
+        if buf is None or buf.numel() < sum(need):
+            if buf is not None:
+                _RETIRED.append(buf)   # a graph captured on this stream may hold its address
+            buf = torch.empty(sum(need), dtype=torch.uint8, device=device)
+            _QUANT_SCRATCH[(device, stream)] = buf
+        scratch = buf.data_ptr()
+        for a, size in zip(arr, need):
+            a.scratch, a.scratch_bytes = scratch, size
+            scratch += size
         rc = _lib.lib().xdit_fp8_quant_batch(arr, n)
     if rc != 0:
         _lib.check(rc)
