@@ -202,8 +202,10 @@ typedef struct {
   int32_t claimers;
   int32_t first_claimer;
   int32_t counter;
-  int32_t workgroups;          /* grid of the attention kernel; a plain launch (ranges == 0) of more than fit on the
-                                  GPU at once starts as many as do, which run the others one after the other */
+  int32_t workgroups;          /* workgroups the attention kernel's work is cut into; all of them are launched,
+                                  except in a plain launch (ranges == 0) of more than there are compute units
+                                  whose workgroups fill a compute unit alone: one per compute unit is then
+                                  started and runs the others one after the other */
   int32_t streamed;            /* != 0: streamed sharing instead of ranges: the `claimers` workgroups are dealt
                                   out over the shared tiles in contiguous groups; every member owns
                                   `range_len` KV iterations of its tile and draws the others one at a

@@ -309,8 +309,10 @@ __device__ __forceinline__ bool split_loop(const AttnParams& p, unsigned char* s
       };
 #pragma unroll
       for (int n = 0; n < 3; n++) read_v(0, n);
-      // One sum where 256 registers do not hold two (16 heads of 4000 at head_dim 88, 96: 540, 554 us with two, 521, 514
-      // with one), two otherwise (37000 keys at head_dim 72: 3754 us, 3978 with one).
+      // One sum or two, by measurement: with two wavefronts per SIMD head_dims 72 to 96 leave a few registers over 256
+      // to scratch memory either way (14 to 22).  16 heads of 4000 at head_dim 88, 96: 535, 536 us with two, 524, 528 with
+      // one; at 72, 80: 487, 489 with two, 491 to 499, 489 with one; 2 heads of 37000 at 72, 80: 6325, 6375 with two,
+      // 6460, 6425 with one.
       constexpr int NS = KS == 1 && (D8 == 11 || D8 == 12) ? 1 : 2;
       f32x16 sum[NS];
       static_for<12 * DB>([&](auto I) {

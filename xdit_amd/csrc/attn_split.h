@@ -479,7 +479,8 @@ static inline unsigned split_grid(const AttnParams& q) {
 // workgroups fill a compute unit alone, one workgroup per compute unit that runs tile after tile
 // (plain_stride): the next tile's queries and first keys are then on their way while the rows of the current
 // one are stored, and no compute unit waits for a workgroup to be dispatched.  40 heads of 32760 queries on
-// 512 keys 412 -> 391 us, four ring steps of 24 heads of 4608 x 1152 345 -> 339.  Workgroups that share a
+// 512 keys 425 -> 409 us, four ring steps of 24 heads of 4608 x 1152 354 -> 349 (both sides on one box; no change on
+// long key ranges, 5 heads of 75600 in fp8).  Workgroups that share a
 // compute unit hide each other's start already, and dealing their tiles out beforehand costs more than it
 // gives (128 rows: 24 heads of 14933 on 512 keys 111.3 -> 116.2 us, head_dim 64, 24 heads of 18882 on 77 keys
 // 33.5 -> 34.6).  The tiles of a workgroup lie a multiple of eight apart in the dispatch order, so they stay
