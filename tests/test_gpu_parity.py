@@ -1574,12 +1574,16 @@ def test_fp8_quant_static_scale_of_every_bf16_value(gpu, scale):
     assert torch.equal(y.view(torch.uint8), want) and (y.view(torch.uint8) == 0x80).any()
 
 
-@pytest.mark.parametrize("dtype,D,Sk,Sk2", [(torch.bfloat16, 128, 70, 0), (torch.float16, 72, 120, 0), (torch.bfloat16, 64, 129, 40), (torch.float8_e4m3fn, 128, 200, 0)])
-@pytest.mark.parametrize("rows", [128, 256, 384])
+@pytest.mark.parametrize("dtype,D,Sk,Sk2,rows", [(torch.bfloat16, 128, 70, 0, 256), (torch.bfloat16, 128, 70, 0, 384), (torch.float16, 72, 120, 0, 256),
+                                                 (torch.float16, 72, 120, 0, 384), (torch.bfloat16, 64, 129, 40, 384), (torch.bfloat16, 56, 129, 40, 256),
+                                                 (torch.float8_e4m3fn, 128, 200, 0, 256), (torch.float8_e4m3fn, 128, 200, 0, 384),
+                                                 (torch.float8_e4m3fn, 64, 200, 33, 384)])
 def test_plain_launch_of_fewer_workgroups_than_tiles(gpu, force_rows, dtype, D, Sk, Sk2, rows):
     """A plain launch planned for eight compute units (every workgroup runs several query tiles, the last
     ones ragged, XCDs with one tile more than others) against one workgroup per tile: the same bits, as
-    a forward and as a ring step that folds into an accumulator."""
+    a forward and as a ring step that folds into an accumulator.  The shapes whose workgroups fill a compute unit
+    alone, by the registers they take (more than 128 at 256 rows, more than 80 at 384): those that share one, of 128 rows
+    and mostly of 256 rows at head_dim 64, keep one tile each."""
     g = torch.Generator().manual_seed(D + Sk)
     f8 = dtype == torch.float8_e4m3fn
     mk = lambda s: torch.randn(2, 5, s, D, generator=g).to(dtype).to(gpu)
