@@ -188,6 +188,9 @@ int xdit_attn_fwd_noalloc(const xdit_attn_args* args);
  * rows with `kv_iterations` tiles of 32 keys, or, when those would leave more than a quarter of
  * the compute units without a workgroup, of 64 rows with tiles of 64 keys.  No counterpart in the
  * reference.
+ * A plain 16-bit forward over few keys (xdit_attn_fwd at most four tiles of 64 keys at head_dim above 64, eight below, both
+ * segments together) with rows_per_workgroup and balance left at 0 runs on a kernel that holds the keys in LDS and deals
+ * out its rows otherwise; it gives the bits of the launch described here.
  */
 typedef struct {
   uint32_t struct_size;        /* = sizeof(xdit_launch_plan), set by the caller */

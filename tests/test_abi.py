@@ -594,6 +594,47 @@ def test_plain_launch_of_fewer_workgroups_covers_every_tile_once(tmp_path):
     assert out.returncode == 0 and int(out.stdout.split()[1]) > 10000, out.stdout
 
 
+RESIDENT_HARNESS = r"""
+// Deals out the query rows of launches over few keys with the code the kernel runs.
+#include <cstdio>
+#include <vector>
+#include "resident_walk.h"
+int main() {
+  long n = 0;
+  for (int cus : {1, 3, 8, 100, 256, 304})
+    for (int bh : {1, 2, 5, 24, 40, 300, 2000})
+      for (int Sq : {1, 31, 32, 33, 100, 1024, 4250, 14933, 32760})
+        for (int nt = 1; nt <= 8; nt++)
+          for (int wavefronts : {8, 12}) {
+            if ((long)bh * Sq > 2000000) continue;
+            const int groups = (Sq + 31) / 32, parts = xdit::resident_parts(bh, Sq, nt, wavefronts, cus);
+            if (parts < 1 || parts > groups) { printf("%d parts of %d groups\n", parts, groups); return 1; }
+            const int total = bh * parts, per_xcd = (total + 7) / 8;
+            std::vector<int> cover((size_t)bh * groups, 0);
+            for (int w = 0; w < 8 * per_xcd; w++) {
+              xdit::ResidentPart r;
+              if (!xdit::resident_part(w, per_xcd, total, parts, Sq, r)) continue;
+              if (r.bh < 0 || r.bh >= bh || r.g0 < 0 || r.g0 >= r.g1 || r.g1 > groups || r.g1 - r.g0 > (groups + parts - 1) / parts) { printf("part\n"); return 1; }
+              for (int g = r.g0; g < r.g1; g++) cover[(size_t)r.bh * groups + g]++;
+            }
+            for (int c : cover) if (c != 1) { printf("a group is covered %d times\n", c); return 1; }
+            n++;
+          }
+  printf("ok %ld\n", n);
+  return 0;
+}
+"""
+
+
+def test_launch_over_few_keys_covers_every_row_group_once(tmp_path):
+    src = tmp_path / "resident.cpp"
+    src.write_text(RESIDENT_HARNESS)
+    exe = tmp_path / "resident"
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "xdit_amd", "csrc"), str(src), "-o", str(exe)])
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0 and int(out.stdout.split()[1]) > 2000, out.stdout
+
+
 def test_launch_plan_of_the_fp32_kernel():
     """fp32 problems run one workgroup per query tile: 128-row tiles with 32-key KV tiles, or
     64-row tiles with 64-key KV tiles when the 128-row tiles would fill less than three quarters

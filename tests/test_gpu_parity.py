@@ -1603,6 +1603,45 @@ def test_plain_launch_of_fewer_workgroups_than_tiles(gpu, force_rows, dtype, D, 
     assert all(torch.equal(a, b) for a, b in zip(*got))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,Sq,Sq2,Sk,Sk2", [(128, 1, 0, 1, 0), (128, 777, 0, 256, 0), (128, 300, 85, 100, 120), (128, 33, 0, 65, 128), (120, 97, 0, 190, 0),
+                                             (104, 400, 0, 64, 0), (96, 500, 31, 129, 60), (88, 1000, 0, 77, 0), (80, 65, 0, 256, 0), (72, 2000, 0, 120, 0),
+                                             (64, 513, 0, 512, 0), (64, 31, 17, 300, 200), (56, 200, 0, 450, 0), (32, 100, 0, 77, 0), (8, 70, 0, 9, 0)])
+def test_few_keys_resident_in_lds_give_the_bits_of_the_tiled_launch(gpu, dtype, D, Sq, Sq2, Sk, Sk2):
+    """The kernel that keeps a head's keys in LDS, planned for few and for all compute units (one to many row groups
+    a wavefront), against the tiled kernel (forced by its rows per workgroup): the same bits, in both memory orders, with
+    the tensors framed in NaN columns, and next to the oracle."""
+    g = torch.Generator().manual_seed(D + Sq + Sk)
+    B, H = 2, 3
+
+    def mk(s, bshd):
+        x = torch.randn(B, H, s, D, generator=g).to(dtype)
+        if s == 0:
+            return None
+        shape = (B, s, H, D + 16) if bshd else (B, H, s, D + 16)
+        frame = torch.full(shape, float("nan"), dtype=dtype, device=gpu)
+        view = (frame.transpose(1, 2) if bshd else frame)[..., 8:8 + D]
+        view.copy_(x)
+        return view
+    for bshd in (False, True):
+        q, q2, k, v, k2, v2 = mk(Sq, bshd), mk(Sq2, bshd), mk(Sk, bshd), mk(Sk, bshd), mk(Sk2, bshd), mk(Sk2, bshd)
+        frame = torch.zeros((B, Sq + Sq2, H, D + 16) if bshd else (B, H, Sq + Sq2, D + 16), dtype=dtype, device=gpu)
+        out = (frame.transpose(1, 2) if bshd else frame)[..., 8:8 + D]
+        got = []
+        for tuning in (dict(rows_per_workgroup=128), dict(), dict(cu_count=1), dict(cu_count=9)):
+            ops.TUNING.update(tuning)
+            try:
+                o, l = ops.attn_fwd(q, k, v, k2=k2, v2=v2, q2=q2, out=out)
+            finally:
+                ops.TUNING.update(rows_per_workgroup=0, cu_count=0)
+            assert frame[..., :8].count_nonzero() == 0 and frame[..., 8 + D:].count_nonzero() == 0   # nothing beside the rows
+            got.append((o.clone(), l))
+        assert all(torch.equal(a, b) for other in got[1:] for a, b in zip(got[0], other))
+    cat = lambda a, b: (a if b is None else torch.cat([a, b], 2)).cpu()
+    ro, rl = O.attn_fwd_ref(cat(q, q2), cat(k, k2), cat(v, v2))
+    assert _err(got[1][0], ro) <= 2e-2 and _err(got[1][1], rl) <= 1e-3
+
+
 @pytest.mark.parametrize("strategy", ["front", "rear"])
 @pytest.mark.parametrize("case", ["bf16", "fp16", "fp8", "bshd", "views"])
 def test_usp_joint_queries_are_read_where_they_are(gpu, monkeypatch, strategy, case):

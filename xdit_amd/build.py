@@ -12,7 +12,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJDIR = os.path.join(HERE, "csrc", "build")
 LIB = os.path.join(HERE, "libxdit_amd_attn.so")
-SOURCES = ["api.hip", "attn_fwd_16.hip", "attn_fwd_16_ring.hip", "attn_fwd_fp8.hip", "attn_fwd_f32.hip", "lse_merge.hip", "fp8_quant.hip", "qk_prologue.hip"]
+SOURCES = ["api.hip", "attn_fwd_16.hip", "attn_fwd_16_ring.hip", "attn_fwd_16_resident.hip", "attn_fwd_fp8.hip", "attn_fwd_f32.hip", "lse_merge.hip", "fp8_quant.hip", "qk_prologue.hip"]
 FLAGS = [
     # an atomic under a one-lane branch stays one plain atomic whose result is awaited where it is used
     "-mllvm", "-amdgpu-atomic-optimizer-strategy=None",

@@ -10,6 +10,7 @@
 
 #include "attn_split.h"
 #include "launchers.h"
+#include "resident_walk.h"
 
 // Scratch of xdit_attn_fwd_noalloc: the balanced launch's partial results and range counter live
 // here instead of in a caller workspace.  One copy per GPU the library runs on, held until the
@@ -167,6 +168,14 @@ LaunchChoice choose_launch(const xdit_attn_args* a, bool plain = false, bool fol
     }
   }
   return best;
+}
+
+// Whether a 16-bit forward runs on the kernel that keeps the keys of a head in LDS: where they fit, unless the
+// caller asks for a shape or a balance of the tiled launch.
+bool resident_path(const xdit_attn_args* a) {
+  const int D = kernel_head_dim(a->D);
+  const int64_t nt = (a->Sk + xdit::kKeysPerTile - 1) / xdit::kKeysPerTile + (a->Sk2 + xdit::kKeysPerTile - 1) / xdit::kKeysPerTile;
+  return mfma16_path(a) && a->rows_per_workgroup == 0 && a->balance == 0 && nt <= (D == 128 ? xdit::kResidentTiles<128> : xdit::kResidentTiles<64>);
 }
 
 // The two tuning fields of xdit_attn_args.
@@ -400,7 +409,10 @@ static int attn_fwd_impl(const xdit_attn_args* a, const xdit_ring_acc* acc, cons
   // launch follows: the next call on it may then say "preserved" whether this one is balanced or not.
   if (p.ws_out != nullptr && !p.ws_preserved) xdit::launch_counter_reset(p.ws_out, stream);
   hipError_t e;
-  if (fp8 || mfma16_path(a)) {
+  if (acc == nullptr && resident_path(a)) {
+    p.d_actual = a->D;
+    e = xdit::launch_attn_fwd_16_resident(p, a->dtype == XDIT_DTYPE_FP16, kernel_head_dim(a->D), stream);
+  } else if (fp8 || mfma16_path(a)) {
     const int D = fp8 ? a->D : kernel_head_dim(a->D);
     if (!fp8) p.d_actual = a->D;
     const bool fused = acc != nullptr;

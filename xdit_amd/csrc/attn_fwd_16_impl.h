@@ -43,6 +43,132 @@ constexpr int kRowsPerWave = 32;
 // LDS fragment reads are issued this many MFMAs ahead of the MFMA that consumes them.
 constexpr int kPrefetch = 4;
 
+// The arithmetic of one wavefront on one KV tile in LDS.
+template <typename T, int D, int DC>
+struct TileMath {
+  typedef TileGeom<D> G;
+  typedef typename Mfma16<T>::vec8 vec8;
+  typedef typename Mfma16<T>::vec2 vec2;
+  static_assert(DC % 16 == 0 && DC <= D, "computed head_dim");
+  static constexpr int KSTEPS = DC / 16;          // contraction steps of QK^T
+  static constexpr int DBLOCKS = (DC + 31) / 32;  // 32-row blocks of O^T
+
+  // ---- LDS read addresses: one per-lane base each for K and V, the rest are immediates ------
+  // K fragment (A operand of S^T) for key block kb, step ks: row 32kb + l32, bytes 32ks + 16hh.
+  //   row -> piece (row % NG), slot (row / NG)
+  static constexpr int K_KB_STEP = (32 / G::NG) * G::ROW_BYTES;  // +32 rows = +32/NG slots
+  static __device__ __forceinline__ unsigned k_read_offset(int lane) {
+    const int l32 = lane & 31, hh = lane >> 5;
+    return (l32 % G::NG) * G::K_PITCH + (l32 / G::NG) * G::ROW_BYTES + hh * 16;
+  }
+  // V^T fragment (A operand of O^T) for d block db, key step j (16 keys), half rd (keys +0 / +8):
+  // as a SOURCE lane of the transposed read, lane (group g = lane/16, s = lane%16) supplies the
+  // 8 bytes at key row 16j + 8rd + 4hh + s/4, elements d = 32db + 16(g%2) + 4(s%4) .. +3; the
+  // read returns to lane (g, i) the four keys of that row group at d = 32db + 16(g%2) + i.
+  // +8 rows (rd) and +16 rows (j): both keep row % NG pattern simple because NG is 8 or 16.
+  static constexpr int V_RD_STEP = (G::NG == 16) ? 8 * G::V_PITCH : G::ROW_BYTES;  // NG=8: +8 rows = +1 slot
+  static constexpr int V_J_STEP = (16 / G::NG) * G::ROW_BYTES;
+  static __device__ __forceinline__ unsigned v_read_offset(int lane) {
+    const int vsrc_row = 4 * (lane >> 5) + ((lane & 15) >> 2);  // row within the 16-key step, rd = 0
+    return G::K_BYTES + (vsrc_row % G::NG) * G::V_PITCH + (vsrc_row / G::NG) * G::ROW_BYTES + (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+  }
+
+  // S^T = K Q^T : 2 blocks of 32 keys x 32 queries
+  static __device__ __forceinline__ void logits(f32x16 (&sacc)[2], const vec8 (&qf)[KSTEPS], unsigned kaddr) {
+    constexpr int PD = kPrefetch;   // K fragment reads in flight
+    constexpr int NR = 2 * KSTEPS;  // reads (= MFMAs) of this product
+    vec8 kf[NR];  // in MFMA order: contraction step i / 2 of key block i % 2, so that consecutive MFMAs share their Q fragment
+    static_for<PD>([&](auto I) {
+      constexpr int i_ = I;
+      lds_read_b128<(i_ % 2) * K_KB_STEP + (i_ / 2) * 32>(kf[i_], kaddr);
+    });
+#pragma unroll
+    for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) sacc[kb][e] = 0.f;
+    static_for<NR>([&](auto I) {
+      constexpr int i_ = I;
+      constexpr int younger = (i_ + PD <= NR ? PD : NR - i_) - 1;
+      lds_wait<younger>(kf[i_]);
+      sacc[i_ % 2] = Mfma16<T>::mma(kf[i_], qf[i_ / 2], sacc[i_ % 2]);
+      if constexpr (i_ + PD >= NR && i_ + 1 < NR) __builtin_amdgcn_sched_barrier(0);  // issued before the next wait, not after the last one
+      if constexpr (i_ + PD < NR) {
+        constexpr int n = i_ + PD;
+        lds_read_b128<(n % 2) * K_KB_STEP + (n / 2) * 32>(kf[n], kaddr);
+      }
+    });
+  }
+
+  // Only the first `left` keys of the tile exist.
+  static __device__ __forceinline__ void mask(f32x16 (&sacc)[2], int left) {
+    const int hh = lane_now() >> 5;
+#pragma unroll
+    for (int kb = 0; kb < 2; kb++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        int key = 32 * kb + 8 * (e >> 2) + 4 * hh + (e & 3);
+        if (key >= left) sacc[kb][e] = -INFINITY;
+      }
+  }
+
+  // The largest logit of the lane's query in this tile (both halves of the wavefront agree).
+  static __device__ __forceinline__ float row_max(const f32x16 (&sacc)[2]) {
+    float mx = sacc[0][0];
+#pragma unroll
+    for (int e = 1; e < 16; e++) mx = fmaxf(mx, sacc[0][e]);
+#pragma unroll
+    for (int e = 0; e < 16; e++) mx = fmaxf(mx, sacc[1][e]);
+    return max_halves(mx);
+  }
+
+  // P^T as B operands: pf[j] = keys 16j..16j+15 of this tile (permuted inside); l_part grows by this lane's
+  // share of their sum.  mc: the row maximum in use, in log2 units.
+  static __device__ __forceinline__ void probabilities(const f32x16 (&sacc)[2], float c, float mc, float& l_part, vec8 (&pf)[4]) {
+#pragma unroll
+    for (int kb = 0; kb < 2; kb++) {
+#pragma unroll
+      for (int e = 0; e < 16; e += 2) {
+        float p0 = fast_exp2(__builtin_fmaf(sacc[kb][e], c, -mc));
+        float p1 = fast_exp2(__builtin_fmaf(sacc[kb][e + 1], c, -mc));
+        l_part += p0 + p1;
+        f32x2 pp = {p0, p1};
+        vec2 pk = __builtin_convertvector(pp, vec2);
+        const int j = 2 * kb + (e >> 3);
+        pf[j][(e & 7)] = pk[0];
+        pf[j][(e & 7) + 1] = pk[1];
+      }
+    }
+  }
+
+  // O^T += V^T P^T
+  static __device__ __forceinline__ void values(f32x16 (&oacc)[DBLOCKS], const vec8 (&pf)[4], unsigned vaddr) {
+    constexpr int PD = kPrefetch;  // MFMAs whose two V^T reads are in flight
+    constexpr int NM = 4 * DBLOCKS;
+    typedef __attribute__((ext_vector_type(8))) short s16x8;
+    s16x4 v0[NM], v1[NM];
+    static_for<PD>([&](auto I) {
+      constexpr int i_ = I;
+      constexpr int off = (i_ / DBLOCKS) * V_J_STEP + (i_ % DBLOCKS) * 64;
+      lds_read_tr16_b64<off>(v0[i_], vaddr);
+      lds_read_tr16_b64<off + V_RD_STEP>(v1[i_], vaddr);
+    });
+    static_for<NM>([&](auto I) {
+      constexpr int i_ = I;
+      constexpr int younger = 2 * ((i_ + PD <= NM ? PD : NM - i_) - 1);
+      lds_wait2<younger>(v0[i_], v1[i_]);
+      s16x8 vv = __builtin_shufflevector(v0[i_], v1[i_], 0, 1, 2, 3, 4, 5, 6, 7);
+      oacc[i_ % DBLOCKS] = Mfma16<T>::mma(__builtin_bit_cast(vec8, vv), pf[i_ / DBLOCKS], oacc[i_ % DBLOCKS]);
+      if constexpr (i_ + PD >= NM && i_ + 1 < NM) __builtin_amdgcn_sched_barrier(0);
+      if constexpr (i_ + PD < NM) {
+        constexpr int n = i_ + PD;
+        constexpr int off = (n / DBLOCKS) * V_J_STEP + (n % DBLOCKS) * 64;
+        lds_read_tr16_b64<off>(v0[n], vaddr);
+        lds_read_tr16_b64<off + V_RD_STEP>(v1[n], vaddr);
+      }
+    });
+  }
+};
+
 // Output staging block of a wavefront in the epilogue: 32 rows of 64 16-bit columns, rows 8 bytes
 // apart from a multiple of 128 so that the 8-byte writes of the 32 lanes of a half hit 32 banks.
 constexpr int kStagePitchBytes = 64 * 2 + 8;
@@ -80,11 +206,11 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
   constexpr int kWaves = NW;
   constexpr int kRowsPerBlock = kRowsPerWave * kWaves;
   typedef typename Mfma16<T>::vec8 vec8;
-  typedef typename Mfma16<T>::vec2 vec2;
   typedef TileGeom<D> G;
-  static_assert(DC % 16 == 0 && DC <= D && (PAD || DC == D), "computed head_dim");
-  constexpr int KSTEPS = DC / 16;          // contraction steps of QK^T
-  constexpr int DBLOCKS = (DC + 31) / 32;  // 32-row blocks of O^T
+  typedef TileMath<T, D, DC> M;
+  static_assert(PAD || DC == D, "computed head_dim");
+  constexpr int KSTEPS = M::KSTEPS;
+  constexpr int DBLOCKS = M::DBLOCKS;
   constexpr int kStagePitch = kStagePitchBytes;   // LDS row pitch of the output staging block
   constexpr int kStageBytes = kStageBytesPerWave;
 
@@ -160,23 +286,10 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
     ld_left -= kKeysPerTile;
   };
 
-  // ---- LDS read addresses: one per-lane base each for K and V, the rest are immediates ------
-  // K fragment (A operand of S^T) for key block kb, step ks: row 32kb + l32, bytes 32ks + 16hh.
-  //   row -> piece (row % NG), slot (row / NG)
-  unsigned kbase_off = lds_base + (l32 % G::NG) * G::K_PITCH + (l32 / G::NG) * G::ROW_BYTES + hh * 16;
+  unsigned kbase_off = lds_base + M::k_read_offset(lane);
   asm volatile("" : "+v"(kbase_off));  // one register, not its summands, lives through the loop
-  constexpr int K_KB_STEP = (32 / G::NG) * G::ROW_BYTES;  // +32 rows = +32/NG slots
-  // V^T fragment (A operand of O^T) for d block db, key step j (16 keys), half rd (keys +0 / +8):
-  // as a SOURCE lane of the transposed read, lane (group g = lane/16, s = lane%16) supplies the
-  // 8 bytes at key row 16j + 8rd + 4hh + s/4, elements d = 32db + 16(g%2) + 4(s%4) .. +3; the
-  // read returns to lane (g, i) the four keys of that row group at d = 32db + 16(g%2) + i.
-  const int vsrc_row = 4 * hh + ((lane & 15) >> 2);  // row within the 16-key step, rd = 0
-  unsigned vbase_off = lds_base + G::K_BYTES + (vsrc_row % G::NG) * G::V_PITCH + (vsrc_row / G::NG) * G::ROW_BYTES +
-                       (16 * ((lane >> 4) & 1) + 4 * (lane & 3)) * 2;
+  unsigned vbase_off = lds_base + M::v_read_offset(lane);
   asm volatile("" : "+v"(vbase_off));
-  // +8 rows (rd) and +16 rows (j): both keep row % NG pattern simple because NG is 8 or 16.
-  constexpr int V_RD_STEP = (G::NG == 16) ? 8 * G::V_PITCH : G::ROW_BYTES;  // NG=8: +8 rows = +1 slot
-  constexpr int V_J_STEP = (16 / G::NG) * G::ROW_BYTES;
 
   const float c = pp->scale * kLog2e;  // logits are kept in log2 units
 
@@ -294,52 +407,14 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
       const unsigned kaddr = kbase_off + buf * G::BUF_BYTES;
       const unsigned vaddr = vbase_off + buf * G::BUF_BYTES;
 
-      // ---- S^T = K Q^T : 2 blocks of 32 keys x 32 queries ---------------------------------
       f32x16 sacc[2];
-      {
-        constexpr int PD = kPrefetch;   // K fragment reads in flight
-        constexpr int NR = 2 * KSTEPS;  // reads (= MFMAs) of this product
-        vec8 kf[NR];  // in MFMA order: contraction step i / 2 of key block i % 2, so that consecutive MFMAs share their Q fragment
-        static_for<PD>([&](auto I) {
-          constexpr int i_ = I;
-          lds_read_b128<(i_ % 2) * K_KB_STEP + (i_ / 2) * 32>(kf[i_], kaddr);
-        });
-#pragma unroll
-        for (int kb = 0; kb < 2; kb++)
-#pragma unroll
-          for (int e = 0; e < 16; e++) sacc[kb][e] = 0.f;
-        static_for<NR>([&](auto I) {
-          constexpr int i_ = I;
-          constexpr int younger = (i_ + PD <= NR ? PD : NR - i_) - 1;
-          lds_wait<younger>(kf[i_]);
-          sacc[i_ % 2] = Mfma16<T>::mma(kf[i_], qf[i_ / 2], sacc[i_ % 2]);
-          if constexpr (i_ + PD >= NR && i_ + 1 < NR) __builtin_amdgcn_sched_barrier(0);  // issued before the next wait, not after the last one
-          if constexpr (i_ + PD < NR) {
-            constexpr int n = i_ + PD;
-            lds_read_b128<(n % 2) * K_KB_STEP + (n / 2) * 32>(kf[n], kaddr);
-          }
-        });
-      }
-      // ---- mask keys past the end of the segment (only its last tile can be partial) -------
-      if (left < kKeysPerTile) {
-        const int hh = lane_now() >> 5;
-#pragma unroll
-        for (int kb = 0; kb < 2; kb++)
-#pragma unroll
-          for (int e = 0; e < 16; e++) {
-            int key = 32 * kb + 8 * (e >> 2) + 4 * hh + (e & 3);
-            if (key >= left) sacc[kb][e] = -INFINITY;
-          }
-      }
+      M::logits(sacc, qf, kaddr);
+      if (left < kKeysPerTile) M::mask(sacc, left);  // keys past the end of the segment (only its last tile can be partial)
 
       // ---- online softmax ---------------------------------------------------------------
-      float mx = sacc[0][0];
-#pragma unroll
-      for (int e = 1; e < 16; e++) mx = fmaxf(mx, sacc[0][e]);
-#pragma unroll
-      for (int e = 0; e < 16; e++) mx = fmaxf(mx, sacc[1][e]);
-      mx = max_halves(mx);
-      const float m_new = fmaxf(m_used, mx);
+      // (The rescaling stands here and not in TileMath: there it costs a register, which is the one too many
+      // for four wavefronts of head_dim 64 on a SIMD: 24 heads of 14933 on 512 keys 62.8 -> 73.3 us.)
+      const float m_new = fmaxf(m_used, M::row_max(sacc));
       const bool grow = (m_new - m_used) * c > kLazyRescaleLog2;  // true on the first tile (-inf)
       if (__builtin_amdgcn_ballot_w64(grow) != 0) {
         const float alpha = fast_exp2((m_used - m_new) * c);  // 0 on the first tile
@@ -350,50 +425,9 @@ __device__ __forceinline__ void attn_workgroup(unsigned char* smem) {
 #pragma unroll
           for (int e = 0; e < 16; e++) oacc[db][e] *= alpha;
       }
-      const float mc = m_used * c;
-      vec8 pf[4];  // P^T as B operands: pf[j] = keys 16j..16j+15 of this tile (permuted inside)
-#pragma unroll
-      for (int kb = 0; kb < 2; kb++) {
-#pragma unroll
-        for (int e = 0; e < 16; e += 2) {
-          float p0 = fast_exp2(__builtin_fmaf(sacc[kb][e], c, -mc));
-          float p1 = fast_exp2(__builtin_fmaf(sacc[kb][e + 1], c, -mc));
-          l_part += p0 + p1;
-          f32x2 pp = {p0, p1};
-          vec2 pk = __builtin_convertvector(pp, vec2);
-          const int j = 2 * kb + (e >> 3);
-          pf[j][(e & 7)] = pk[0];
-          pf[j][(e & 7) + 1] = pk[1];
-        }
-      }
-
-      // ---- O^T += V^T P^T ------------------------------------------------------------------
-      {
-        constexpr int PD = kPrefetch;  // MFMAs whose two V^T reads are in flight
-        constexpr int NM = 4 * DBLOCKS;
-        typedef __attribute__((ext_vector_type(8))) short s16x8;
-        s16x4 v0[NM], v1[NM];
-        static_for<PD>([&](auto I) {
-          constexpr int i_ = I;
-          constexpr int off = (i_ / DBLOCKS) * V_J_STEP + (i_ % DBLOCKS) * 64;
-          lds_read_tr16_b64<off>(v0[i_], vaddr);
-          lds_read_tr16_b64<off + V_RD_STEP>(v1[i_], vaddr);
-        });
-        static_for<NM>([&](auto I) {
-          constexpr int i_ = I;
-          constexpr int younger = 2 * ((i_ + PD <= NM ? PD : NM - i_) - 1);
-          lds_wait2<younger>(v0[i_], v1[i_]);
-          s16x8 vv = __builtin_shufflevector(v0[i_], v1[i_], 0, 1, 2, 3, 4, 5, 6, 7);
-          oacc[i_ % DBLOCKS] = Mfma16<T>::mma(__builtin_bit_cast(vec8, vv), pf[i_ / DBLOCKS], oacc[i_ % DBLOCKS]);
-          if constexpr (i_ + PD >= NM && i_ + 1 < NM) __builtin_amdgcn_sched_barrier(0);
-          if constexpr (i_ + PD < NM) {
-            constexpr int n = i_ + PD;
-            constexpr int off = (n / DBLOCKS) * V_J_STEP + (n % DBLOCKS) * 64;
-            lds_read_tr16_b64<off>(v0[n], vaddr);
-            lds_read_tr16_b64<off + V_RD_STEP>(v1[n], vaddr);
-          }
-        });
-      }
+      vec8 pf[4];
+      M::probabilities(sacc, c, m_used * c, l_part, pf);
+      M::values(oacc, pf, vaddr);
       if (drawing && wave == 0 && lane_now() == 0) {
         const bool in_pool = draw < (unsigned)pool_len;
         drawn[i & 1] = in_pool ? seg.pool0 + (int)draw : -1;   // position i + 2

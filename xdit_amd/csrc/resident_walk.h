@@ -1,0 +1,50 @@
+// How the attention kernel that keeps the keys of a head in LDS (attn_fwd_16_resident.hip) deals out query rows: index
+// arithmetic only, plain C++ for the kernel and for a host test.
+#pragma once
+#include <stdint.h>
+
+#include "attn_walk.h"
+
+namespace xdit {
+
+// KV tiles (of 64 keys) that the kernel built for head_dim D holds: with the staging blocks of 12 wavefronts they
+// fill 159 of the 160 KiB of LDS.
+template <int D> constexpr int kResidentTiles = D == 128 ? 4 : 8;
+
+// A workgroup's work: groups [g0, g1) of 32 query rows of (batch, head) bh.
+struct ResidentPart {
+  int bh, g0, g1;
+};
+
+// Workgroup w of a launch that cuts the row groups of every (batch, head) into `parts` (at most as many as there are
+// groups) parts of equal size, give or take one.  False when there is nothing for it.
+XDIT_HD bool resident_part(int w, int tiles_per_xcd, int total, int parts, int Sq, ResidentPart& r) {
+  const int tile = xcd_tile_index(w, tiles_per_xcd);
+  if (tile >= total) return false;
+  const int64_t groups = (Sq + 31) / 32;
+  r.bh = tile / parts;
+  const int i = tile - r.bh * parts;
+  r.g0 = (int)(groups * i / parts);
+  r.g1 = (int)(groups * (i + 1) / parts);
+  return true;
+}
+
+// Parts per (batch, head): what makes the rounds of workgroups, one to a compute unit, shortest, where a
+// workgroup takes its prologue (about four KV tiles' worth: keys and queries from memory) and the groups of its
+// busiest wavefront, each `nt` tiles and about two for the rows' way in and out.
+inline int resident_parts(int64_t bh, int Sq, int nt, int wavefronts, int cus) {
+  const int64_t groups = (Sq + 31) / 32;
+  int64_t best = 1;
+  double best_cost = -1;
+  for (int64_t rounds = 1; rounds <= 6; rounds++) {
+    int64_t parts = rounds * cus / bh;
+    if (parts < 1) parts = 1;
+    if (parts > groups) parts = groups;
+    const int64_t per_wave = ((groups + parts - 1) / parts + wavefronts - 1) / wavefronts;
+    const double cost = (double)((bh * parts + cus - 1) / cus) * (4.0 + (double)per_wave * (nt + 2));
+    if (best_cost < 0 || cost < best_cost) { best = parts; best_cost = cost; }
+  }
+  return (int)best;
+}
+
+}  // namespace xdit
