@@ -1138,6 +1138,40 @@ def test_fp8_quant_bit_exact(gpu, dtype):
     assert d0.item() == 1.0 and torch.all(y0.float() == 0)
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("B,H,S,D,block", [(1, 2, 1, 64, 64), (1, 3, 37, 128, 128), (2, 2, 129, 128, 64), (1, 2, 33, 128, 32), (1, 8, 30011, 128, 128)])
+def test_fp8_quant_rotation_bytes(gpu, dtype, B, H, S, D, block):
+    """Bytes of the rotated quantiser against the butterfly in its own order (strides 1, 2, 4, ...) in fp32 torch: same
+    roundings, so no byte may differ, signs of zeros included; rows of zeros of either sign, rows that cancel, a NaN; more
+    rows than one round of workgroups takes eight of."""
+    dt = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}[dtype]
+    x = torch.randn(B, H, S, D, generator=torch.Generator().manual_seed(S)).to(dt)
+    if S > 32:
+        x[:, :, 3] = 0.0
+        x[:, :, 4] = -0.0
+        x[:, :, 5, ::2] = 0.0
+        x[:, :, 5, 1::2] = -0.0
+        x[:, :, 6:20] = x[:, :, 6:20].sign()
+        x[:, :, 20:24, : D // 2] = 0.0
+        x[:, :, 24, D // 2:] = x[:, :, 24, : D // 2]
+        x[0, 0, 30, 7] = float("nan")
+    r = x.float().reshape(B, H, S, D // block, block)
+    m = 1
+    while m < block:
+        v = r.reshape(B, H, S, D // block, block // (2 * m), 2, m)
+        r = torch.stack([v[..., 0, :] + v[..., 1, :], v[..., 0, :] - v[..., 1, :]], dim=-2).reshape(B, H, S, D // block, block)
+        m *= 2
+    entry = torch.tensor(1.0) / torch.tensor(float(block)).sqrt()
+    r = (r * entry.to(dt).float()).to(dt).float().reshape(B, H, S, D)
+    scale = r.nan_to_num(nan=0.0).abs().amax(dim=(2, 3), keepdim=True) / 448.0
+    want = (r / scale).to(torch.float8_e4m3fn)
+    y, d = ops.fp8_quant(x.to(gpu), hadamard_block=block)
+    assert torch.equal(d.cpu(), scale[:, :, 0, 0])
+    nan = r.isnan()
+    assert torch.equal(y.cpu().float().isnan(), nan)
+    assert torch.equal(y.cpu().view(torch.uint8)[~nan], want.view(torch.uint8)[~nan])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("block,D", [(128, 128), (32, 128), (8, 64), (2, 128), (64, 64), (16, 96)])
 def test_fp8_quant_with_hadamard_rotation(gpu, dtype, block, D):

@@ -25,20 +25,14 @@ namespace xdit {
 namespace quant {
 
 constexpr float kFp8Max = 448.0f;
+constexpr int kFiniteNonZero = 0x198;  // class mask: normal and subnormal numbers of either sign
 
-template <typename T> __device__ __forceinline__ void load8(const T* p, float (&x)[8]);
-template <> __device__ __forceinline__ void load8<float>(const float* p, float (&x)[8]) {
-  f32x4 a = ((const f32x4*)p)[0], b = ((const f32x4*)p)[1];
-  for (int i = 0; i < 4; i++) { x[i] = a[i]; x[4 + i] = b[i]; }
-}
-template <> __device__ __forceinline__ void load8<__bf16>(const __bf16* p, float (&x)[8]) {
-  bf16x8 v = *(const bf16x8*)p;
-  for (int i = 0; i < 8; i++) x[i] = (float)v[i];
-}
-template <> __device__ __forceinline__ void load8<_Float16>(const _Float16* p, float (&x)[8]) {
-  f16x8 v = *(const f16x8*)p;
-  for (int i = 0; i < 8; i++) x[i] = (float)v[i];
-}
+// Eight consecutive elements as they are in memory, in 16-byte loads.
+template <typename T> struct Chunk {
+  static constexpr int N = sizeof(T) / 2;
+  typedef __attribute__((ext_vector_type(8 / N))) T vec;
+  vec x[N];
+};
 
 // The value of the lane whose index differs in exactly bit log2(M) (M = 1, 2, 4 or 8), within the 16
 // lanes of a DPP row: quad permutes, the rotation by 8, and for 4 the half-row mirror (lane ^ 7)
@@ -67,36 +61,91 @@ __device__ __forceinline__ void hadamard_level(float (&v)[8], int c) {
   }
 }
 
-// Rotates the rows by the Sylvester-Hadamard matrix of size `block` along head_dim, in place in
+// The same level up to a sign that the lane keeps in `r`: own + other or own - other, one multiply-add whose DPP
+// operand is the other's value, where the form above changes the sign first (and for 4 moves twice).  Both partners of
+// a later level carry the same sign, so it passes through sums unchanged and every rounding is that of the level above
+// (one instruction per element for two: the two passes over q, k and v of Flux-1024 49.5 -> 46 us).
+// The waits at both ends are the two states between a VALU write and a DPP read of a register.
+#define XDIT_FMAC8(CTRL) \
+  asm("s_nop 1\n" \
+      "v_fmac_f32_dpp %0, %0, %8 " CTRL " row_mask:0xf bank_mask:0xf\n" \
+      "v_fmac_f32_dpp %1, %1, %8 " CTRL " row_mask:0xf bank_mask:0xf\n" \
+      "v_fmac_f32_dpp %2, %2, %8 " CTRL " row_mask:0xf bank_mask:0xf\n" \
+      "v_fmac_f32_dpp %3, %3, %8 " CTRL " row_mask:0xf bank_mask:0xf\n" \
+      "v_fmac_f32_dpp %4, %4, %8 " CTRL " row_mask:0xf bank_mask:0xf\n" \
+      "v_fmac_f32_dpp %5, %5, %8 " CTRL " row_mask:0xf bank_mask:0xf\n" \
+      "v_fmac_f32_dpp %6, %6, %8 " CTRL " row_mask:0xf bank_mask:0xf\n" \
+      "v_fmac_f32_dpp %7, %7, %8 " CTRL " row_mask:0xf bank_mask:0xf\n" \
+      "s_nop 1" \
+      : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]) : "v"(sign))
+template <int M>
+__device__ __forceinline__ void hadamard_signed_level(float (&v)[8], int c, float& r) {
+  const float sign = (c & M) != 0 ? -1.f : 1.f;
+  r *= sign;
+  if constexpr (M == 1) XDIT_FMAC8("quad_perm:[1,0,3,2]");
+  else if constexpr (M == 2) XDIT_FMAC8("quad_perm:[2,3,0,1]");
+  else if constexpr (M == 8) XDIT_FMAC8("row_ror:8");
+  else {
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = __builtin_fmaf(lane_xor<M>(v[j]), sign, v[j]);
+  }
+}
+#undef XDIT_FMAC8
+
+// Rotates the N rows by the Sylvester-Hadamard matrix of size `block` along head_dim, in place in
 // the 8-element chunks the threads hold: the three butterfly levels inside a chunk in
 // registers, the levels across chunks by exchanging with the lane that holds chunk c ^ m of the
 // same row (the chunks of a block, at most 16, sit in consecutive, block-aligned lanes of one wavefront).
 // Entries are +-r with r = `scale` rounded to T and the result is rounded to T, like the output
 // of a matmul with the matrix held in T.  `c` is the chunk's index within its row.
-template <typename T>
-__device__ __forceinline__ void hadamard_rows(float (&v)[8], int block, float scale, int c) {
-  if (block >= 2) {
+template <typename T, int N>
+__device__ __forceinline__ void hadamard_rows(float (&x)[N][8], int block, float scale, int c) {
+  float r = (float)(T)scale;
+  int plain = 1;
 #pragma unroll
-    for (int j = 0; j < 8; j += 2) { const float a = v[j], b = v[j + 1]; v[j] = a + b; v[j + 1] = a - b; }
-  }
-  if (block >= 4) {
+  for (int n = 0; n < N; n++) {
+    float (&v)[8] = x[n];
+    if (block >= 2) {
 #pragma unroll
-    for (int j = 0; j < 8; j += 4) {
-#pragma unroll
-      for (int i = 0; i < 2; i++) { const float a = v[j + i], b = v[j + i + 2]; v[j + i] = a + b; v[j + i + 2] = a - b; }
+      for (int j = 0; j < 8; j += 2) { const float a = v[j], b = v[j + 1]; v[j] = a + b; v[j + 1] = a - b; }
     }
-  }
-  if (block >= 8) {
+    if (block >= 4) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) { const float a = v[i], b = v[i + 4]; v[i] = a + b; v[i + 4] = a - b; }
-  }
-  if (block >= 16) hadamard_level<1>(v, c);
-  if (block >= 32) hadamard_level<2>(v, c);
-  if (block >= 64) hadamard_level<4>(v, c);
-  if (block >= 128) hadamard_level<8>(v, c);
-  const float r = (float)(T)scale;
+      for (int j = 0; j < 8; j += 4) {
 #pragma unroll
-  for (int j = 0; j < 8; j++) v[j] = (float)(T)(v[j] * r);
+        for (int i = 0; i < 2; i++) { const float a = v[j + i], b = v[j + i + 2]; v[j + i] = a + b; v[j + i + 2] = a - b; }
+      }
+    }
+    if (block >= 8) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) { const float a = v[i], b = v[i + 4]; v[i] = a + b; v[i + 4] = a - b; }
+    }
+    plain &= __builtin_amdgcn_classf(v[0], kFiniteNonZero);
+  }
+  // The signed form where the first element of every chunk is a finite number other than zero: that rules out rows of
+  // zeros alone, whose signs it does not keep, and infinities and NaN.
+  if (block >= 64 && __builtin_amdgcn_ballot_w64(!plain) == 0) {
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+      float rn = r;
+      hadamard_signed_level<1>(x[n], c, rn);
+      hadamard_signed_level<2>(x[n], c, rn);
+      hadamard_signed_level<4>(x[n], c, rn);
+      if (block >= 128) hadamard_signed_level<8>(x[n], c, rn);
+#pragma unroll
+      for (int j = 0; j < 8; j++) x[n][j] = (float)(T)__builtin_fmaf(x[n][j], rn, 0.f);  // a sum of zero is a positive zero
+    }
+    return;
+  }
+#pragma unroll
+  for (int n = 0; n < N; n++) {
+    if (block >= 16) hadamard_level<1>(x[n], c);
+    if (block >= 32) hadamard_level<2>(x[n], c);
+    if (block >= 64) hadamard_level<4>(x[n], c);
+    if (block >= 128) hadamard_level<8>(x[n], c);
+#pragma unroll
+    for (int j = 0; j < 8; j++) x[n][j] = (float)(T)(x[n][j] * r);
+  }
 }
 
 __global__ void fill_zero_kernel(float* p, int n) {
@@ -107,14 +156,20 @@ __global__ void fill_zero_kernel(float* p, int n) {
 // Both tensor passes: grid = (most blocks per slice, most B*H, tensors of the batch); a job's slices
 // have `blocks` workgroups, what is beyond them leaves at once.  A row of D elements is held by D/8
 // consecutive threads (8 elements each), a workgroup covers 256 / (D/8) rows per step and every
-// thread keeps kRowsInFlight rows in flight; rows advance by whole grid steps, so there is no
-// division in the loop and the trip count is the same for every thread of a workgroup (the
-// lanes of a row exchange data in the Hadamard rotation).
-constexpr int kRowsInFlight = 4;
-constexpr int kAbsmaxRowsInFlight = 8;  // the read-only pass: nothing but loads to keep in flight
+// thread works on kRowsInFlight rows while the next ones are on their way; rows advance by whole grid steps, so there is
+// no division in the loop and the trip count is the same for every thread of a workgroup (the
+// lanes of a row exchange data in the Hadamard rotation).  Two rows: the rotation is close behind the loads (about 150
+// VALU instructions per 16 bytes), so what hides it is wavefronts, six to a SIMD here.  q, k and v of Flux-1024 and of a
+// 75600 x 5 shard: 52 and 167 us with four and eight rows at once and no request ahead (five to a SIMD), 49 and 154
+// with two, 46 and 152 with the request ahead and the rule below.
+constexpr int kRowsInFlight = 2;
+// Rows per thread: eight, or as many as make all tensors of a call one round of the workgroups that fit (256 compute
+// units, six each by registers).  Fewer rows pay for the fold of the partial maxima more often (four: 54 and 180 us of the
+// calls above where eight took 49 and 154), and a second round that is not full leaves the memory idle.
+constexpr int kWorkgroups = 256 * 6;
 
 // `before` runs once per step, between a step's loads and their use.
-template <typename T, int kRowsInFlight = quant::kRowsInFlight, typename G, typename F>
+template <typename T, typename G, typename F>
 __device__ __forceinline__ void for_each_chunk(const QuantParams& p, const T* x, int64_t S, int64_t xs_s, int blocks, G&& before, F&& f) {
   const int cpr = p.D >> 3;
   const int rpb = 256 / cpr;              // rows per workgroup step
@@ -122,20 +177,30 @@ __device__ __forceinline__ void for_each_chunk(const QuantParams& p, const T* x,
   const int r = threadIdx.x / cpr;
   const bool lane_live = r < rpb;
   const int64_t step = (int64_t)blocks * rpb;
-  for (int64_t base = (int64_t)blockIdx.x * rpb; base < S; base += step * kRowsInFlight) {
-    float v[kRowsInFlight][8];
-    int64_t s[kRowsInFlight];
+  // the rows of the next step are requested before those of this one are used
+  Chunk<T> next[kRowsInFlight];
+  auto request = [&](int64_t base) {
 #pragma unroll
     for (int j = 0; j < kRowsInFlight; j++) {
-      s[j] = base + j * step + r;
-      const int64_t sc = s[j] < S ? s[j] : S - 1;  // rows past the end re-read the last row
-      load8<T>(x + sc * xs_s + c * 8, v[j]);
+      const int64_t s = base + j * step + r;
+      next[j] = *(const Chunk<T>*)(x + (s < S ? s : S - 1) * xs_s + c * 8);  // rows past the end re-read the last row
     }
+  };
+  int64_t base = (int64_t)blockIdx.x * rpb;
+  if (base < S) request(base);
+  for (; base < S; base += step * kRowsInFlight) {
+    float v[kRowsInFlight][8];
     before();
 #pragma unroll
+    for (int j = 0; j < kRowsInFlight; j++)
+#pragma unroll
+      for (int i = 0; i < 8; i++) v[j][i] = (float)next[j].x[i / (8 / Chunk<T>::N)][i % (8 / Chunk<T>::N)];
+    if (base + step * kRowsInFlight < S) request(base + step * kRowsInFlight);
+    if (p.had_block > 1) hadamard_rows<T>(v, p.had_block, p.had_scale, c);
+#pragma unroll
     for (int j = 0; j < kRowsInFlight; j++) {
-      if (p.had_block > 1) hadamard_rows<T>(v[j], p.had_block, p.had_scale, c);
-      f(v[j], s[j], c, lane_live && s[j] < S);
+      const int64_t s = base + j * step + r;
+      f(v[j], s, c, lane_live && s < S);
     }
   }
 }
@@ -167,8 +232,8 @@ __global__ __launch_bounds__(256) void absmax_kernel(const QuantBatch batch) {
       for (int j = 0; j < 8; j++) m = fmaxf(m, fabsf(v[j]));  // fmaxf drops NaN operands
     }
   };
-  for_each_chunk<T, kAbsmaxRowsInFlight>(p, (const T*)p.x + b * p.xs_b + h * p.xs_h, p.S, p.xs_s, p.reduce_blocks, [] {}, take);
-  if (p.S2 > 0) for_each_chunk<T, kAbsmaxRowsInFlight>(p, (const T*)p.x2 + b * p.x2s_b + h * p.x2s_h, p.S2, p.x2s_s, p.reduce_blocks, [] {}, take);
+  for_each_chunk<T>(p, (const T*)p.x + b * p.xs_b + h * p.xs_h, p.S, p.xs_s, p.reduce_blocks, [] {}, take);
+  if (p.S2 > 0) for_each_chunk<T>(p, (const T*)p.x2 + b * p.x2s_b + h * p.x2s_h, p.S2, p.x2s_s, p.reduce_blocks, [] {}, take);
   m = block_max(m);
   if (threadIdx.x == 0) {
     if (p.partials != nullptr) p.partials[(int64_t)bh * p.reduce_blocks + blockIdx.x] = m;
@@ -188,7 +253,6 @@ __global__ __launch_bounds__(256) void absmax_kernel(const QuantBatch batch) {
 // division's in 4 * 10^9 random cases as well.)  The bounds need the remainder's and the reciprocal's exponents in range:
 // scales outside [2^-80, 2^80] take the division itself, and where q is a zero, an infinity or a NaN it
 // is the quotient already (the remainder would cost a negative zero its sign and make an infinity a NaN).
-constexpr int kFiniteNonZero = 0x198;  // class mask: normal and subnormal numbers of either sign
 struct Divider {
   float scale, r;
   bool plain;
@@ -270,28 +334,34 @@ __global__ void finalize_kernel(const QuantParams p, int n) {
 template <typename T>
 static hipError_t run(QuantBatch& batch, hipStream_t stream) {
   int cast_x = 1, reduce_x = 0, bh_max = 1;
+  int64_t groups = 0;  // workgroup steps of one row per thread
+  for (int i = 0; i < batch.n; i++) {
+    const int rpb = 256 / (batch.job[i].D >> 3);
+    groups += (int64_t)batch.job[i].B * batch.job[i].H * (((int64_t)batch.job[i].S + batch.job[i].S2 + rpb - 1) / rpb);
+  }
+  const int64_t fit = (groups + kWorkgroups - 1) / kWorkgroups, per_thread = fit < 8 ? 8 : fit;
   for (int i = 0; i < batch.n; i++) {
     QuantParams& p = batch.job[i];
     const int BH = p.B * p.H;
     const int rpb = 256 / (p.D >> 3);
     const int64_t rows = (int64_t)p.S + p.S2;
-    int per_slice = (int)((rows + rpb * 2 * quant::kRowsInFlight - 1) / (rpb * 2 * quant::kRowsInFlight));  // ~8 rows per thread
+    int64_t per_slice = (rows + rpb * per_thread - 1) / (rpb * per_thread);
     if (per_slice < 1) per_slice = 1;
     if (per_slice > 2048) per_slice = 2048;
-    p.cast_blocks = per_slice;
+    p.cast_blocks = (int)per_slice;
     p.reduce_blocks = 0;
     if (p.scale_in == nullptr) {
       if (p.partials != nullptr) {
         // one slot per workgroup: as many workgroups as the scratch holds slots for
         p.reduce_blocks = (int)(p.partial_slots / BH);
-        if (p.reduce_blocks > per_slice) p.reduce_blocks = per_slice;
+        if (p.reduce_blocks > per_slice) p.reduce_blocks = (int)per_slice;
         if (p.reduce_blocks < 1) return hipErrorInvalidValue;
       } else {
         // every workgroup ends in one atomic max on its slice's entry: keep their number near 1024,
         // same-address atomics are served one at a time
         p.reduce_blocks = 1024 / BH;
         if (p.reduce_blocks < 1) p.reduce_blocks = 1;
-        if (p.reduce_blocks > per_slice) p.reduce_blocks = per_slice;
+        if (p.reduce_blocks > per_slice) p.reduce_blocks = (int)per_slice;
         hipLaunchKernelGGL(fill_zero_kernel, dim3((BH + 255) / 256), dim3(256), 0, stream, p.amax, BH);
       }
     }
