@@ -92,6 +92,18 @@ __device__ __forceinline__ void hadamard_signed_level(float (&v)[8], int c, floa
 }
 #undef XDIT_FMAC8
 
+// x r rounded to T.  fp16: one rounding of the exact product, zeros positive (the mixed multiply-add, named
+// here because the compiler takes it or a rounded fp32 product and a conversion by the code around).
+template <typename T, bool SIGNED_ZERO = false>
+__device__ __forceinline__ float rounded_product(float x, float r) {
+  if constexpr (sizeof(T) == 2 && !__is_same(T, __bf16)) {
+    unsigned y;
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(y) : "v"(x), "v"(r));
+    return (float)__builtin_bit_cast(_Float16, (unsigned short)y);
+  }
+  return (float)(T)(SIGNED_ZERO ? x * r : __builtin_fmaf(x, r, 0.f));  // a sum of zero is a positive zero
+}
+
 // Rotates the N rows by the Sylvester-Hadamard matrix of size `block` along head_dim, in place in
 // the 8-element chunks the threads hold: the three butterfly levels inside a chunk in
 // registers, the levels across chunks by exchanging with the lane that holds chunk c ^ m of the
@@ -133,7 +145,7 @@ __device__ __forceinline__ void hadamard_rows(float (&x)[N][8], int block, float
       hadamard_signed_level<4>(x[n], c, rn);
       if (block >= 128) hadamard_signed_level<8>(x[n], c, rn);
 #pragma unroll
-      for (int j = 0; j < 8; j++) x[n][j] = (float)(T)__builtin_fmaf(x[n][j], rn, 0.f);  // a sum of zero is a positive zero
+      for (int j = 0; j < 8; j++) x[n][j] = rounded_product<T>(x[n][j], rn);
     }
     return;
   }
@@ -144,7 +156,7 @@ __device__ __forceinline__ void hadamard_rows(float (&x)[N][8], int block, float
     if (block >= 64) hadamard_level<4>(x[n], c);
     if (block >= 128) hadamard_level<8>(x[n], c);
 #pragma unroll
-    for (int j = 0; j < 8; j++) x[n][j] = (float)(T)(x[n][j] * r);
+    for (int j = 0; j < 8; j++) x[n][j] = rounded_product<T, true>(x[n][j], r);
   }
 }
 
