@@ -1142,7 +1142,8 @@ def test_fp8_quant_bit_exact(gpu, dtype):
 @pytest.mark.parametrize("B,H,S,D,block", [(1, 2, 1, 64, 64), (1, 3, 37, 128, 128), (2, 2, 129, 128, 64), (1, 2, 33, 128, 32), (1, 8, 30011, 128, 128)])
 def test_fp8_quant_rotation_bytes(gpu, dtype, B, H, S, D, block):
     """Bytes of the rotated quantiser against the butterfly in its own order (strides 1, 2, 4, ...) in fp32 torch: same
-    roundings, so no byte may differ, signs of zeros included; rows of zeros of either sign, rows that cancel, a NaN; more
+    roundings, so no byte may differ, signs of zeros included; rows of zeros of either sign, rows that cancel, a NaN, rows whose
+    negative zeros stand beside chunk sums other than zero (alone in their wavefronts and among others); more
     rows than one round of workgroups takes eight of."""
     dt = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}[dtype]
     x = torch.randn(B, H, S, D, generator=torch.Generator().manual_seed(S)).to(dt)
@@ -1155,6 +1156,8 @@ def test_fp8_quant_rotation_bytes(gpu, dtype, B, H, S, D, block):
         x[:, :, 20:24, : D // 2] = 0.0
         x[:, :, 24, D // 2:] = x[:, :, 24, : D // 2]
         x[0, 0, 30, 7] = float("nan")
+        for first, pattern in ((25, [-0.0, 0.0, -0.0, 0.0, 1.0, 1.0, 1.0, 1.0]), (32, [-0.0, 0.0, -0.0, 0.0, 1.0, 1.0, 1.0, 1.0]), (48, [-0.0, -0.0, 1.0, -1.0, 3.0, 0.0, 3.0, 0.0])):
+            x[:, :, first:first + (1 if first == 25 else 16)] = torch.tensor(pattern).repeat(D // 8).to(dt)
     r = x.float().reshape(B, H, S, D // block, block)
     m = 1
     while m < block:

@@ -26,6 +26,7 @@ namespace quant {
 
 constexpr float kFp8Max = 448.0f;
 constexpr int kFiniteNonZero = 0x198;  // class mask: normal and subnormal numbers of either sign
+constexpr int kFinite = 0x1f8;         // ... and zeros
 
 // Eight consecutive elements as they are in memory, in 16-byte loads.
 template <typename T> struct Chunk {
@@ -113,7 +114,7 @@ __device__ __forceinline__ float rounded_product(float x, float r) {
 template <typename T, int N>
 __device__ __forceinline__ void hadamard_rows(float (&x)[N][8], int block, float scale, int c) {
   float r = (float)(T)scale;
-  int plain = 1;
+  int plain = 1, least = 0;
 #pragma unroll
   for (int n = 0; n < N; n++) {
     float (&v)[8] = x[n];
@@ -132,11 +133,14 @@ __device__ __forceinline__ void hadamard_rows(float (&x)[N][8], int block, float
 #pragma unroll
       for (int i = 0; i < 4; i++) { const float a = v[i], b = v[i + 4]; v[i] = a + b; v[i + 4] = a - b; }
     }
-    plain &= __builtin_amdgcn_classf(v[0], kFiniteNonZero);
+    plain &= __builtin_amdgcn_classf(v[0], kFinite);
+#pragma unroll
+    for (int j = 0; j < 8; j++) least = min(least, __float_as_int(v[j]));
   }
-  // The signed form where the first element of every chunk is a finite number other than zero: that rules out rows of
-  // zeros alone, whose signs it does not keep, and infinities and NaN.
-  if (block >= 64 && __builtin_amdgcn_ballot_w64(!plain) == 0) {
+  // The signed form where a chunk holds no infinity or NaN (its first element is the sum of all) and, from here on, no negative
+  // zero, whose bits are the least integer: the signed form ends in positive zeros only, and so does the other one
+  // then, as its sums are negative zeros only where both terms are.
+  if (block >= 64 && __builtin_amdgcn_ballot_w64(!plain || least == (int)0x80000000) == 0) {
 #pragma unroll
     for (int n = 0; n < N; n++) {
       float rn = r;
