@@ -1670,6 +1670,7 @@ def test_few_keys_resident_in_lds_give_the_bits_of_the_tiled_launch(gpu, dtype, 
         out = (frame.transpose(1, 2) if bshd else frame)[..., 8:8 + D]
         got = []
         for tuning in (dict(rows_per_workgroup=128), dict(), dict(cu_count=1), dict(cu_count=9)):
+            out.fill_(float("nan"))   # a row that a launch leaves out does not keep the bytes of the one before
             ops.TUNING.update(tuning)
             try:
                 o, l = ops.attn_fwd(q, k, v, k2=k2, v2=v2, q2=q2, out=out)
