@@ -188,12 +188,11 @@ int xdit_attn_fwd_noalloc(const xdit_attn_args* args);
  * rows with `kv_iterations` tiles of 32 keys, or, when those would leave more than a quarter of
  * the compute units without a workgroup, of 64 rows with tiles of 64 keys.  No counterpart in the
  * reference.
- * A plain 16-bit forward over few keys (xdit_attn_fwd at most four tiles of 64 keys at head_dim above 64, eight below, both
- * segments together) with rows_per_workgroup and balance left at 0 runs on a kernel that holds the keys in LDS and deals
- * out its rows otherwise; it gives the bits of the launch described here.
+ * A 16-bit forward over few keys can run on another kernel instead (resident_parts > 0): the other fields then still
+ * describe the launch it takes the place of.
  */
 typedef struct {
-  uint32_t struct_size;        /* = sizeof(xdit_launch_plan), set by the caller */
+  uint32_t struct_size;        /* = sizeof(xdit_launch_plan), set by the caller (or its size without resident_parts) */
   int32_t rows_per_workgroup;
   int32_t query_tiles;
   int32_t kv_iterations;
@@ -220,6 +219,11 @@ typedef struct {
                                   fold the shared tiles at their ends, a slice of rows each */
   int32_t ring_step;           /* INPUT, set by the caller like struct_size: != 0 plans the launch of
                                   xdit_attn_fwd_accumulate for these arguments, 0 that of xdit_attn_fwd */
+  int32_t resident_parts;      /* > 0: the call runs on the kernel that holds the keys of a (batch, head) in LDS (16-bit, at most
+                                  four tiles of 64 keys at head_dim above 64, eight up to 64, both segments together;
+                                  rows_per_workgroup and balance 0): the query rows of every (batch, head) are cut into
+                                  this many parts, a workgroup each.  The result has the bits of a plain launch */
+  int32_t reserved0;           /* 0 */
 } xdit_launch_plan;
 
 int xdit_attn_launch_plan(const xdit_attn_args* args, xdit_launch_plan* plan);

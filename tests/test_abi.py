@@ -341,6 +341,24 @@ def test_launch_plan_of_the_named_shapes():
     assert _lib.lib().xdit_attn_launch_plan(ctypes.byref(a), ctypes.byref(p)) == _lib.XDIT_ERR_UNSUPPORTED
 
 
+def test_launch_plan_names_the_kernel_of_few_keys():
+    """A 16-bit forward over few keys runs on the kernel that keeps them in LDS: the plan says so and into how many parts it cuts
+    the rows; the ring step, long key ranges, fp8 and launches that the caller shapes do not.  A caller with the
+    structure as it was without that field still gets its plan, and nothing behind it is written."""
+    cross = _plan(2, 16, 4096, 120, D=72, cus=256)
+    assert 1 < cross.resident_parts <= 128
+    assert _plan(1, 24, 40000, 190, Sk2=56, cus=256).resident_parts == 10
+    for other in (_plan(2, 16, 4096, 120, D=72, cus=256, ring_step=True), _plan(2, 16, 4096, 120, D=72, cus=256, rows=128),
+                  _plan(2, 16, 4096, 120, D=72, cus=256, balance=1), _plan(1, 24, 40000, 257, cus=256), _plan(1, 24, 40000, 250, Sk2=10, cus=256),
+                  _plan(1, 24, 40000, 200, dtype=_lib.DTYPE_FP8_E4M3FN, cus=256)):
+        assert other.resident_parts == 0
+    a = _attn_args(B=2, H=16, Sq=4096, Sk=120, D=72, cu_count=256)
+    p = _lib.LaunchPlan()
+    p.struct_size, p.resident_parts = _lib.LaunchPlan.resident_parts.offset, 12345
+    assert _lib.lib().xdit_attn_launch_plan(ctypes.byref(a), ctypes.byref(p)) == 0
+    assert p.resident_parts == 12345 and p.query_tiles == cross.query_tiles
+
+
 def test_launch_choice_against_measured_option_times():
     """The library's choice of launch (query rows per workgroup, balanced or not) held to
     measurements: tests/golden/launch_option_times.json records the settled time of every launch

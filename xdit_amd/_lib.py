@@ -122,6 +122,8 @@ class LaunchPlan(ctypes.Structure):
         ("fold_in_kernel", ctypes.c_int32),
         ("parts_first", ctypes.c_int32),
         ("ring_step", ctypes.c_int32),
+        ("resident_parts", ctypes.c_int32),
+        ("reserved0", ctypes.c_int32),
     ]
 
 

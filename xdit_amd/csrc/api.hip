@@ -4,6 +4,7 @@
 
 #include <cmath>
 #include <cstdarg>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -519,8 +520,9 @@ int xdit_attn_launch_plan(const xdit_attn_args* a, xdit_launch_plan* out) {
   if (a == nullptr || out == nullptr) return fail(XDIT_ERR_INVALID_ARG, "args or plan is NULL");
   if (a->struct_size != sizeof(xdit_attn_args))
     return fail(XDIT_ERR_INVALID_ARG, "struct_size %u != %zu (ABI mismatch)", a->struct_size, sizeof(xdit_attn_args));
-  if (out->struct_size != sizeof(xdit_launch_plan))
-    return fail(XDIT_ERR_INVALID_ARG, "plan struct_size %u != %zu (ABI mismatch)", out->struct_size, sizeof(xdit_launch_plan));
+  const uint32_t size = out->struct_size;
+  if (size != sizeof(xdit_launch_plan) && size != offsetof(xdit_launch_plan, resident_parts))
+    return fail(XDIT_ERR_INVALID_ARG, "plan struct_size %u != %zu (ABI mismatch)", size, sizeof(xdit_launch_plan));
   if (a->B <= 0 || a->H <= 0 || a->Sq <= 0 || a->Sk <= 0 || a->Sk2 < 0 || a->Sq > (int64_t(1) << 30) ||
       a->Sk > (int64_t(1) << 30) || a->Sk2 > (int64_t(1) << 30) ||
       (int64_t)a->B * a->H * ((a->Sq + 31) / 32) > (int64_t(1) << 30))
@@ -537,8 +539,7 @@ int xdit_attn_launch_plan(const xdit_attn_args* a, xdit_launch_plan* out) {
     // the fp32 kernel: one workgroup per query tile, no shared last round, no workspace
     const int rows = xdit::attn_fwd_f32_rows(p);
     const int keys = rows == 64 ? 64 : 32;
-    const uint32_t size = out->struct_size;
-    std::memset(out, 0, sizeof(*out));
+    std::memset(out, 0, size);
     out->struct_size = size;
     out->rows_per_workgroup = rows;
     out->query_tiles = (int32_t)(a->B * a->H * ((a->Sq + rows - 1) / rows));
@@ -553,8 +554,7 @@ int xdit_attn_launch_plan(const xdit_attn_args* a, xdit_launch_plan* out) {
   const int rows = choice.rows;
   p.split_policy = choice.policy;
   const size_t need = fp8 ? xdit::attn_fwd_fp8_workspace(p, a->D, rows, &q, ring_step) : xdit::attn_fwd_16_workspace(p, kernel_head_dim(a->D), rows, &q, ring_step);
-  const uint32_t size = out->struct_size;
-  std::memset(out, 0, sizeof(*out));
+  std::memset(out, 0, size);
   out->struct_size = size;
   out->ring_step = ring_step;
   out->rows_per_workgroup = rows;
@@ -573,6 +573,8 @@ int xdit_attn_launch_plan(const xdit_attn_args* a, xdit_launch_plan* out) {
   out->parts_first = q.split_order;
   if (q.split_dyn) out->range_len = q.split_s0;
   out->workgroups = (int32_t)xdit::split_grid(q);
+  if (size == sizeof(xdit_launch_plan) && !ring_step && resident_path(a))
+    out->resident_parts = xdit::resident_parts((int64_t)a->B * a->H, (int)a->Sq, out->kv_iterations, xdit::resident_wavefronts(a->D), xdit::resident_cus(a->cu_count));
   return XDIT_OK;
 }
 

@@ -237,19 +237,18 @@ static hipError_t launch_typed_resident(const AttnParams& p, int D, int nt, hipS
   const int d = p.d_actual == D ? 0 : p.d_actual;
   AttnParams q = p;
   q.d_actual = d;
-  // Twelve wavefronts where three to a SIMD leave the registers for it: computed over 80 columns they are ahead of
-  // eight with the queries requested ahead (2 x 16 heads of 4096 on 120 keys 15.5 against 16.5 us, 24 of 40000 80.7
-  // against 84), over 96 behind (24 of 40000 on 256 keys 141 against 138).
+  // Computed over 80 columns twelve wavefronts are ahead of eight with the queries requested ahead (2 x 16 heads of 4096
+  // on 120 keys 15.5 against 16.5 us, 24 of 40000 80.7 against 84), over 96 behind (24 of 40000 on 256 keys 141 against 138).
   if (D == 128) {
-    if (d == 0) return launch_resident<T, 128, 128, 8, false>(q, nt, stream);
-    if (d <= 80) return launch_resident<T, 128, 80, 12, true>(q, nt, stream);
-    if (d <= 96) return launch_resident<T, 128, 96, 8, true>(q, nt, stream);
-    if (d <= 112) return launch_resident<T, 128, 112, 8, true>(q, nt, stream);
-    return launch_resident<T, 128, 128, 8, true>(q, nt, stream);
+    if (d == 0) return launch_resident<T, 128, 128, resident_wavefronts(128), false>(q, nt, stream);
+    if (d <= 80) return launch_resident<T, 128, 80, resident_wavefronts(80), true>(q, nt, stream);
+    if (d <= 96) return launch_resident<T, 128, 96, resident_wavefronts(96), true>(q, nt, stream);
+    if (d <= 112) return launch_resident<T, 128, 112, resident_wavefronts(112), true>(q, nt, stream);
+    return launch_resident<T, 128, 128, resident_wavefronts(128), true>(q, nt, stream);
   }
-  if (d == 0) return launch_resident<T, 64, 64, 12, false>(q, nt, stream);
-  if (d <= 32) return launch_resident<T, 64, 32, 12, true>(q, nt, stream);
-  return launch_resident<T, 64, 64, 12, true>(q, nt, stream);
+  if (d == 0) return launch_resident<T, 64, 64, resident_wavefronts(64), false>(q, nt, stream);
+  if (d <= 32) return launch_resident<T, 64, 32, resident_wavefronts(32), true>(q, nt, stream);
+  return launch_resident<T, 64, 64, resident_wavefronts(64), true>(q, nt, stream);
 }
 
 hipError_t launch_attn_fwd_16_resident(const AttnParams& p, int dtype_is_fp16, int D, hipStream_t stream) {

@@ -314,8 +314,9 @@ def attn_fwd(q, k, v, softmax_scale=None, causal=False, k2=None, v2=None,
 def launch_plan(q, k, k2=None, streamed=None, ring_step=False):
     """How `attn_fwd(q, k, v, k2=..)` would be launched (a dict of the fields of xdit_launch_plan):
     rows per workgroup, query tiles, whole tiles, shared ranges and their length, claimers,
-    whether ranges are handed out through the counter, workgroups, workspace bytes.  Host
-    arithmetic only; bf16 / fp16 / fp32 (head_dim up to 128) and fp8 (head_dim 128 or 64)."""
+    whether ranges are handed out through the counter, workgroups, workspace bytes; with
+    `resident_parts` > 0 the call runs on the few-keys kernel in place of that launch, the query rows of
+    every (batch, head) cut into that many parts.  Host arithmetic only; bf16 / fp16 / fp32 (head_dim up to 128) and fp8 (head_dim 128 or 64)."""
     a = _lib.AttnArgs()
     a.struct_size = ctypes.sizeof(_lib.AttnArgs)
     a.dtype = _code(q.dtype)
