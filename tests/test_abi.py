@@ -383,6 +383,24 @@ def test_launch_choice_against_measured_option_times():
         assert len(xs) > 40 and sum(xs) / len(xs) <= 0.03, (dtype, sum(xs) / len(xs))
 
 
+def test_choice_of_the_few_keys_kernel_against_measured_times():
+    """Which of the two kernels a 16-bit call over few keys runs on, held to the recorded times of both: where the kernel that
+    keeps the keys in LDS is taken it is at most 10 % slower than the tiled launch, and over all problems the choice is at
+    most 1 % slower than the faster kernel.  Launches of more threads than fit in 2^32 stay on the tiled kernel."""
+    import json
+    data = json.load(open(os.path.join(ROOT, "tests", "golden", "few_keys_times.json")))
+    assert len(data["problems"]) > 350
+    excess, taken = [], 0
+    for B, H, Sq, Sk, D, tiled, resident in data["problems"]:
+        p = _plan(B, H, Sq, Sk, D=D, cus=data["cu_count"])
+        if p.resident_parts:
+            taken += 1
+            assert resident <= 1.10 * tiled, (B, H, Sq, Sk, D, tiled, resident)
+        excess.append((resident if p.resident_parts else tiled) / min(tiled, resident) - 1.0)
+    assert taken > 70 and sum(excess) / len(excess) <= 0.01, (taken, sum(excess) / len(excess))
+    assert _plan(1 << 18, 16, 1200, 100, D=72, cus=256).resident_parts == 1 and _plan(1 << 19, 16, 1200, 100, D=72, cus=256).resident_parts == 0
+
+
 WALK_HARNESS = r"""
 // Walks every workgroup of a planned launch with the code the kernels run (attn_walk.h) and
 // checks the coverage: stdin holds one launch per line.

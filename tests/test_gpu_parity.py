@@ -1647,10 +1647,13 @@ def test_plain_launch_of_fewer_workgroups_than_tiles(gpu, force_rows, dtype, D, 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("D,Sq,Sq2,Sk,Sk2", [(128, 1, 0, 1, 0), (128, 777, 0, 256, 0), (128, 300, 85, 100, 120), (128, 33, 0, 65, 128), (120, 97, 0, 190, 0),
                                              (104, 400, 0, 64, 0), (96, 500, 31, 129, 60), (88, 1000, 0, 77, 0), (80, 65, 0, 256, 0), (72, 2000, 0, 120, 0),
-                                             (64, 513, 0, 512, 0), (64, 31, 17, 300, 200), (56, 200, 0, 450, 0), (32, 100, 0, 77, 0), (8, 70, 0, 9, 0)])
+                                             (64, 513, 0, 512, 0), (64, 31, 17, 300, 200), (56, 200, 0, 450, 0), (32, 100, 0, 77, 0), (8, 70, 0, 9, 0),
+                                             (128, 1300, 0, 250, 0), (128, 1100, 201, 100, 120), (128, 2010, 0, 60, 0), (120, 1234, 0, 190, 0), (112, 1500, 0, 130, 0),
+                                             (104, 1111, 0, 64, 0), (96, 1500, 31, 129, 60), (88, 1777, 0, 256, 0), (80, 999, 0, 256, 0), (64, 600, 0, 100, 0),
+                                             (64, 2001, 0, 500, 0), (64, 601, 17, 70, 50), (56, 1200, 0, 450, 0), (32, 3000, 0, 77, 0), (8, 1500, 0, 9, 0)])
 def test_few_keys_resident_in_lds_give_the_bits_of_the_tiled_launch(gpu, dtype, D, Sq, Sq2, Sk, Sk2):
     """The kernel that keeps a head's keys in LDS, planned for few and for all compute units (one to many row groups
-    a wavefront), against the tiled kernel (forced by its rows per workgroup): the same bits, in both memory orders, with
+    a wavefront; with every number of them at which it is taken), against the tiled kernel (forced by its rows per workgroup): the same bits, in both memory orders, with
     the tensors framed in NaN columns, and next to the oracle."""
     g = torch.Generator().manual_seed(D + Sq + Sk)
     B, H = 2, 3
@@ -1664,12 +1667,22 @@ def test_few_keys_resident_in_lds_give_the_bits_of_the_tiled_launch(gpu, dtype, 
         view = (frame.transpose(1, 2) if bshd else frame)[..., 8:8 + D]
         view.copy_(x)
         return view
+    def parts(tuning):
+        meta = [torch.empty(B, H, s, D, dtype=dtype, device="meta") for s in (Sq + Sq2, Sk, Sk2)]
+        ops.TUNING.update(tuning)
+        try:
+            return ops.launch_plan(*meta)["resident_parts"]
+        finally:
+            ops.TUNING.update(rows_per_workgroup=0, cu_count=0)
+    tunings = [dict(rows_per_workgroup=128), dict(), dict(cu_count=1), dict(cu_count=9)]
+    tunings += [t for t in (dict(cu_count=c) for c in (2, 3, 4, 6, 12, 20, 40)) if parts(t)]
+    assert parts(tunings[0]) == 0 and (Sq < 600 or any(parts(t) for t in tunings))
     for bshd in (False, True):
         q, q2, k, v, k2, v2 = mk(Sq, bshd), mk(Sq2, bshd), mk(Sk, bshd), mk(Sk, bshd), mk(Sk2, bshd), mk(Sk2, bshd)
         frame = torch.zeros((B, Sq + Sq2, H, D + 16) if bshd else (B, H, Sq + Sq2, D + 16), dtype=dtype, device=gpu)
         out = (frame.transpose(1, 2) if bshd else frame)[..., 8:8 + D]
         got = []
-        for tuning in (dict(rows_per_workgroup=128), dict(), dict(cu_count=1), dict(cu_count=9)):
+        for tuning in tunings:
             out.fill_(float("nan"))   # a row that a launch leaves out does not keep the bytes of the one before
             ops.TUNING.update(tuning)
             try:

@@ -94,10 +94,11 @@ bool mfma16_path(const xdit_attn_args* a) {
 struct LaunchChoice {
   int rows;    // query rows per workgroup
   int policy;  // AttnParams::split_policy: 1 plain launch, 2 balanced when the planner offers a plan
+  double us;   // its estimated time
 };
 
 LaunchChoice choose_launch(const xdit_attn_args* a, bool plain = false, bool fold_only = false) {
-  LaunchChoice best = {128, 1};
+  LaunchChoice best = {128, 1, 0.0};
   const int D = kernel_head_dim(a->D);
   if (D == 0) return best;
   const bool fp8 = a->dtype == XDIT_DTYPE_FP8_E4M3FN;
@@ -168,15 +169,22 @@ LaunchChoice choose_launch(const xdit_attn_args* a, bool plain = false, bool fol
       if (best_cost < 0 || cost < best_cost) { best.rows = rows; best.policy = policy; best_cost = cost; }
     }
   }
+  best.us = best_cost;
   return best;
 }
 
-// Whether a 16-bit forward runs on the kernel that keeps the keys of a head in LDS: where they fit, unless the
+// Whether a 16-bit forward runs on the kernel that keeps the keys of a head in LDS instead of the tiled launch chosen for
+// it: where they fit, that launch would be a plain one (whose bits this kernel gives) and its estimated time is longer, unless the
 // caller asks for a shape or a balance of the tiled launch.
-bool resident_path(const xdit_attn_args* a) {
+// Of 14405 problems (B*H 1..32768, 16..100000 rows, 1..256 keys, 512 up to head_dim 64, head_dims 32..128, both memory orders) it
+// was more than 2 % slower in 7583 when every call over few keys took it, and is in 122 now; the choice is 0.3 % slower than the faster
+// of the two on average.  us, tiled and this kernel (bf16): 12 heads of 8192 on 226 keys at head_dim 128 22.6 and 24.5, 512 of 64 on 64
+// at 96 6.6 and 10.7, 3 of 1349 on 120 at 128 7.7 and 8.2, all tiled now; 48 of 32760 on 77 at 128 220 and 185.
+bool resident_path(const xdit_attn_args* a, const LaunchChoice& tiled) {
   const int D = kernel_head_dim(a->D);
   const int64_t nt = (a->Sk + xdit::kKeysPerTile - 1) / xdit::kKeysPerTile + (a->Sk2 + xdit::kKeysPerTile - 1) / xdit::kKeysPerTile;
-  return mfma16_path(a) && a->rows_per_workgroup == 0 && a->balance == 0 && nt <= (D == 128 ? xdit::kResidentTiles<128> : xdit::kResidentTiles<64>);
+  if (!mfma16_path(a) || tiled.policy != 1 || a->rows_per_workgroup != 0 || a->balance != 0 || nt > (D == 128 ? xdit::kResidentTiles<128> : xdit::kResidentTiles<64>)) return false;
+  return xdit::resident_us((int64_t)a->B * a->H, (int)a->Sq, (int)nt, a->D, xdit::resident_cus(a->cu_count), tiled.rows) < tiled.us;
 }
 
 // The two tuning fields of xdit_attn_args.
@@ -410,16 +418,14 @@ static int attn_fwd_impl(const xdit_attn_args* a, const xdit_ring_acc* acc, cons
   // launch follows: the next call on it may then say "preserved" whether this one is balanced or not.
   if (p.ws_out != nullptr && !p.ws_preserved) xdit::launch_counter_reset(p.ws_out, stream);
   hipError_t e;
-  if (acc == nullptr && resident_path(a)) {
-    p.d_actual = a->D;
-    e = xdit::launch_attn_fwd_16_resident(p, a->dtype == XDIT_DTYPE_FP16, kernel_head_dim(a->D), stream);
-  } else if (fp8 || mfma16_path(a)) {
+  if (fp8 || mfma16_path(a)) {
     const int D = fp8 ? a->D : kernel_head_dim(a->D);
     if (!fp8) p.d_actual = a->D;
     const bool fused = acc != nullptr;
     LaunchChoice c = choose_launch(a, p.ws_out == nullptr, fused);  // no workspace: the shape that suits a plain launch
+    const bool resident = !fused && resident_path(a, c);
     p.split_policy = c.policy;
-    if (c.policy == 2) {
+    if (!resident && c.policy == 2) {
       // a workspace too small for the chosen balanced plan: the best PLAIN launch, not that shape run plain
       xdit::AttnParams plan;
       const size_t need = fp8 ? xdit::attn_fwd_fp8_workspace(p, D, c.rows, &plan, fused) : xdit::attn_fwd_16_workspace(p, D, c.rows, &plan, fused);
@@ -428,7 +434,8 @@ static int attn_fwd_impl(const xdit_attn_args* a, const xdit_ring_acc* acc, cons
         p.split_policy = c.policy;
       }
     }
-    if (fp8) e = xdit::launch_attn_fwd_fp8(p, D, out_dtype == XDIT_DTYPE_FP16, c.rows, stream);
+    if (resident) e = xdit::launch_attn_fwd_16_resident(p, a->dtype == XDIT_DTYPE_FP16, D, stream);
+    else if (fp8) e = xdit::launch_attn_fwd_fp8(p, D, out_dtype == XDIT_DTYPE_FP16, c.rows, stream);
     else e = fused ? xdit::launch_attn_fwd_16_ring(p, a->dtype == XDIT_DTYPE_FP16, D, c.rows, stream)
                    : xdit::launch_attn_fwd_16(p, a->dtype == XDIT_DTYPE_FP16, D, c.rows, stream);
   } else {
@@ -573,7 +580,7 @@ int xdit_attn_launch_plan(const xdit_attn_args* a, xdit_launch_plan* out) {
   out->parts_first = q.split_order;
   if (q.split_dyn) out->range_len = q.split_s0;
   out->workgroups = (int32_t)xdit::split_grid(q);
-  if (size == sizeof(xdit_launch_plan) && !ring_step && resident_path(a))
+  if (size == sizeof(xdit_launch_plan) && !ring_step && resident_path(a, choice))
     out->resident_parts = xdit::resident_parts((int64_t)a->B * a->H, (int)a->Sq, out->kv_iterations, xdit::resident_wavefronts(a->D), xdit::resident_cus(a->cu_count));
   return XDIT_OK;
 }

@@ -52,4 +52,25 @@ inline int resident_parts(int64_t bh, int Sq, int nt, int wavefronts, int cus) {
   return (int)best;
 }
 
+// Estimated us of that launch, on the scale of choose_launch's estimate for the tiled launch of `tiled_rows` rows per workgroup that it
+// would take the place of: rounds of workgroups, each a prologue and the average, not the busiest, number of row groups of
+// its wavefronts, which share the compute unit.  Keys pay for their way into LDS only where enough groups meet them there: with
+// a group or less per wavefront all of them have to land before the first product.
+// The rates are the lowest at which at most 8 in 1000 problems were sent here that were more than 4 % slower for it (14000 of them, see
+// resident_path).  Against tiled launches of 256 and 384 rows they are lower, as these show their prologue and
+// epilogue in full, and lowest where rows are no whole half lines of 128 bytes, whose streaming stores cost those launches most.
+inline double resident_us(int64_t bh, int Sq, int nt, int head_dim, int cus, int tiled_rows) {
+  const int nw = resident_wavefronts(head_dim);
+  const double never = 1e30;
+  if (bh > (int64_t)0xffffffff / (64 * nw) - 8) return never;  // a launch holds at most 2^32 threads
+  const int parts = resident_parts(bh, Sq, nt, nw, cus);
+  const double rounds = (double)((bh * parts + cus - 1) / cus);
+  const double per_wave = (double)((Sq + 31) / 32) / parts / nw;
+  const bool many_rows = tiled_rows > 128;
+  if (head_dim == 64) return many_rows ? 1.06 * rounds * (1.5 + per_wave) * (nt + 2) - 6.0 : never;
+  if (head_dim < 64) return rounds * (1.5 + per_wave) * (many_rows ? (head_dim > 32 ? 0.65 : 0.75) * (nt + 4) : 1.03 * (nt + 2)) - 4.0;
+  const double rate = many_rows ? (head_dim % 32 == 0 ? 1.9 : 1.35) : head_dim <= 80 ? 1.6 : head_dim <= 104 || head_dim == 128 ? 1.65 : head_dim <= 112 ? 1.87 : 1.57;
+  return rate * rounds * (8.0 + (0.5 + per_wave) * nt) - 4.0;
+}
+
 }  // namespace xdit
