@@ -175,14 +175,14 @@ __global__ void fill_zero_kernel(float* p, int n) {
 // thread works on kRowsInFlight rows while the next ones are on their way; rows advance by whole grid steps, so there is
 // no division in the loop and the trip count is the same for every thread of a workgroup (the
 // lanes of a row exchange data in the Hadamard rotation).  Two rows: the rotation is close behind the loads (about 150
-// VALU instructions per 16 bytes), so what hides it is wavefronts, six to a SIMD here.  q, k and v of Flux-1024 and of a
-// 75600 x 5 shard: 52 and 167 us with four and eight rows at once and no request ahead (five to a SIMD), 49 and 154
-// with two, 46 and 152 with the request ahead and the rule below.
+// VALU instructions per 16 bytes), so what hides it is wavefronts, five to seven to a SIMD by registers.
+// q, k and v of Flux-1024 and of a 75600 x 5 shard: 45.9 and 161 us with four rows (eight in the abs-max) at once and no request
+// ahead, at four to five wavefronts, 40.5 and 144 now; three or four rows a step of the abs-max are no faster at the rule below.
 constexpr int kRowsInFlight = 2;
-// Rows per thread: eight, or as many as make all tensors of a call one round of the workgroups that fit (256 compute
-// units, six each by registers).  Fewer rows pay for the fold of the partial maxima more often (four: 54 and 180 us of the
-// calls above where eight took 49 and 154), and a second round that is not full leaves the memory idle.
-constexpr int kWorkgroups = 256 * 6;
+// Rows per thread.  As many as make all tensors of a call one round of the workgroups that fit at once leave the memory to a
+// few of them at the end: cast of q, k and v of 40 heads of 32760 345 us where eight rows take 273, 2 x 48 of 17776 at head_dim 64
+// 220 and 181, 24 of 16384 104 and 88, 5 of 75600 91 and 83, 24 of 4608 23.5 and 24.2; 16 rows take 284, 190, 94, 85 and 25.3.
+constexpr int kRowsPerThread = 8;
 
 // `before` runs once per step, between a step's loads and their use.
 template <typename T, typename G, typename F>
@@ -350,34 +350,28 @@ __global__ void finalize_kernel(const QuantParams p, int n) {
 template <typename T>
 static hipError_t run(QuantBatch& batch, hipStream_t stream) {
   int cast_x = 1, reduce_x = 0, bh_max = 1;
-  int64_t groups = 0;  // workgroup steps of one row per thread
-  for (int i = 0; i < batch.n; i++) {
-    const int rpb = 256 / (batch.job[i].D >> 3);
-    groups += (int64_t)batch.job[i].B * batch.job[i].H * (((int64_t)batch.job[i].S + batch.job[i].S2 + rpb - 1) / rpb);
-  }
-  const int64_t fit = (groups + kWorkgroups - 1) / kWorkgroups, per_thread = fit < 8 ? 8 : fit;
   for (int i = 0; i < batch.n; i++) {
     QuantParams& p = batch.job[i];
     const int BH = p.B * p.H;
     const int rpb = 256 / (p.D >> 3);
     const int64_t rows = (int64_t)p.S + p.S2;
-    int64_t per_slice = (rows + rpb * per_thread - 1) / (rpb * per_thread);
+    int per_slice = (int)((rows + rpb * kRowsPerThread - 1) / (rpb * kRowsPerThread));
     if (per_slice < 1) per_slice = 1;
     if (per_slice > 2048) per_slice = 2048;
-    p.cast_blocks = (int)per_slice;
+    p.cast_blocks = per_slice;
     p.reduce_blocks = 0;
     if (p.scale_in == nullptr) {
       if (p.partials != nullptr) {
         // one slot per workgroup: as many workgroups as the scratch holds slots for
         p.reduce_blocks = (int)(p.partial_slots / BH);
-        if (p.reduce_blocks > per_slice) p.reduce_blocks = (int)per_slice;
+        if (p.reduce_blocks > per_slice) p.reduce_blocks = per_slice;
         if (p.reduce_blocks < 1) return hipErrorInvalidValue;
       } else {
         // every workgroup ends in one atomic max on its slice's entry: keep their number near 1024,
         // same-address atomics are served one at a time
         p.reduce_blocks = 1024 / BH;
         if (p.reduce_blocks < 1) p.reduce_blocks = 1;
-        if (p.reduce_blocks > per_slice) p.reduce_blocks = (int)per_slice;
+        if (p.reduce_blocks > per_slice) p.reduce_blocks = per_slice;
         hipLaunchKernelGGL(fill_zero_kernel, dim3((BH + 255) / 256), dim3(256), 0, stream, p.amax, BH);
       }
     }
