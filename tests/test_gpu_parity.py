@@ -1697,6 +1697,42 @@ def test_few_keys_resident_in_lds_give_the_bits_of_the_tiled_launch(gpu, dtype, 
     assert _err(got[1][0], ro) <= 2e-2 and _err(got[1][1], rl) <= 1e-3
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,Sk,cus", [(64, 300, 3), (72, 200, 1), (128, 200, 1)])
+@pytest.mark.parametrize("case", ["nan_then_inf", "nan_tile", "ninf_tile", "inf"])
+def test_few_keys_rows_beside_rows_that_are_not_finite(gpu, dtype, D, Sk, cus, case):
+    """A row whose logits are all NaN (or -inf) in the first KV tile and +inf in a later one makes the whole wavefront
+    rescale there, which rounds the 31 rows beside it once more: the kernel that keeps the keys in LDS does so exactly where the tiled
+    one does, so its finite rows have the same bits, and the others are NaN in both."""
+    g = torch.Generator().manual_seed(D)
+    H, S = 3, 700
+    q, k, v = (torch.randn(1, H, s, D, generator=g) for s in (S, Sk, Sk))
+    rows = torch.arange(5, S, 32)
+    k[..., 0] = k[..., 0].abs() + 0.01
+    k[:, :, 64:128] *= 1.5
+    if case == "nan_tile":
+        k[:, 1, :64, 3] = float("nan")
+    else:
+        q[:, :, rows, 0] = float("-inf" if case == "ninf_tile" else "inf")
+    if case == "nan_then_inf":
+        q[:, :, rows, 1] = float("inf")
+        k[:, :, :64, 1], k[:, :, 64:, 1] = -1.0, 1.0
+    elif case == "ninf_tile":
+        k[:, :, 64:, 0] *= -1
+    q, k, v = (x.to(dtype).to(gpu) for x in (q, k, v))
+    got = []
+    for tuning, resident in ((dict(rows_per_workgroup=128), False), (dict(cu_count=cus), True)):
+        ops.TUNING.update(tuning)
+        try:
+            assert (ops.launch_plan(q, k)["resident_parts"] > 0) == resident
+            got.append([x.cpu() for x in ops.attn_fwd(q, k, v)])
+        finally:
+            ops.TUNING.update(rows_per_workgroup=0, cu_count=0)
+    for a, b in zip(*got):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(nan=0.0), b.nan_to_num(nan=0.0))
+    assert got[0][0].isnan().any() and not got[0][0].isnan().all()
+
+
 @pytest.mark.parametrize("strategy", ["front", "rear"])
 @pytest.mark.parametrize("case", ["bf16", "fp16", "fp8", "bshd", "views"])
 def test_usp_joint_queries_are_read_where_they_are(gpu, monkeypatch, strategy, case):

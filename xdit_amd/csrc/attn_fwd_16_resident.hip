@@ -140,7 +140,7 @@ __global__ __launch_bounds__(64 * NW, NW == 12 ? 3 : 2) void attn_fwd_16_residen
       if (left < kKeysPerTile) M::mask(sacc, left);
       const float mx = M::row_max(sacc);
       if (t == 0) {
-        m_used = mx;
+        m_used = fmaxf(m_used, mx);  // -inf where all logits are NaN, as in the tiled kernel: a later tile may rescale the rows beside such a row
       } else {
         const float m_new = fmaxf(m_used, mx);
         const bool grow = (m_new - m_used) * c > kLazyRescaleLog2;
