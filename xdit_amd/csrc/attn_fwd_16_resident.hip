@@ -109,7 +109,7 @@ __global__ __launch_bounds__(64 * NW, NW == 12 ? 3 : 2) void attn_fwd_16_residen
   __syncthreads();
 
   const unsigned lds0 = (unsigned)(uintptr_t)(XDIT_LDS unsigned char*)smem;
-  unsigned kaddr0 = lds0 + M::k_read_offset(lane), vaddr0 = lds0 + M::v_read_offset(lane);
+  unsigned kaddr0 = M::k_read_address(lds0, l32, hh), vaddr0 = M::v_read_address(lds0, lane, hh);
   asm volatile("" : "+v"(kaddr0), "+v"(vaddr0));  // one register each through the loop
   XDIT_LDS unsigned char* const stage = (XDIT_LDS unsigned char*)smem + nt * G::BUF_BYTES + wave * kResidentStageBytes;
   const float c = p.scale * kLog2e;  // logits are kept in log2 units
