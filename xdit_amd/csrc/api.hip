@@ -80,7 +80,8 @@ bool mfma16_path(const xdit_attn_args* a) {
 // Rate and segment cost depend on what a compute unit holds (Cost below).  One 4-wavefront workgroup
 // leaves every SIMD a single wavefront with nothing to overlap its softmax with (1.5 times the time per
 // row of 12 wavefronts); two of them hide each other's prologue and epilogue, which a lone 8- or
-// 12-wavefront workgroup exposes in full (what decides cross-attention on a few dozen keys).
+// 12-wavefront workgroup exposes in full (what decides cross-attention on a few dozen keys where it stays on this
+// kernel, see resident_path).
 // Balancing pays wherever the tiles leave compute units idle in the last round (the best plain
 // launch is 21 % slower on average than the best of the six, up to 3.8 times on a few heads of
 // 1000 to 3000 tokens) and costs a few per cent where they do not.  The constants are fitted to the

@@ -8,12 +8,13 @@
 // way while it computes, and one wavefront's loads and stores run beside another's products.
 // The arithmetic of a row is that of the tiled kernel, in the same order (TileMath), so the bits are the same.
 //
-// us of a call with the tiled kernel and here (bf16): head_dim 128, 24 heads of 40000 rows on 77 / 120 keys 117 -> 101 /
-// 120 -> 105, 40 of 32760 on 226 257 -> 226, 2 x 16 of 4096 on 256 28.5 -> 26.5; head_dim 72, 24 of 40000 on 120
-// 100 -> 81 (BSHD memory 106 -> 88), 2 x 16 of 4096 on 120 17.7 -> 15.5; 88, 48 of 60000 on 120 339 -> 271; 96, 24 of 40000
-// on 256 147 -> 138; 64, on 77, 120, 256, 512 keys 60.5 -> 60.2, 63.5 -> 61.9, 93.8 -> 92.5, 62.8 -> 60.7 (the
-// last of 14933 rows).  What is left (2 x 16 heads of 4096 at 72): 2 us of launch, 5 until keys and queries
-// are there, 1.5 per tile of a wavefront (its products beside another's softmax, as in the tiled loop), 1.5 for the rows out.
+// It is taken where its estimated time is the shorter one (resident_path in api.hip).  us of a call with the tiled kernel and
+// here (bf16): head_dim 128, 24 heads of 40000 rows on 77 / 120 keys 114 -> 99.7 / 118 -> 102, 40 of 32760 on 226 249 -> 218, 48 of 32760 on
+// 77 202 -> 181; head_dim 72, 24 of 40000 on 120 97.8 -> 78.7 (BSHD memory 104 -> 84.7), 2 x 16 of 4096 on 120 16.7 -> 13.6; 88, 48 of
+// 60000 on 120 336 -> 267; 96, 24 of 40000 on 256 144 -> 134; 64, 24 of 14933 on 512 61.4 -> 59.3.
+// What is left (2 x 16 heads at 72 on 120 keys, eight workgroups a head): 11.9 us with one row group per wavefront (3072 rows),
+// then 6.1 to 7.1 us for each further one (two to six: 19.0, 25.1, 32.1, 38.9, 46.0 us), in which 28 MB of rows come in and go out:
+// 4.2 TB/s, near the rate of a copy.  So about five are the launch and the way of the keys and first queries.
 #include "attn_fwd_16_impl.h"
 #include "resident_walk.h"
 

@@ -14,8 +14,8 @@
 // reference's `x / scale` bit for bit.  Optionally both passes first rotate each row along head_dim by a
 // block Hadamard matrix (_fp8_hadamard_rotate, attention_backend.py:703-714), in registers.
 // Several tensors (the q, k and v of one attention call) go through the same launches, blockIdx.z
-// selecting the tensor.  Flux-1024's q, k and v (85 MB) with the rotation of q and k: 19.5 us for the
-// abs-max (4.4 TB/s) and 26.3 us for the cast (4.9 TB/s), two launches; with a launch pair per tensor, the
+// selecting the tensor.  Flux-1024's q, k and v (85 MB) with the rotation of q and k: 16.5 us for the
+// abs-max (5.1 TB/s) and 25.2 us for the cast (5.1 TB/s), two launches; with a launch pair per tensor, the
 // rotation by shuffles and a compiler-made division it was six launches and 116 us.
 #include "common.h"
 #include "launchers.h"
