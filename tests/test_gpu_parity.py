@@ -1576,6 +1576,21 @@ def test_fp8_quant_batch_equals_single_calls(gpu, S, Sq, D, S2, dtype, per_tenso
         assert torch.equal(y.view(torch.uint8), quotient.to(torch.float8_e4m3fn).view(torch.uint8))
 
 
+@pytest.mark.parametrize("H,S,S2,D", [(24, 3217, 0, 128), (24, 3201, 16, 128), (16, 9641, 0, 64), (24, 3001, 0, 128), (24, 9216, 0, 128)])
+def test_fp8_quant_batch_at_either_number_of_rows_per_thread(gpu, H, S, S2, D):
+    """q, k and v that fill one round of workgroups with ten rows a thread (the first three on 256 compute units), and
+    others, against one call per tensor, whose grids differ: the same bytes, every one written."""
+    g = torch.Generator(device=gpu).manual_seed(S)
+    mk = lambda n: torch.randn(1, H, n, D, generator=g, device=gpu).bfloat16()
+    jobs = [(mk(S), True, None, D, None), (mk(S), False, None, D, mk(S2) if S2 else None), (mk(S + S2), True, None, 0, None)]
+    for got, (x, pt, scale, had, x2) in zip(ops.fp8_quant_batch(jobs), jobs):
+        want = [ops.fp8_quant(x[:, h:h + 1], per_tensor=pt, scale=got[-1][:1, h], hadamard_block=had, x2=None if x2 is None else x2[:, h:h + 1]) for h in range(H)]
+        whole = ops.fp8_quant(x, per_tensor=pt, scale=scale, hadamard_block=had, x2=x2)
+        assert torch.equal(got[-1], whole[-1])
+        for i, y in enumerate(got[:-1]):
+            assert torch.equal(y.view(torch.uint8), torch.cat([w[i] for w in want], 1).view(torch.uint8))
+
+
 @pytest.mark.parametrize("dtypes", [(torch.float32, torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32, torch.float32),
                                     (torch.float16, torch.bfloat16, torch.float32)])
 @pytest.mark.parametrize("joint", [None, "front", "rear"])

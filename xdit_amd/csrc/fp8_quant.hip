@@ -14,9 +14,10 @@
 // reference's `x / scale` bit for bit.  Optionally both passes first rotate each row along head_dim by a
 // block Hadamard matrix (_fp8_hadamard_rotate, attention_backend.py:703-714), in registers.
 // Several tensors (the q, k and v of one attention call) go through the same launches, blockIdx.z
-// selecting the tensor.  Flux-1024's q, k and v (85 MB) with the rotation of q and k: 16.5 us for the
-// abs-max (5.1 TB/s) and 25.2 us for the cast (5.1 TB/s), two launches; with a launch pair per tensor, the
+// selecting the tensor.  Flux-1024's q, k and v (85 MB) with the rotation of q and k: 17.2 us for the
+// abs-max (4.9 TB/s) and 23.7 us for the cast (5.4 TB/s), two launches; with a launch pair per tensor, the
 // rotation by shuffles and a compiler-made division it was six launches and 116 us.
+#include "attn_split.h"
 #include "common.h"
 #include "launchers.h"
 
@@ -179,9 +180,13 @@ __global__ void fill_zero_kernel(float* p, int n) {
 // q, k and v of Flux-1024 and of a 75600 x 5 shard: 45.9 and 161 us with four rows (eight in the abs-max) at once and no request
 // ahead, at four to five wavefronts, 40.5 and 144 now; three or four rows a step of the abs-max are no faster at the rule below.
 constexpr int kRowsInFlight = 2;
-// Rows per thread.  As many as make all tensors of a call one round of the workgroups that fit at once leave the memory to a
-// few of them at the end: cast of q, k and v of 40 heads of 32760 345 us where eight rows take 273, 2 x 48 of 17776 at head_dim 64
-// 220 and 181, 24 of 16384 104 and 88, 5 of 75600 91 and 83, 24 of 4608 23.5 and 24.2; 16 rows take 284, 190, 94, 85 and 25.3.
+// Rows per thread: eight, and for bf16 9 to 18 where that is a single round of the workgroups that fit at once, 94 % of it work
+// (rows of a workgroup come in pairs, so an odd number costs the next even one).  Of 2936 problems in that band (one tensor or q, k and
+// v, with and without rotation, 500 to 60000 rows, inputs in the cache or not) the 1230 of such rounds take 3.2 % less than with eight
+// rows, 4 % of them over 1 % longer; in the emptier ones it depends on the rest (one rotated tensor 2 % longer, one without rotation 7 %
+// less), 26 % over 1 % longer, up to 9 %.  Beyond 18 rows the memory is left to a few workgroups at the end (45 % of 557 longer,
+// 40 heads of 9450 by 10 %), and fp16 and fp32, with other numbers of wavefronts, take 2.5 and 3.2 % longer in a round of nine rows or more.
+// q, k and v with the rotation, eight rows and one round: 24 heads of 4608 43.6 and 41.6 us, 24 of 6000 56.6 and 53.9.
 constexpr int kRowsPerThread = 8;
 
 // `before` runs once per step, between a step's loads and their use.
@@ -347,15 +352,36 @@ __global__ void finalize_kernel(const QuantParams p, int n) {
   p.descale[i] = am > 0.f ? am / kFp8Max : 1.0f;
 }
 
+// The rule above.  Workgroups are rounded up per (batch, head), so they are counted for each number of rows.
+template <typename T>
+static int rows_per_thread(const QuantBatch& batch) {
+  if (!__is_same(T, __bf16)) return kRowsPerThread;
+  const int64_t slots = (int64_t)resident_cus() * 6;  // six to a compute unit by the registers of the cast (the abs-max: seven)
+  for (int rows = kRowsPerThread; rows <= 18; rows++) {
+    int64_t workgroups = 0, steps = 0;  // steps: of one row per thread
+    for (int i = 0; i < batch.n; i++) {
+      const QuantParams& p = batch.job[i];
+      const int64_t rpb = 256 / (p.D >> 3), slice = ((int64_t)p.S + p.S2 + rpb - 1) / rpb;
+      steps += (int64_t)p.B * p.H * slice;
+      workgroups += (int64_t)p.B * p.H * ((slice + rows - 1) / rows);
+    }
+    if (workgroups > slots) continue;
+    const int64_t room = slots * ((rows + kRowsInFlight - 1) / kRowsInFlight * kRowsInFlight);
+    return steps * 100 >= room * 94 ? rows : kRowsPerThread;
+  }
+  return kRowsPerThread;
+}
+
 template <typename T>
 static hipError_t run(QuantBatch& batch, hipStream_t stream) {
+  const int per_thread = rows_per_thread<T>(batch);
   int cast_x = 1, reduce_x = 0, bh_max = 1;
   for (int i = 0; i < batch.n; i++) {
     QuantParams& p = batch.job[i];
     const int BH = p.B * p.H;
     const int rpb = 256 / (p.D >> 3);
     const int64_t rows = (int64_t)p.S + p.S2;
-    int per_slice = (int)((rows + rpb * kRowsPerThread - 1) / (rpb * kRowsPerThread));
+    int per_slice = (int)((rows + rpb * per_thread - 1) / (rpb * per_thread));
     if (per_slice < 1) per_slice = 1;
     if (per_slice > 2048) per_slice = 2048;
     p.cast_blocks = per_slice;
