@@ -221,7 +221,7 @@ typedef struct {
                                   xdit_attn_fwd_accumulate for these arguments, 0 that of xdit_attn_fwd */
   int32_t resident_parts;      /* > 0: the call runs on the kernel that holds the keys of a (batch, head) in LDS (16-bit, at most
                                   four tiles of 64 keys at head_dim above 64, eight up to 64, both segments together;
-                                  rows_per_workgroup and balance 0; where its estimated time is the shorter one): the query
+                                  rows_per_workgroup and balance 0; where it is expected to take less time): the query
                                   rows of every (batch, head) are cut into this many parts, a workgroup each.  The result
                                   has the bits of the launch it takes the place of, which is always a plain one (ranges == 0) */
   int32_t reserved0;           /* 0 */

@@ -175,17 +175,20 @@ LaunchChoice choose_launch(const xdit_attn_args* a, bool plain = false, bool fol
 }
 
 // Whether a 16-bit forward runs on the kernel that keeps the keys of a head in LDS instead of the tiled launch chosen for
-// it: where they fit, that launch would be a plain one (whose bits this kernel gives) and its estimated time is longer, unless the
-// caller asks for a shape or a balance of the tiled launch.
+// it: where they fit, that launch would be a plain one (whose bits this kernel gives) and its estimated time is longer or there are
+// row groups enough, unless the caller asks for a shape or a balance of the tiled launch.
 // Of 14405 problems (B*H 1..32768, 16..100000 rows, 1..256 keys, 512 up to head_dim 64, head_dims 32..128, both memory orders) it
-// was more than 2 % slower in 7583 when every call over few keys took it, and is in 122 now; the choice is 0.3 % slower than the faster
-// of the two on average.  us, tiled and this kernel (bf16): 12 heads of 8192 on 226 keys at head_dim 128 22.6 and 24.5, 512 of 64 on 64
+// was more than 2 % slower in 7583 when every call over few keys took it, and in 122 by the estimates.  Those alone left 2180 of
+// another 23406 (B*H 1..128, 256..80000 rows) on a tiled launch that was more than 2 % slower (563 of them 8 %); with the row groups it is
+// 1213 (127) and 117 are more than 2 % slower here; the choice is 0.3 % slower than the faster kernel on average.  us, tiled and this kernel (bf16): 12 heads of 8192 on 226 keys at head_dim 128 22.6 and 24.5, 512 of 64 on 64
 // at 96 6.6 and 10.7, 3 of 1349 on 120 at 128 7.7 and 8.2, all tiled now; 48 of 32760 on 77 at 128 220 and 185.
 bool resident_path(const xdit_attn_args* a, const LaunchChoice& tiled) {
   const int D = kernel_head_dim(a->D);
   const int64_t nt = (a->Sk + xdit::kKeysPerTile - 1) / xdit::kKeysPerTile + (a->Sk2 + xdit::kKeysPerTile - 1) / xdit::kKeysPerTile;
   if (!mfma16_path(a) || tiled.policy != 1 || a->rows_per_workgroup != 0 || a->balance != 0 || nt > (D == 128 ? xdit::kResidentTiles<128> : xdit::kResidentTiles<64>)) return false;
-  return xdit::resident_us((int64_t)a->B * a->H, (int)a->Sq, (int)nt, a->D, xdit::resident_cus(a->cu_count), tiled.rows) < tiled.us;
+  const int64_t bh = (int64_t)a->B * a->H;
+  const int cus = xdit::resident_cus(a->cu_count);
+  return xdit::resident_us(bh, (int)a->Sq, (int)nt, a->D, cus, tiled.rows) < tiled.us || xdit::resident_enough_groups(bh, (int)a->Sq, (int)nt, a->D, cus, tiled.rows);
 }
 
 // The two tuning fields of xdit_attn_args.

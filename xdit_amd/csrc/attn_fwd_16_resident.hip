@@ -8,7 +8,7 @@
 // way while it computes, and one wavefront's loads and stores run beside another's products.
 // The arithmetic of a row is that of the tiled kernel, in the same order (TileMath), so the bits are the same.
 //
-// It is taken where its estimated time is the shorter one (resident_path in api.hip).  us of a call with the tiled kernel and
+// It is taken where it is expected to take less time (resident_path in api.hip).  us of a call with the tiled kernel and
 // here (bf16): head_dim 128, 24 heads of 40000 rows on 77 / 120 keys 114 -> 99.7 / 118 -> 102, 40 of 32760 on 226 249 -> 218, 48 of 32760 on
 // 77 202 -> 181; head_dim 72, 24 of 40000 on 120 97.8 -> 78.7 (BSHD memory 104 -> 84.7), 2 x 16 of 4096 on 120 16.7 -> 13.6; 88, 48 of
 // 60000 on 120 336 -> 267; 96, 24 of 40000 on 256 144 -> 134; 64, 24 of 14933 on 512 61.4 -> 59.3.

@@ -73,4 +73,19 @@ inline double resident_us(int64_t bh, int Sq, int nt, int head_dim, int cus, int
   return rate * rounds * (8.0 + (0.5 + per_wave) * nt) - 4.0;
 }
 
+// Whether the wavefronts have so many row groups (on average over the chip) that the keys pay for their way into LDS whatever the
+// estimates say, which are coarse between one and two rounds of the tiled launch.  Heads with at least two workgroups each only; and not at
+// head_dims 72, 80 and 96, where the estimates choose as well.  Of 23406 timed problems this sends 1248 more here than
+// the estimates do: at head_dim 128 614 with 4 % less time (median), at 88 and 104 to 120 267 with 12 %, at 64 (over more than one KV tile) 263
+// with 4 %, below 104 with 16 %; 4 % of them take over 2 % longer, 13 % at worst.  One group per wavefront is where the tiled launch starts a
+// second round; at 88 between one and one and a half calls on power-of-two rows are up to 12 % slower (12 heads of 8192 on 256 keys).
+inline bool resident_enough_groups(int64_t bh, int Sq, int nt, int head_dim, int cus, int tiled_rows) {
+  if (bh > cus / 2 || (head_dim > 64 && head_dim <= 80) || head_dim == 96) return false;
+  const int nw = resident_wavefronts(head_dim);
+  const int64_t workgroups = bh * resident_parts(bh, Sq, nt, nw, cus);
+  const double per_wave = (double)(bh * ((Sq + 31) / 32)) / (double)(workgroups > cus ? workgroups : cus) / nw;
+  if (head_dim <= 64) return tiled_rows <= 128 && per_wave > (head_dim < 64 ? 3.0 : 8.0) && (head_dim < 64 || nt > 1);
+  return per_wave > (head_dim == 88 ? 1.5 : 1.0);
+}
+
 }  // namespace xdit
